@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <cstring>
 #include <string>
+#include <type_traits>
 
 #include "../../include/tfdtd.h"
 #include "common.h"
@@ -198,24 +199,308 @@ __global__ __launch_bounds__(256) void yee_half_step_kernel(const HalfStep<real>
     half_step_cell<real, forward>(a, i);
 }
 
-// Cells per thread of the batched half step: a workgroup covers 256 * kBatchSpan cells of one grid, so
-// the search for its grid and the descriptor loads are shared by more cells (2: 2% faster on the
-// 64-grid uneven batch than 1 or 4).
+// ---------------------------------------------------------------- half step marched over x planes
+//
+// A wavefront takes 64 consecutive cells of the flattened (y, z) plane and marches them over `span` x
+// planes.  What depends on y and z alone -- the coordinates, the neighbours' offsets, the slab rows and
+// their coefficients -- is computed once per march, x is uniform (its slab, its coefficients and the plane
+// addresses are scalar), and every field access is a uniform base plus a 32-bit lane offset, so a cell
+// costs little more than its own arithmetic.  One thread per cell of the whole grid (half_step_cell) was
+// bound by its 64-bit divisions, per-term slab tests and dependent descriptor loads: a step of both
+// families plus its trace took 26.5 us on 160x120x40 cells, 49.1 us on 200x160x60, 124 us on 192^3, 325 us
+// on 256^3 (FP32), 30.5 us on 97x83x61 (FP64); the march takes 18.1, 35.7, 106, 286 and 20.9 us.  What
+// bounds it now is the traffic: past the 256 MB cache 5 TB/s of a copy's 5.5, inside it about 6 of 8.2.
+template <typename real>
+struct PlaneAxis {          // CPML rows of one axis, shared by its two terms: low side, then high side
+    int lo[2], hi[2];       // empty: lo == hi == 0
+    unsigned psi[2];        // byte offset of each term's low-side memory in the family's buffer
+    unsigned high[2];       // what to add for the high side
+    unsigned coef, coef_high;   // byte offset of b | c | inv_k of the low side, and what to add for the high side
+};
+
+struct Divider {            // q = (mulhi(m, n) + n) >> s for n < 2^31
+    unsigned m, s;
+};
+
+template <typename real>
+struct PlaneStep {
+    int nx, ny, nz, nyz;
+    int span, columns;      // planes per march, 64-cell columns of a plane
+    Divider by_nz, by_columns;
+    int xcd, spare;         // workgroups an XCD takes in a row
+    const real* src;
+    real* dst;
+    const real* inverse;
+    real* psi;
+    const real* coef;
+    PlaneAxis<real> axis[3];
+    int box_lo[3], box_hi[3];
+    int nsrc;
+    int periodic_mask, pec_mask;
+    real courant;
+    real pec_factor[3];
+    Source<real> srcs[TFDTD_MAX_SOURCES];
+    long long source_samples;
+    const long long* counter;
+};
+
+__device__ __forceinline__ unsigned divide(unsigned n, Divider d) { return (__umulhi(n, d.m) + n) >> d.s; }
+
+// A value at a uniform base plus a 32-bit byte offset of the lane.
+template <typename real>
+__device__ __forceinline__ real at_byte(const real* base, unsigned off) {
+    return *global(reinterpret_cast<const real*>(reinterpret_cast<const char*>(base) + off));
+}
+
+template <typename real>
+__device__ __forceinline__ void put_byte(real* base, unsigned off, real v) {
+    *global(reinterpret_cast<real*>(reinterpret_cast<char*>(base) + off)) = v;
+}
+
+template <typename real>
+__device__ __forceinline__ Cell<real> cell_at_byte(const real* base, unsigned off) {
+    const auto p = global(reinterpret_cast<const real*>(reinterpret_cast<const char*>(base) + off));
+    return Cell<real>{{p[0], p[1], p[2]}};
+}
+
+// The CPML row of the y or z axis a lane lies in: the memory of its two terms and their coefficients.
+template <typename real>
+struct PlaneHit {
+    bool on;
+    unsigned at[2];     // byte offsets of the two terms' memory in the current plane
+    unsigned stride;    // bytes per x plane
+    real b, c, ik;
+};
+
+// The row k of an axis: w is its slab's width; `on` false leaves the rest unused.
+template <typename real>
+struct AxisRow {
+    bool on;
+    int q, w;
+    unsigned psi[2], coef;
+};
+
+template <typename real>
+__device__ __forceinline__ AxisRow<real> axis_row(const PlaneAxis<real>& p, int k, bool inside) {
+    const int k0 = k - p.lo[0], k1 = k - p.lo[1], w0 = p.hi[0] - p.lo[0], w1 = p.hi[1] - p.lo[1];
+    const bool low = (unsigned)k0 < (unsigned)w0, high = (unsigned)k1 < (unsigned)w1;
+    AxisRow<real> r;
+    r.on = inside & (low | high);
+    r.q = low ? k0 : k1;
+    r.w = low ? w0 : w1;
+    for (int t = 0; t < 2; ++t) r.psi[t] = p.psi[t] + (low ? 0u : p.high[t]);
+    r.coef = p.coef + (low ? 0u : p.coef_high);
+    return r;
+}
+
+template <typename real, bool forward, int INV, bool FLAT>
+__device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const unsigned item) {
+    constexpr unsigned W = sizeof(real);
+    const int nx = a.nx, ny = a.ny, nz = FLAT ? 1 : a.nz, nyz = a.nyz;
+    // Spare lanes of the last column and spare wavefronts of the last workgroup repeat a cell and store nothing.
+    const unsigned chunks = (unsigned)(nx + a.span - 1) / (unsigned)a.span;
+    const unsigned xchunk = min(divide(item, a.by_columns), chunks - 1u);
+    const unsigned cell = (item - xchunk * a.columns) * 64u + (threadIdx.x & 63u);
+    const bool owned = cell < (unsigned)nyz;
+    const unsigned r = min(cell, (unsigned)nyz - 1u);
+    const int xa = (int)xchunk * a.span, xb = min(nx, xa + a.span);
+    const int y = FLAT ? (int)r : (int)divide(r, a.by_nz), z = FLAT ? 0 : (int)(r - (unsigned)y * nz);
+    const unsigned off = r * (3 * W);
+    const bool iny = forward ? y < ny - 1 : y > 0, inz = !FLAT && (forward ? z < nz - 1 : z > 0);
+    const bool wrapx = a.periodic_mask & 1, wrapy = a.periodic_mask & 2, wrapz = !FLAT && (a.periodic_mask & 4);
+    const unsigned rowb = (unsigned)nz * (3 * W), lasty = (unsigned)(ny - 1) * rowb, lastz = (unsigned)(nz - 1) * (3 * W);
+    const unsigned offy = forward ? (iny ? off + rowb : wrapy ? off - lasty : off) : (iny ? off - rowb : wrapy ? off + lasty : off);
+    const unsigned offz = forward ? (inz ? off + 3 * W : wrapz ? off - lastz : off) : (inz ? off - 3 * W : wrapz ? off + lastz : off);
+    const long long plane = 3LL * nyz;
+    const real* src = a.src + xa * plane;
+    real* dst = a.dst + xa * plane;
+    real one = real(0);
+    if (INV == 0) one = global(a.inverse)[0];
+    // Backward differences carry the plane just left as x - 1, forward ones the plane fetched as x + 1.
+    Cell<real> here = cell_at_byte(src, off);
+    Cell<real> side = cell_at_byte(forward ? src : xa > 0 ? src - plane : wrapx ? a.src + (nx - 1) * plane : src, off);
+    const AxisRow<real> ry = axis_row(a.axis[1], y, iny);
+    PlaneHit<real> hy{ry.on, {0u, 0u}, 0u, real(0), real(0), real(0)};
+    if (ry.on) {
+        const unsigned e = ((unsigned)ry.q * nz + z) * W, wide = (unsigned)ry.w * W, k = ry.coef + (unsigned)ry.q * W;
+        hy.stride = wide * nz;
+        hy.at[0] = ry.psi[0] + e + xa * hy.stride;
+        hy.at[1] = ry.psi[1] + e + xa * hy.stride;
+        hy.b = at_byte(a.coef, k);
+        hy.c = at_byte(a.coef, k + wide);
+        hy.ik = at_byte(a.coef, k + 2 * wide);
+    }
+    PlaneHit<real> hz{false, {0u, 0u}, 0u, real(0), real(0), real(0)};
+    if (!FLAT) {
+        const AxisRow<real> rz = axis_row(a.axis[2], z, inz);
+        hz.on = rz.on;
+        if (rz.on) {
+            const unsigned wide = (unsigned)rz.w * W, e = y * wide + (unsigned)rz.q * W, k = rz.coef + (unsigned)rz.q * W;
+            hz.stride = wide * ny;
+            hz.at[0] = rz.psi[0] + e + xa * hz.stride;
+            hz.at[1] = rz.psi[1] + e + xa * hz.stride;
+            hz.b = at_byte(a.coef, k);
+            hz.c = at_byte(a.coef, k + wide);
+            hz.ik = at_byte(a.coef, k + 2 * wide);
+        }
+    }
+    const bool source = owned && a.nsrc > 0 && y >= a.box_lo[1] && y < a.box_hi[1] && z >= a.box_lo[2] && z < a.box_hi[2];
+    real* const psi = a.psi;
+    for (int x = xa; x < xb; ++x) {
+        const bool inx = forward ? x < nx - 1 : x > 0;
+        if (forward) side = cell_at_byte(inx ? src + plane : wrapx ? a.src : src, off);
+        const Cell<real> old = cell_at_byte(dst, off);
+        Cell<real> inv;
+        if (INV == 3) inv = cell_at_byte(a.inverse + x * plane, off);
+        else {
+            const real v = INV == 1 ? at_byte(a.inverse + (long long)x * nyz, r * W) : one;
+            inv = Cell<real>{{v, v, v}};
+        }
+        const Cell<real> nby = cell_at_byte(src, offy);
+        Cell<real> nbz{{real(0), real(0), real(0)}};
+        if (!FLAT) nbz = cell_at_byte(src, offz);
+        Cell<real> ahead = here;      // backward: the next plane, read with this one's neighbours
+        if (!forward && x + 1 < xb) ahead = cell_at_byte(src + plane, off);
+        // Every CPML memory value is read before the first store (a load behind a store would wait for it).
+        real mx[2], my[2], mz[2];
+        const AxisRow<real> rx = axis_row(a.axis[0], x, inx);
+        real bx = real(0), cx = real(0), ikx = real(0);
+        unsigned atx[2] = {0u, 0u};
+        if (rx.on) {
+            const unsigned wide = (unsigned)rx.w * W, k = rx.coef + (unsigned)rx.q * W, e = ((unsigned)rx.q * nyz + r) * W;
+            bx = at_byte(a.coef, k);
+            cx = at_byte(a.coef, k + wide);
+            ikx = at_byte(a.coef, k + 2 * wide);
+            for (int t = 0; t < 2; ++t) {
+                atx[t] = rx.psi[t] + e;
+                mx[t] = at_byte(psi, atx[t]);
+            }
+        }
+        if (hy.on)
+            for (int t = 0; t < 2; ++t) my[t] = at_byte(psi, hy.at[t]);
+        if (hz.on)
+            for (int t = 0; t < 2; ++t) mz[t] = at_byte(psi, hz.at[t]);
+        real curl[3] = {real(0), real(0), real(0)};
+        // The two terms of one axis: difference, CPML row, sum into the curl in term order.
+        auto axis_terms = [&](auto axis_tag, bool in, bool wrap, const Cell<real>& nb, bool hit, real b, real c, real ik, real* m) {
+            constexpr int axis = decltype(axis_tag)::value;
+            const real pec = forward && ((a.pec_mask >> axis) & 1) ? -a.pec_factor[axis] : real(0);
+            const bool pecs = forward && ((a.pec_mask >> axis) & 1);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int t = 2 * axis + k, ic = term_in(t), oc = term_out(t);
+                real d = forward ? nb.v[ic] - here.v[ic] : here.v[ic] - nb.v[ic];
+                if (hit) {
+                    m[k] = m[k] * b + c * d;
+                    d = d * ik + m[k];
+                }
+                if (!in && !wrap) d = pecs ? pec * here.v[ic] : real(0);
+                curl[oc] = term_sign(t) > 0 ? curl[oc] + d : curl[oc] - d;
+            }
+        };
+        axis_terms(std::integral_constant<int, 0>{}, inx, wrapx, side, rx.on, bx, cx, ikx, mx);
+        axis_terms(std::integral_constant<int, 1>{}, iny, wrapy, nby, hy.on, hy.b, hy.c, hy.ik, my);
+        if (!FLAT) axis_terms(std::integral_constant<int, 2>{}, inz, wrapz, nbz, hz.on, hz.b, hz.c, hz.ik, mz);
+        real out[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const real coefficient = a.courant * inv.v[m];
+            out[m] = forward ? old.v[m] - coefficient * curl[m] : old.v[m] + coefficient * curl[m];
+        }
+        if (source && x >= a.box_lo[0] && x < a.box_hi[0]) {
+            const long long n = *global(a.counter);
+            for (int k = 0; k < a.nsrc && n < a.source_samples; ++k) {
+                const Source<real>& box = a.srcs[k];
+                if (x >= box.lo[0] && x < box.hi[0] && y >= box.lo[1] && y < box.hi[1] && z >= box.lo[2] &&
+                    z < box.hi[2]) {
+                    const real v = global(box.values)[n];
+                    if (box.comp == 0) out[0] = out[0] + v;
+                    else if (box.comp == 1) out[1] = out[1] + v;
+                    else out[2] = out[2] + v;
+                }
+            }
+        }
+        if (owned) {
+            if (rx.on)
+                for (int t = 0; t < 2; ++t) put_byte(psi, atx[t], mx[t]);
+            if (hy.on)
+                for (int t = 0; t < 2; ++t) put_byte(psi, hy.at[t], my[t]);
+            if (hz.on)
+                for (int t = 0; t < 2; ++t) put_byte(psi, hz.at[t], mz[t]);
+            const auto to = global(reinterpret_cast<real*>(reinterpret_cast<char*>(dst) + off));
+            to[0] = out[0];
+            to[1] = out[1];
+            to[2] = out[2];
+        }
+        if (!forward) { side = here; here = ahead; }
+        else here = side;
+        for (int t = 0; t < 2; ++t) { hy.at[t] += hy.stride; hz.at[t] += hz.stride; }
+        src += plane;
+        dst += plane;
+    }
+}
+
+// The wavefront's number among those of its grid, as a scalar.
+__device__ __forceinline__ unsigned wave_item(unsigned block) {
+    return block * 4u + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+}
+
+constexpr unsigned kXcdRun = 128;
+
+// Workgroup b runs on XCD b % 8.  Within each run of 8 * xcd workgroups every XCD takes `xcd` consecutive ones.
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned blocks, unsigned run) {
+    const unsigned first = b / (8u * run) * (8u * run);
+    if (first + 8u * run > blocks) return b;
+    const unsigned k = b - first;
+    return first + (k & 7u) * run + (k >> 3);
+}
+
+template <typename real, bool forward, int INV, bool FLAT>
+__global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void plane_half_step_kernel(const PlaneStep<real> a) {
+    march_half_step<real, forward, INV, FLAT>(a, wave_item(xcd_block(blockIdx.x, gridDim.x, a.xcd)));
+}
+
+// One grid of a batched half step: its plane march where `march` is set, else the general step.
+template <typename real>
+struct BatchStep {
+    HalfStep<real> general;
+    PlaneStep<real> plane;
+    int march, inverse_stride;
+};
+
+// Cells per thread of the general batched half step: a workgroup covers 256 * kBatchSpan cells of one
+// grid, so the search for its grid and the descriptor loads are shared by more cells.
 constexpr int kBatchSpan = 2;
 
 // Many grids in one launch: block b belongs to the last grid g with prefix[g] <= b; the grids'
 // descriptors are a table in device memory, read with wave-uniform loads.
 template <typename real, bool forward>
-__global__ __launch_bounds__(256) void batch_half_step_kernel(const HalfStep<real>* __restrict__ table,
+__global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void batch_half_step_kernel(const BatchStep<real>* __restrict__ table,
                                                               const int* __restrict__ prefix, int grids) {
-    const int b = blockIdx.x;
+    const int b = (int)xcd_block(blockIdx.x, gridDim.x, kXcdRun);
     int lo = 0, hi = grids;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
         if (prefix[mid] <= b) lo = mid;
         else hi = mid;
     }
-    const HalfStep<real>& a = table[lo];
+    const BatchStep<real>& t = table[lo];
+    if (t.march) {
+        const unsigned item = wave_item((unsigned)(b - prefix[lo]));
+        const bool flat = t.plane.nz == 1;
+        if (forward) {
+            if (flat) march_half_step<real, true, 0, true>(t.plane, item);
+            else march_half_step<real, true, 0, false>(t.plane, item);
+        } else if (t.inverse_stride == 1) {
+            if (flat) march_half_step<real, false, 1, true>(t.plane, item);
+            else march_half_step<real, false, 1, false>(t.plane, item);
+        } else {
+            if (flat) march_half_step<real, false, 3, true>(t.plane, item);
+            else march_half_step<real, false, 3, false>(t.plane, item);
+        }
+        return;
+    }
+    const HalfStep<real>& a = t.general;
     const long long cells = (long long)a.nx * a.ny * a.nz;
     const long long base = (long long)(b - prefix[lo]) * (256 * kBatchSpan) + threadIdx.x;
 #pragma unroll
@@ -471,11 +756,127 @@ int make_half_step(const tfdtd_half_step* d, HalfStep<real>* a) {
     return TFDTD_OK;
 }
 
+Divider make_divider(unsigned d) {
+    unsigned s = 0;
+    while ((1ull << s) < d) ++s;
+    return Divider{(unsigned)(((1ull << 32) * ((1ull << s) - d)) / d + 1), s};
+}
+
+// Planes per march: two share the lane's set-up and the plane between them (18.9 against 20.7 us a step on
+// 160x120x40 cells, 12,000 column-planes; 22.2 against 24.7 us on 97x83x61 in FP64, 7,760; four planes:
+// 18.8 and 22.3).  A grid of few wavefronts keeps one, as it needs them all to fill the chip: 7.3 us
+// against 8.5 on 160x120x1, 320 column-planes.
+constexpr long long kSpanItems = 4096;
+
+// Workgroups that one XCD takes in a row: neighbouring rows and planes are then read through one L2.
+// Runs of 1 / 32 / 128 take 40.0 / 36.5 / 35.7 us on 200x160x60 cells, 117.7 / 106.8 / 105.9 us on 192^3 and
+// 292 / 304 / 286 us on 256^3 (384: 299); grids of few workgroups take shorter runs (97x83x61, 970
+// workgroups: 20.9 us with 32, 22.2 with 128) so that every XCD has its share.
+inline unsigned xcd_run(long long blocks) { return (unsigned)std::min<long long>(std::max<long long>(blocks / 32, 1), kXcdRun); }
+
+template <typename real>
+long long plane_blocks(const PlaneStep<real>& a) {
+    return ((long long)a.columns * ((a.nx + a.span - 1) / a.span) + 3) / 4;
+}
+
+// The plane march of a half step: true when the grid's layout allows it.  The two terms of an axis must
+// share their slab rows and one coefficient block b | c | inv_k on each side, the family's memory, its
+// coefficients and a plane's fields must each span less than 4 GiB (32-bit byte offsets), x and y need
+// two cells or more, and the coefficient is per cell or component for E, one value for H.  Everything
+// else keeps the general step.
+template <typename real>
+bool make_plane_step(const HalfStep<real>& h, bool forward, PlaneStep<real>* out) {
+    PlaneStep<real>& a = *out;
+    std::memset(&a, 0, sizeof a);
+    constexpr long long limit = 0xffffffffLL;
+    const long long nyz = (long long)h.ny * h.nz;
+    if (forward ? h.inverse_stride != 0 : h.inverse_stride == 0) return false;
+    if (h.nx < 2 || h.ny < 2 || nyz * 3 * (long long)sizeof(real) > limit) return false;
+    auto address = [](const void* p) { return reinterpret_cast<const char*>(p); };
+    const char* psi = nullptr;
+    const char* coef = nullptr;
+    for (const Slab<real>& s : h.slab)
+        if (s.hi > s.lo) {
+            if (!psi || address(s.psi) < psi) psi = address(s.psi);
+            if (!coef || address(s.b) < coef) coef = address(s.b);
+        }
+    const int dims[3] = {h.nx, h.ny, h.nz};
+    for (int ax = 0; ax < 3; ++ax) {
+        unsigned at[2][2] = {{0u, 0u}, {0u, 0u}}, block[2] = {0u, 0u};
+        for (int side = 0; side < 2; ++side) {
+            const Slab<real>& p = h.slab[4 * ax + side];
+            const Slab<real>& q = h.slab[4 * ax + 2 + side];
+            const int w = p.hi - p.lo;
+            if (p.lo != q.lo || p.hi != q.hi) return false;
+            if (w == 0) continue;
+            if (p.b != q.b || p.c != q.c || p.inv_k != q.inv_k || p.c != p.b + w || p.inv_k != p.b + 2 * w) return false;
+            const long long bytes = w * ((long long)h.nx * nyz / dims[ax]) * (long long)sizeof(real);
+            const long long offset[3] = {address(p.psi) - psi, address(q.psi) - psi, address(p.b) - coef};
+            if (offset[0] + bytes > limit || offset[1] + bytes > limit || offset[2] + 3LL * w * (long long)sizeof(real) > limit) return false;
+            at[side][0] = (unsigned)offset[0];
+            at[side][1] = (unsigned)offset[1];
+            block[side] = (unsigned)offset[2];
+            a.axis[ax].lo[side] = p.lo;
+            a.axis[ax].hi[side] = p.hi;
+        }
+        for (int t = 0; t < 2; ++t) {
+            a.axis[ax].psi[t] = at[0][t];
+            a.axis[ax].high[t] = at[1][t] - at[0][t];
+        }
+        a.axis[ax].coef = block[0];
+        a.axis[ax].coef_high = block[1] - block[0];
+    }
+    a.psi = reinterpret_cast<real*>(const_cast<char*>(psi));
+    a.coef = reinterpret_cast<const real*>(coef);
+    a.nx = h.nx; a.ny = h.ny; a.nz = h.nz; a.nyz = (int)nyz;
+    a.columns = (int)((nyz + 63) / 64);
+    a.span = (long long)a.columns * h.nx < kSpanItems ? 1 : 2;
+    a.by_nz = make_divider((unsigned)h.nz);
+    a.by_columns = make_divider((unsigned)a.columns);
+    const long long items = (long long)a.columns * ((h.nx + a.span - 1) / a.span);
+    if (items > 0x7ffffff0LL) return false;
+    a.xcd = (int)xcd_run(plane_blocks(a));
+    a.src = h.src; a.dst = h.dst; a.inverse = h.inverse;
+    a.courant = h.courant;
+    a.periodic_mask = h.periodic_mask; a.pec_mask = h.pec_mask;
+    for (int k = 0; k < 3; ++k) {
+        a.pec_factor[k] = h.pec_factor[k];
+        a.box_lo[k] = h.box_lo[k]; a.box_hi[k] = h.box_hi[k];
+    }
+    a.nsrc = h.nsrc;
+    std::memcpy(a.srcs, h.srcs, sizeof a.srcs);
+    a.source_samples = h.source_samples;
+    a.counter = h.counter;
+    return true;
+}
+
+template <typename real>
+void launch_plane_step(const PlaneStep<real>& a, bool forward, int inverse_stride, hipStream_t stream) {
+    const dim3 grid((unsigned)plane_blocks(a)), block(256);
+    const bool flat = a.nz == 1;
+    if (forward) {
+        if (flat) hipLaunchKernelGGL((plane_half_step_kernel<real, true, 0, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((plane_half_step_kernel<real, true, 0, false>), grid, block, 0, stream, a);
+    } else if (inverse_stride == 1) {
+        if (flat) hipLaunchKernelGGL((plane_half_step_kernel<real, false, 1, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((plane_half_step_kernel<real, false, 1, false>), grid, block, 0, stream, a);
+    } else {
+        if (flat) hipLaunchKernelGGL((plane_half_step_kernel<real, false, 3, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((plane_half_step_kernel<real, false, 3, false>), grid, block, 0, stream, a);
+    }
+}
+
 template <typename real>
 int launch_half_step(const tfdtd_half_step* d, hipStream_t stream) {
     HalfStep<real> a;
     int status = make_half_step(d, &a);
     if (status) return status;
+    const bool forward = d->family == TFDTD_FAMILY_H;
+    PlaneStep<real> p;
+    if (make_plane_step(a, forward, &p)) {
+        launch_plane_step(p, forward, d->inverse_stride, stream);
+        return check_launch("yee_half_step");
+    }
     const long long count = (long long)d->nx * d->ny * d->nz;
     const long long blocks = (count + 255) / 256;
     if (blocks > 0x7fffffffLL) return fail(TFDTD_EINVAL, "grid too large for one launch");
@@ -642,16 +1043,20 @@ int observe(const tfdtd_observe* d, hipStream_t stream) {
 template <typename real>
 int pack_half_steps(const tfdtd_half_step* steps, int count, void* host_table, size_t bytes, int32_t* prefix) {
     if (count < 1 || !steps || !prefix) return fail(TFDTD_EINVAL, "batch: at least one descriptor and a prefix array");
-    if (!host_table || bytes < sizeof(HalfStep<real>) * (size_t)count) return fail(TFDTD_EINVAL, "batch: table buffer too small");
-    HalfStep<real>* table = static_cast<HalfStep<real>*>(host_table);
+    if (!host_table || bytes < sizeof(BatchStep<real>) * (size_t)count) return fail(TFDTD_EINVAL, "batch: table buffer too small");
+    BatchStep<real>* table = static_cast<BatchStep<real>*>(host_table);
     long long total = 0;
     for (int k = 0; k < count; ++k) {
         if (steps[k].family != steps[0].family || steps[k].dtype != steps[0].dtype)
             return fail(TFDTD_EINVAL, "batch: descriptor %d differs in family or dtype", k);
-        const int status = make_half_step(steps + k, table + k);
+        BatchStep<real>& t = table[k];
+        const int status = make_half_step(steps + k, &t.general);
         if (status) return status;
+        t.march = make_plane_step(t.general, steps[k].family == TFDTD_FAMILY_H, &t.plane) ? 1 : 0;
+        t.inverse_stride = t.general.inverse_stride;
         prefix[k] = (int32_t)total;
-        total += ((long long)steps[k].nx * steps[k].ny * steps[k].nz + 256 * kBatchSpan - 1) / (256 * kBatchSpan);
+        total += t.march ? plane_blocks(t.plane)
+                         : ((long long)steps[k].nx * steps[k].ny * steps[k].nz + 256 * kBatchSpan - 1) / (256 * kBatchSpan);
         if (total > 0x7fffffffLL) return fail(TFDTD_EINVAL, "batch: too many cells for one launch");
     }
     prefix[count] = (int32_t)total;
@@ -680,7 +1085,7 @@ extern "C" {
 
 size_t tfdtd_batch_table_bytes(int32_t count, int32_t dtype) {
     if (count < 0) return 0;
-    return (size_t)count * (dtype == TFDTD_F64 ? sizeof(HalfStep<double>) : sizeof(HalfStep<float>));
+    return (size_t)count * (dtype == TFDTD_F64 ? sizeof(BatchStep<double>) : sizeof(BatchStep<float>));
 }
 
 int tfdtd_batch_pack(const tfdtd_half_step* steps, int32_t count, void* host_table, size_t bytes, int32_t* block_prefix) {
@@ -697,11 +1102,11 @@ int tfdtd_batch_half_step(const void* device_table, const int32_t* device_prefix
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int* prefix = reinterpret_cast<const int*>(device_prefix);
     if (dtype == TFDTD_F32) {
-        const HalfStep<float>* t = static_cast<const HalfStep<float>*>(device_table);
+        const BatchStep<float>* t = static_cast<const BatchStep<float>*>(device_table);
         if (family == TFDTD_FAMILY_E) hipLaunchKernelGGL((batch_half_step_kernel<float, false>), dim3(total_blocks), dim3(256), 0, s, t, prefix, count);
         else hipLaunchKernelGGL((batch_half_step_kernel<float, true>), dim3(total_blocks), dim3(256), 0, s, t, prefix, count);
     } else if (dtype == TFDTD_F64) {
-        const HalfStep<double>* t = static_cast<const HalfStep<double>*>(device_table);
+        const BatchStep<double>* t = static_cast<const BatchStep<double>*>(device_table);
         if (family == TFDTD_FAMILY_E) hipLaunchKernelGGL((batch_half_step_kernel<double, false>), dim3(total_blocks), dim3(256), 0, s, t, prefix, count);
         else hipLaunchKernelGGL((batch_half_step_kernel<double, true>), dim3(total_blocks), dim3(256), 0, s, t, prefix, count);
     } else {
