@@ -24,7 +24,7 @@ extern "C" {
 #define TFDTD_MAX_SEGMENTS 12   /* 6 curl terms x 2 PML faces, per family */
 #define TFDTD_MAX_SOURCES 16    /* soft source boxes per family */
 
-enum { TFDTD_OK = 0, TFDTD_EINVAL = 1, TFDTD_EHIP = 2 };
+enum { TFDTD_OK = 0, TFDTD_EINVAL = 1, TFDTD_EHIP = 2, TFDTD_EUNSUPPORTED = 3 };
 enum { TFDTD_F32 = 0, TFDTD_F64 = 1 };
 enum { TFDTD_FAMILY_E = 0, TFDTD_FAMILY_H = 1 };
 
@@ -485,6 +485,31 @@ int tfdtd_conv_wgrad(const tfdtd_conv* conv, const void* dy_t, const void* x, in
 /* dpre = dy * GELU'(pre) (activation 1) or dy (0), in FP32 and bf16. */
 int tfdtd_gelu_backward(const float* dy, const float* pre, int64_t count, int32_t activation, float* dpre, void* dpre16,
                         void* stream);
+
+/* The bf16 operands of a layer from its FP32 weights [co][ks^3][ci], in one launch: w16 [co][kp] for the
+ * forward, weight_t [ci][ks^3*co] for the input gradient (null: not wanted), and nonfinite
+ * int32[tfdtd_conv_weight_parts(conv)], 1 where a part of the weights holds an infinity or NaN. */
+int tfdtd_conv_weight_parts(const tfdtd_conv* conv);
+int tfdtd_conv_weights(const tfdtd_conv* conv, const float* weight, void* w16, void* weight_t, int32_t* nonfinite, void* stream);
+/* tfdtd_conv_forward with any of its outputs: pre FP32, y FP32 (the value of the bf16 activation), act bf16.
+ * With `nonfinite` (of tfdtd_conv_weights) a tap that is padding for all rows of a workgroup is skipped when every
+ * weight is finite.  TFDTD_EUNSUPPORTED where channels (multiples of 8, or kp 32) or the 16-byte alignment
+ * of the operands leave the layer to tfdtd_conv_forward; likewise tfdtd_conv_dgrad_rows to tfdtd_conv_dgrad. */
+int tfdtd_conv_forward_rows(const tfdtd_conv* conv, const void* x, const void* weight, const int32_t* nonfinite, const float* bias,
+                            int32_t activation, float* pre, float* y, void* act, void* stream);
+int tfdtd_conv_dgrad_rows(const tfdtd_conv* conv, const void* dy, const void* weight_t, const int32_t* nonfinite, float* dx,
+                          void* stream);
+/* The weight gradient from dy bf16 [m_out][co] as the input gradient reads it (no transposed copy):
+ * partial float[tfdtd_conv_wgrad_splits(conv)][co][kp].  Channels must be multiples of 8, or kp 32;
+ * tfdtd_conv_wgrad_splits returns 0 for other layers, which take tfdtd_conv_wgrad. */
+int tfdtd_conv_wgrad_splits(const tfdtd_conv* conv);
+int tfdtd_conv_wgrad_rows(const tfdtd_conv* conv, const void* dy, const void* x, float* partial, float* dw, void* stream);
+/* dpre16 = bf16(dy * GELU'(pre)) (activation 1) or bf16(dy) (0) of a [rows][channels] layer output, and
+ * bias_grad[channels] the sum over the rows of the unrounded values (FP64, rounded once); partial is
+ * double[TFDTD_BIAS_BLOCKS][channels].  channels: a multiple of 4, at most 1024. */
+#define TFDTD_BIAS_BLOCKS 2048
+int tfdtd_gelu_backward_rows(const float* dy, const float* pre, int64_t rows, int32_t channels, int32_t activation, void* dpre16,
+                             double* partial, float* bias_grad, void* stream);
 
 /* Copies the calling thread's last error message; returns its length. */
 size_t tfdtd_last_error(char* buffer, size_t size);

@@ -120,6 +120,8 @@ class NormGrid(ctypes.Structure):
 
 
 ADE_MAX_POLES = 16
+BIAS_BLOCKS = 2048
+EUNSUPPORTED = 3
 
 
 class Ade(ctypes.Structure):
@@ -189,6 +191,13 @@ PROTOTYPES = {
     'tfdtd_conv_forward': (i32, [vp, vp, vp, vp, i32, vp, vp, vp]),
     'tfdtd_conv_dgrad': (i32, [vp, vp, vp, vp, vp]),
     'tfdtd_conv_wgrad': (i32, [vp, vp, vp, i32, vp, vp, vp]),
+    'tfdtd_conv_weight_parts': (i32, [vp]),
+    'tfdtd_conv_weights': (i32, [vp, vp, vp, vp, vp, vp]),
+    'tfdtd_conv_forward_rows': (i32, [vp, vp, vp, vp, vp, i32, vp, vp, vp, vp]),
+    'tfdtd_conv_dgrad_rows': (i32, [vp, vp, vp, vp, vp, vp]),
+    'tfdtd_conv_wgrad_splits': (i32, [vp]),
+    'tfdtd_conv_wgrad_rows': (i32, [vp, vp, vp, vp, vp, vp]),
+    'tfdtd_gelu_backward_rows': (i32, [vp, vp, i64, i32, i32, vp, vp, vp, vp]),
     'tfdtd_gelu_backward': (i32, [vp, vp, i64, i32, vp, vp, vp]),
     'tfdtd_abi_version': (i32, []),
     'tfdtd_source_digest': (ctypes.c_char_p, []),
@@ -246,6 +255,11 @@ def last_error():
 def check(status, what):
     if status != 0:
         raise RuntimeError(f'{what} failed ({status}): {last_error()}')
+
+
+def address(tensor):
+    """A tensor's device address, None (a null pointer) for no tensor."""
+    return None if tensor is None else tensor.data_ptr()
 
 
 def stream_handle(device=None):

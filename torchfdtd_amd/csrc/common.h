@@ -20,6 +20,27 @@ __device__ __forceinline__ __attribute__((address_space(1))) T* global(T* p) {
     return (__attribute__((address_space(1))) T*)p;
 }
 
+// Division by a value fixed on the host: n / d = (mulhi(m, n) + n) >> s for n < 2^31.
+struct Divider {
+    unsigned m, s;
+};
+
+inline Divider make_divider(unsigned d) {
+    unsigned s = 0;
+    while ((1ull << s) < d) ++s;
+    return Divider{(unsigned)(((1ull << 32) * ((1ull << s) - d)) / d + 1), s};
+}
+
+__device__ __forceinline__ unsigned divide(unsigned n, Divider d) { return (__umulhi(n, d.m) + n) >> d.s; }
+
+// Workgroup b runs on XCD b % 8.  Within each run of 8 * xcd workgroups every XCD takes `xcd` consecutive ones.
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned blocks, unsigned run) {
+    const unsigned first = b / (8u * run) * (8u * run);
+    if (first + 8u * run > blocks) return b;
+    const unsigned k = b - first;
+    return first + (k & 7u) * run + (k >> 3);
+}
+
 namespace tfdtd_detail {
 inline thread_local std::string last_error;
 }

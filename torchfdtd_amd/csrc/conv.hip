@@ -8,12 +8,16 @@
 // with k = tap*ci + c, tap = (kd*ks + kh)*ks + kw, zero-padded to kp (a multiple of 32);
 // dgrad weights [ci][ks^3*co] (k = tap*co + c); wgrad reads dY transposed [co][m].
 //
-// One workgroup (4 waves) computes a 64 x 64 tile of C = A B over K in steps of 32: the
-// A tile (64 rows x 32 k) and B tile (64 columns x 32 k) are gathered from global memory
-// (the implicit im2col) into LDS with k fastest, and each wave multiplies its 32 x 32
-// quarter with 2 x 2 v_mfma_f32_16x16x32_bf16.  blockIdx.z splits K for the weight
-// gradient, whose reduction runs over every output position.
+// Layers whose channels are multiples of 8 (and one-channel inputs) take gather_gemm_kernel,
+// narrow_forward_kernel and weight_grad_kernel, further down.  Every other layer takes gemm_kernel: one
+// workgroup (4 waves) computes a 64 x 64 tile of C = A B over K in steps of 32: the A tile (64
+// rows x 32 k) and B tile (64 columns x 32 k) are gathered from global memory (the implicit
+// im2col) into LDS with k fastest, and each wave multiplies its 32 x 32 quarter with 2 x 2
+// v_mfma_f32_16x16x32_bf16.  blockIdx.z splits K for the weight gradient, whose reduction
+// runs over every output position.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "../../include/tfdtd.h"
 #include "common.h"
@@ -23,6 +27,8 @@ namespace {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f4;
 typedef unsigned short bf16_bits;
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef short s8 __attribute__((ext_vector_type(8)));
 
 constexpr int BM = 64, BN = 64, BK = 32, LDK = BK + 8;   // LDS rows padded by 16 bytes
 
@@ -209,13 +215,19 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Gemm g) {
             }
 }
 
-// Sum of the K splits of the weight gradient, in split order.
+// Sum of the K splits of the weight gradient: a workgroup takes 64 values, each of its four wavefronts every
+// fourth split.
 __global__ __launch_bounds__(256) void split_sum_kernel(const float* partial, int splits, long long count, float* out) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
+    __shared__ float sums[3][64];
+    const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+    const long long i = (long long)blockIdx.x * 64 + lane;
     float s = 0.f;
-    for (int z = 0; z < splits; ++z) s += partial[z * count + i];
-    out[i] = s;
+    if (i < count)
+#pragma unroll 4
+        for (int z = part; z < splits; z += 4) s += partial[z * count + i];
+    if (part) sums[part - 1][lane] = s;
+    __syncthreads();
+    if (part == 0 && i < count) out[i] = s + sums[0][lane] + sums[1][lane] + sums[2][lane];
 }
 
 // dPre = dY * GELU'(pre) (or dY), written in FP32 and BF16.
@@ -226,6 +238,745 @@ __global__ __launch_bounds__(256) void gelu_backward_kernel(const float* dy, con
     const float v = activation ? dy[i] * gelu_grad(pre[i]) : dy[i];
     dpre[i] = v;
     dpre16[i] = float_to_bf16(v);
+}
+
+// ---------------------------------------------------------------- gathered GEMM
+//
+// The forward convolution and the input gradient are one contraction: C[row][col] is the sum over taps and
+// source channels of source(row's position under the tap)[c] * weight[col][tap * channels + c].  Rows are
+// output positions (forward) or, for the input gradient, the input positions of one parity class of a
+// strided layer: rows of one class see the same taps, so no tap is multiplied that the stride rules out.
+//
+// A workgroup (4 waves) computes BM rows x BN columns over K in stages of 64: source rows and weight rows
+// go from global memory straight into LDS (16 bytes a lane, no registers), `Depth` - 1 stages ahead of the
+// stage being multiplied.  A lane keeps its rows' addresses and a bit per tap (inside or padding) for the
+// whole loop, so a stage costs it one offset and a select; padding reads a chunk of zeros.  A row's 16-byte
+// chunks lie in LDS at chunk ^ ((row >> 1) & 7), which spreads the 16 rows of one operand read over all
+// banks.  Every product enters its accumulator in the order of gemm_kernel (the same MFMA over ascending K),
+// so results are equal bit for bit; a tap that is padding for every row of the workgroup is skipped when the
+// weights are finite (it would add zeros).
+//
+// 64x32x32x16 positions, 64 -> 128 channels, 3x3x3 (0.46 TFLOP): forward 2.72 -> 0.97 ms (480 TFLOP/s), input
+// gradient 3.5 -> 0.75 ms (620).  gemm_kernel gathered through registers with a division chain per chunk and
+// two barriers per 32 of K; here the staged bytes bound it (32 KB a stage and workgroup, 27 taps of x through
+// L2: about 7 TB/s), the matrix cores are busy a fifth to a quarter of the time.
+typedef __attribute__((address_space(3))) void lds_void;
+
+__device__ const uint4 kZeroChunk = {0u, 0u, 0u, 0u};
+
+// 16 bytes of global memory per lane into LDS at `to` + 16 * lane.
+__device__ __forceinline__ void chunk_to_lds(const void* from, bf16_bits* to) {
+    __builtin_amdgcn_global_load_lds(global(const_cast<void*>(from)), (lds_void*)to, 16, 0, 0);
+}
+
+struct GatherGemm {
+    Conv c;
+    int dgrad;                  // 0 forward, 1 input gradient
+    int rows_max;               // rows of the largest class
+    unsigned run;               // row tiles an XCD takes in a row
+    int N, channels, ldw;       // columns, source channels, weight row length
+    const bf16_bits* source;    // forward: x; input gradient: dY
+    const bf16_bits* weight;    // [N][ldw]
+    const int* nonfinite;       // per part of the weights: 1 where a value is not finite (null: no tap is skipped)
+    int parts;
+    const float* bias;
+    int activation;
+    float* pre;                 // forward: pre-activation (may be null); input gradient: dX
+    float* y;                   // forward: FP32 value of the activation (may be null)
+    bf16_bits* act;             // forward: activation (may be null)
+};
+
+// Four consecutive columns of a row to the outputs: bias, pre-activation, activation; the input gradient as it is.
+__device__ __forceinline__ void finish_columns(const GatherGemm& g, long long cell, int col, f4 v) {
+    if (col + 3 < g.N && g.N % 4 == 0) {
+        const long long o = cell * g.N + col;
+        if (g.dgrad) {
+            *reinterpret_cast<f4*>(g.pre + o) = v;
+            return;
+        }
+        if (g.bias)
+            for (int e = 0; e < 4; ++e) v[e] += g.bias[col + e];
+        if (g.pre) *reinterpret_cast<f4*>(g.pre + o) = v;
+        bf16_bits b[4];
+        for (int e = 0; e < 4; ++e) b[e] = float_to_bf16(g.activation ? gelu(v[e]) : v[e]);
+        if (g.act) *reinterpret_cast<uint2*>(g.act + o) = make_uint2(b[0] | (unsigned)b[1] << 16, b[2] | (unsigned)b[3] << 16);
+        if (g.y) {
+            f4 f;
+            for (int e = 0; e < 4; ++e) f[e] = __uint_as_float((unsigned)b[e] << 16);
+            *reinterpret_cast<f4*>(g.y + o) = f;
+        }
+        return;
+    }
+    for (int e = 0; e < 4; ++e) {
+        if (col + e >= g.N) continue;
+        const long long o = cell * g.N + col + e;
+        float f = v[e];
+        if (!g.dgrad && g.bias) f += g.bias[col + e];
+        if (g.pre) g.pre[o] = f;
+        if (g.dgrad) continue;
+        const bf16_bits b = float_to_bf16(g.activation ? gelu(f) : f);
+        if (g.act) g.act[o] = b;
+        if (g.y) g.y[o] = __uint_as_float((unsigned)b << 16);
+    }
+}
+
+// One axis of the rows: its length, where tap k of row q lies (q * mul + at(k)), and where row q itself lies.
+struct RowAxis {
+    int rows, source, mul, first, shift, sign, out_mul;
+    __device__ __forceinline__ int at(int k) const { return (first + sign * k) >> shift; }
+    __device__ __forceinline__ bool meets(int k) const { return ((first + sign * k) & ((1 << shift) - 1)) == 0; }
+};
+
+__device__ __forceinline__ RowAxis row_axis(const GatherGemm& g, int in, int out, int parity, int* begin) {
+    RowAxis a;
+    if (!g.dgrad) {
+        *begin = 0;
+        a = RowAxis{out, in, g.c.stride, -g.c.pad, 0, 1, 1};
+    } else if (g.c.stride == 1) {
+        *begin = 0;
+        a = RowAxis{in, out, 1, g.c.pad, 0, -1, 1};
+    } else {
+        *begin = (parity + g.c.pad) & 1;      // first position z with (z + pad) % 2 == parity
+        a = RowAxis{(in - *begin + 1) >> 1, out, 1, *begin + g.c.pad, 1, -1, 2};
+    }
+    return a;
+}
+
+// K in pieces of 32: (tap, channel) of each, taps in ascending order from a mask.
+struct Pieces {
+    unsigned left;
+    int tap, c;
+    bool more;
+    __device__ __forceinline__ void start(unsigned mask) {
+        more = mask != 0;
+        tap = more ? __builtin_ctz(mask) : 0;
+        left = mask & (mask - 1u);
+        c = 0;
+    }
+    __device__ __forceinline__ void next(int channels) {
+        c += 32;
+        if (c < channels) return;
+        c = 0;
+        more = left != 0;
+        if (more) {
+            tap = __builtin_ctz(left);
+            left &= left - 1u;
+        }
+    }
+};
+
+// `Whole`: the channels are a multiple of 32, so a piece of 32 has one tap; otherwise (a multiple of 8) each
+// 16-byte chunk finds its own.
+template <int BM, int BN, int WM, int WN, int Depth, bool Whole>
+__global__ __launch_bounds__(256) void gather_gemm_kernel(const GatherGemm g) {
+    constexpr int XI = BM / 32, WI = BN / 32;          // staging instructions per wave
+    constexpr int RT = WM / 16, CT = WN / 16;          // 16-row and 16-column tiles per wave
+    constexpr int Stage = (BM + BN) * 64;
+    __shared__ __attribute__((aligned(16))) bf16_bits s0[Stage];
+    __shared__ __attribute__((aligned(16))) bf16_bits s1[Stage];
+    __shared__ __attribute__((aligned(16))) bf16_bits s2[Depth > 2 ? Stage : 8];
+    __shared__ unsigned s_mask, s_bad;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Conv& c = g.c;
+    const int ks = c.ks, taps = ks * ks * ks, C = g.channels;
+    const int cls = blockIdx.z;
+    int begin[3];
+    const RowAxis ax[3] = {row_axis(g, c.di, c.dout, cls & 1, &begin[0]), row_axis(g, c.hi, c.hout, (cls >> 1) & 1, &begin[1]),
+                           row_axis(g, c.wi, c.wout, cls >> 2, &begin[2])};
+    const int rows = c.n * ax[0].rows * ax[1].rows * ax[2].rows;
+    const int row0 = (int)xcd_block(blockIdx.x, gridDim.x, g.run) * BM, col0 = blockIdx.y * BN;
+    if (row0 >= rows) return;                          // a smaller class: the whole workgroup leaves
+    if (tid == 0) { s_mask = 0u; s_bad = 0u; }
+    __syncthreads();
+    // Rows of this lane: position under tap offset 0 and a bit per tap that lies inside the source.
+    const bf16_bits* row_at[XI];
+    unsigned row_taps[XI], any = 0u;
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int row = row0 + (wave * XI + i) * 8 + (lane >> 3);
+        unsigned mask = 0u;
+        long long cell = 0;
+        if (row < rows) {
+            int q[3], t = row / ax[2].rows;
+            q[2] = row - t * ax[2].rows;
+            const int u = t / ax[1].rows;
+            q[1] = t - u * ax[1].rows;
+            const int nb = u / ax[0].rows;
+            q[0] = u - nb * ax[0].rows;
+            unsigned in[3];
+            for (int a = 0; a < 3; ++a) {
+                in[a] = 0u;
+                for (int k = 0; k < ks; ++k) {
+                    const int p = q[a] * ax[a].mul + ax[a].at(k);
+                    if (ax[a].meets(k) && p >= 0 && p < ax[a].source) in[a] |= 1u << k;
+                }
+            }
+            for (int kd = 0; kd < ks; ++kd)
+                for (int kh = 0; kh < ks; ++kh)
+                    if ((in[0] >> kd & 1u) && (in[1] >> kh & 1u)) mask |= in[2] << ((kd * ks + kh) * ks);
+            cell = (((long long)nb * ax[0].source + q[0] * ax[0].mul) * ax[1].source + q[1] * ax[1].mul) * ax[2].source + q[2] * ax[2].mul;
+        }
+        row_at[i] = g.source + cell * C;
+        row_taps[i] = mask;
+        any |= mask;
+    }
+    unsigned todo = taps == 32 ? ~0u : (1u << taps) - 1u;
+    if (Whole && g.nonfinite) {
+        int bad = 0;
+        for (int i = tid; i < g.parts; i += 256) bad |= g.nonfinite[i];
+        atomicOr(&s_mask, any);
+        if (bad) s_bad = 1u;
+        __syncthreads();
+        if (!s_bad) todo = s_mask;
+        todo = (unsigned)__builtin_amdgcn_readfirstlane((int)todo);
+    }
+    // Elements from a row's position under tap offset 0 to its position under a tap (one sample is below 2^31).
+    auto tap_offset = [&](int tap) -> int {
+        const int kd = tap * 57 >> 9, r = tap - 9 * kd, kh = r * 11 >> 5, kw = r - 3 * kh;     // tap / 9, / 3, % 3 (one tap: 0)
+        return ((ax[0].at(kd) * ax[1].source + ax[1].at(kh)) * ax[2].source + ax[2].at(kw)) * C;
+    };
+    const int pieces = Whole ? __popc(todo) * (C / 32) : (taps * C + 31) / 32;
+    const int stages = (pieces + 1) / 2;
+    // A lane's two kinds of chunk (even and odd i): position (lane & 7) of its row holds chunk (lane & 7) ^ swizzle.
+    const int odd = wave * XI & 1;
+    const int chunk_of[2] = {(lane & 7) ^ (((lane >> 4) + 4 * odd) & 7), (lane & 7) ^ (((lane >> 4) + 4 * (odd ^ 1)) & 7)};
+    Pieces at;
+    at.start(todo);
+    int own_tap[2] = {0, 0}, own_c[2] = {0, 0};        // !Whole: the chunk's own tap and channel
+    if (!Whole)
+        for (int v = 0; v < 2; ++v) {
+            own_tap[v] = chunk_of[v] * 8 / C;
+            own_c[v] = chunk_of[v] * 8 % C;
+        }
+    int staged = 0;
+    const bf16_bits* const zero = reinterpret_cast<const bf16_bits*>(&kZeroChunk);
+    auto stage = [&](bf16_bits* into) {
+        int offset[2] = {0, 0};
+        unsigned bit[2] = {0u, 0u};
+        int k[2] = {0, 0};
+        if (Whole) {
+            for (int h = 0; h < 2; ++h) {
+                if (at.more) {
+                    offset[h] = tap_offset(at.tap) + at.c;
+                    bit[h] = 1u << at.tap;
+                    k[h] = at.tap * C + at.c;
+                } else {
+                    k[h] = -1;
+                }
+                at.next(C);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int chunk = chunk_of[i & 1], half = chunk >> 2, within = (chunk & 3) * 8;
+            const bf16_bits* from = zero;
+            if (Whole) {
+                if (row_taps[i] & (half ? bit[1] : bit[0])) from = row_at[i] + (half ? offset[1] : offset[0]) + within;
+            } else if (own_tap[i & 1] < taps && (row_taps[i] >> own_tap[i & 1] & 1u)) {
+                from = row_at[i] + tap_offset(own_tap[i & 1]) + own_c[i & 1];
+            }
+            chunk_to_lds(from, into + (wave * XI + i) * 512);
+        }
+        bf16_bits* const weights = into + BM * 64;
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            const int r = (wave * WI + i) * 8 + (lane >> 3);
+            const int chunk = (lane & 7) ^ ((r >> 1) & 7), half = chunk >> 2, within = (chunk & 3) * 8;
+            const int kk = Whole ? (half ? k[1] : k[0]) : staged * 64 + half * 32;
+            const bf16_bits* from = zero;
+            if (col0 + r < g.N && kk >= 0 && kk + within < g.ldw) from = g.weight + (long long)(col0 + r) * g.ldw + kk + within;
+            chunk_to_lds(from, weights + (wave * WI + i) * 512);
+        }
+        ++staged;
+        if (!Whole)
+            for (int v = 0; v < 2; ++v) {
+                own_c[v] += 64;
+                while (own_c[v] >= C) { own_c[v] -= C; ++own_tap[v]; }
+            }
+    };
+    const int wm = wave / (BN / WN) * WM, wn = wave % (BN / WN) * WN;
+    f4 acc[CT][RT];
+#pragma unroll
+    for (int i = 0; i < CT; ++i)
+#pragma unroll
+        for (int j = 0; j < RT; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    const int fr = lane & 15, fc = lane >> 4, fs = (fr >> 1) & 7;   // operand row, chunk and swizzle of a lane
+    auto multiply = [&](const bf16_bits* from, int number) {
+        const bf16_bits* const weights = from + BM * 64;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (h == 1 && 2 * number + 1 >= pieces) break;
+            const int place = ((4 * h + fc) ^ fs) * 8;
+            bf16x8 x[RT], w[CT];
+#pragma unroll
+            for (int j = 0; j < RT; ++j) x[j] = *reinterpret_cast<const bf16x8*>(from + (wm + 16 * j + fr) * 64 + place);
+#pragma unroll
+            for (int i = 0; i < CT; ++i) w[i] = *reinterpret_cast<const bf16x8*>(weights + (wn + 16 * i + fr) * 64 + place);
+#pragma unroll
+            for (int i = 0; i < CT; ++i)
+#pragma unroll
+                for (int j = 0; j < RT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], x[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    // The barrier after a stage's loads have landed (all but those of later stages) also ends the reads of the
+    // buffer that the next loads overwrite.
+    constexpr int PerStage = XI + WI;
+    auto arrive = [&](bool later) {
+        asm volatile("" ::: "memory");
+        if (Depth > 2 && later) __builtin_amdgcn_s_waitcnt(0x0f70 | PerStage);      // vmcnt(PerStage)
+        else __builtin_amdgcn_s_waitcnt(0x0f70);                                    // vmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (stages > 0) stage(s0);
+    if (Depth > 2 && stages > 1) stage(s1);
+    for (int s = 0; s < stages;) {
+        arrive(Depth > 2 && s + 1 < stages);
+        if (Depth == 2) { if (s + 1 < stages) stage(s1); }
+        else if (s + 2 < stages) stage(s2);
+        multiply(s0, s);
+        if (++s >= stages) break;
+        arrive(Depth > 2 && s + 1 < stages);
+        if (Depth == 2) { if (s + 1 < stages) stage(s0); }
+        else if (s + 2 < stages) stage(s0);
+        multiply(s1, s);
+        if (++s >= stages) break;
+        if (Depth > 2) {
+            arrive(s + 1 < stages);
+            if (s + 2 < stages) stage(s1);
+            multiply(s2, s);
+            ++s;
+        }
+    }
+    // A lane holds four consecutive columns of one row per tile.
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+        const int row = row0 + wm + 16 * j + fr;
+        if (row >= rows) continue;
+        long long cell = row;
+        if (g.dgrad) {
+            int t = row / ax[2].rows;
+            const int qx = row - t * ax[2].rows, u = t / ax[1].rows;
+            const int qy = t - u * ax[1].rows, nb = u / ax[0].rows, qz = u - nb * ax[0].rows;
+            cell = (((long long)nb * c.di + qz * ax[0].out_mul + begin[0]) * c.hi + qy * ax[1].out_mul + begin[1]) * c.wi +
+                   qx * ax[2].out_mul + begin[2];
+        }
+#pragma unroll
+        for (int i = 0; i < CT; ++i) {
+            const int col = col0 + wn + 16 * i + fc * 4;
+            finish_columns(g, cell, col, acc[i][j]);
+        }
+    }
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// Row tiles that one XCD takes in a row, so that the taps' overlapping rows are read through one L2.
+constexpr unsigned kRowRun = 64;
+
+template <int BM, int BN, int WM, int WN, int Depth>
+void launch_gather(GatherGemm g, int classes, hipStream_t stream) {
+    g.run = kRowRun;
+    const dim3 grid((g.rows_max + BM - 1) / BM, (g.N + BN - 1) / BN, classes), block(256);
+    if (g.channels % 32 == 0) hipLaunchKernelGGL((gather_gemm_kernel<BM, BN, WM, WN, Depth, true>), grid, block, 0, stream, g);
+    else hipLaunchKernelGGL((gather_gemm_kernel<BM, BN, WM, WN, Depth, false>), grid, block, 0, stream, g);
+}
+
+// FP32 weights [co][taps][ci] to the bf16 operands of the forward convolution, [co][kp], and of the input
+// gradient, [ci][taps * co] (transposed through LDS), and per tap and 32 x 32 channels whether a value is not finite.
+__global__ __launch_bounds__(256) void weights_kernel(const float* weight, int co, int ci, int taps, int kp, bf16_bits* w16,
+                                                      bf16_bits* transposed, int* nonfinite) {
+    __shared__ bf16_bits tile[32][33];
+    __shared__ int bad;
+    const int tap = blockIdx.x, c0 = blockIdx.y * 32, o0 = blockIdx.z * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    if (threadIdx.x == 0) bad = 0;
+    __syncthreads();
+    bool mine = false;
+    for (int r = ty; r < 32; r += 8) {
+        const int o = o0 + r, c = c0 + tx;
+        if (o < co && c < ci) {
+            const bf16_bits b = float_to_bf16(weight[((long long)o * taps + tap) * ci + c]);
+            mine |= (b & 0x7f80u) == 0x7f80u;      // infinite or NaN, also a finite value that rounds to infinity
+            w16[(long long)o * kp + tap * ci + c] = b;
+            tile[r][tx] = b;
+        }
+        if (tap == taps - 1 && o < co && c0 + 32 >= ci)
+            for (int k = taps * ci + tx; k < kp; k += 32) w16[(long long)o * kp + k] = 0;
+    }
+    __syncthreads();
+    if (transposed)
+        for (int r = ty; r < 32; r += 8) {
+            const int c = c0 + r, o = o0 + tx;
+            if (c < ci && o < co) transposed[((long long)c * taps + tap) * co + o] = tile[tx][r];
+        }
+    if (mine) bad = 1;
+    __syncthreads();
+    if (threadIdx.x == 0) nonfinite[(blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = bad;
+}
+
+// Forward convolution with at most 32 values of K (a one-channel input): no staging pays, a wavefront takes
+// 64 rows, gathers each row's K values into the MFMA operand and keeps the weights of its columns in
+// registers.  Bound by its outputs: 524,288 rows x 32 columns, pre-activation and value in FP32: 57 us
+// against 107 for gemm_kernel and the conversion pass.
+template <int CT>
+__global__ __launch_bounds__(256) void narrow_forward_kernel(const GatherGemm g, int rows, Divider by_w, Divider by_h, Divider by_d) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Conv& c = g.c;
+    const int col0 = blockIdx.y * CT * 16, fr = lane & 15, fc = lane >> 4;
+    bf16x8 w[CT];
+#pragma unroll
+    for (int i = 0; i < CT; ++i) {
+        s8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+        const int col = col0 + 16 * i + fr;
+        if (col < g.N) v = *reinterpret_cast<const s8*>(g.weight + (long long)col * 32 + fc * 8);
+        w[i] = __builtin_bit_cast(bf16x8, v);
+    }
+    const int ks = c.ks, kmax = ks * ks * ks * c.ci;
+    int tz[8], ty[8], tx[8], at[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const int k = fc * 8 + t, tap = k / c.ci;
+        tx[t] = k < kmax ? tap % ks - c.pad : -0x40000000;      // never inside
+        ty[t] = tap / ks % ks - c.pad;
+        tz[t] = tap / (ks * ks) - c.pad;
+        at[t] = ((tz[t] * c.hi + ty[t]) * c.wi + (tap % ks - c.pad)) * c.ci + (k - tap * c.ci);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = (blockIdx.x * 4 + wave) * 64 + 16 * j + fr;
+        const unsigned u = divide((unsigned)row, by_w), v = divide(u, by_h), nb = divide(v, by_d);
+        const int x = (row - (int)u * c.wout) * c.stride, y = (int)(u - v * c.hout) * c.stride, z = (int)(v - nb * c.dout) * c.stride;
+        const bf16_bits* const from = g.source + ((((long long)nb * c.di + z) * c.hi + y) * c.wi + x) * c.ci;
+        s8 taken;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            taken[t] = 0;
+            if (row < rows && (unsigned)(x + tx[t]) < (unsigned)c.wi && (unsigned)(y + ty[t]) < (unsigned)c.hi &&
+                (unsigned)(z + tz[t]) < (unsigned)c.di)
+                taken[t] = (short)from[at[t]];
+        }
+#pragma unroll
+        for (int i = 0; i < CT; ++i) {
+            const f4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], __builtin_bit_cast(bf16x8, taken), f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            if (row < rows) finish_columns(g, row, col0 + 16 * i + fc * 4, sum);
+        }
+    }
+}
+
+// Runs the gathered GEMM when source and weights allow 16-byte chunks; false leaves it to gemm_kernel.
+bool gather_gemm(GatherGemm g, hipStream_t stream) {
+    const long long inside = (long long)g.c.di * g.c.hi * g.c.wi, outside = (long long)g.c.dout * g.c.hout * g.c.wout;
+    if (g.c.n * inside > 0x7fffffffLL || inside * g.channels > 0x7fffffffLL || outside * g.channels > 0x7fffffffLL) return false;
+    if (g.N % 4 == 0 && (!aligned16(g.pre) || !aligned16(g.y) || (reinterpret_cast<uintptr_t>(g.act) & 7u))) return false;
+    if (!g.dgrad && g.ldw == 32 && aligned16(g.weight)) {
+        const int rows = g.c.n * g.c.dout * g.c.hout * g.c.wout, columns = g.N <= 32 ? 2 : 4;
+        const dim3 grid((rows + 255) / 256, (g.N + columns * 16 - 1) / (columns * 16)), block(256);
+        const Divider w = make_divider((unsigned)g.c.wout), h = make_divider((unsigned)g.c.hout), d = make_divider((unsigned)g.c.dout);
+        if (columns == 2) hipLaunchKernelGGL(narrow_forward_kernel<2>, grid, block, 0, stream, g, rows, w, h, d);
+        else hipLaunchKernelGGL(narrow_forward_kernel<4>, grid, block, 0, stream, g, rows, w, h, d);
+        return true;
+    }
+    if (g.channels % 8 || !aligned16(g.source) || !aligned16(g.weight) || g.ldw % 8) return false;
+    int classes = 1;
+    if (g.dgrad && g.c.stride == 2) {
+        classes = 8;
+        g.rows_max = g.c.n * ((g.c.di + 1) / 2) * ((g.c.hi + 1) / 2) * ((g.c.wi + 1) / 2);
+    } else {
+        g.rows_max = g.dgrad ? g.c.n * g.c.di * g.c.hi * g.c.wi : g.c.n * g.c.dout * g.c.hout * g.c.wout;
+    }
+    // The largest tile that still gives each CU two workgroups: its operands are staged least often.  Layers
+    // of few rows take small tiles three stages deep, bound by the latency of their K loop: 2048 rows of 256
+    // columns (8x8x1 x 128 channels in, stride 2) make 32 tiles of 128 x 128 and 256 of 32 x 64.
+    auto blocks = [&](int bm, int bn) { return (long long)((g.rows_max + bm - 1) / bm) * ((g.N + bn - 1) / bn) * classes; };
+    if (g.N <= 32) {
+        if (blocks(128, 32) >= 512) launch_gather<128, 32, 32, 32, 2>(g, classes, stream);
+        else launch_gather<32, 32, 16, 16, 3>(g, classes, stream);
+    } else if (g.N > 64 && blocks(128, 128) >= 512) {
+        launch_gather<128, 128, 64, 64, 2>(g, classes, stream);
+    } else if (blocks(128, 64) >= 512) {
+        launch_gather<128, 64, 64, 32, 2>(g, classes, stream);
+    } else if (blocks(64, 64) >= 512) {
+        launch_gather<64, 64, 32, 32, 3>(g, classes, stream);
+    } else {
+        launch_gather<32, 64, 16, 32, 3>(g, classes, stream);
+    }
+    return true;
+}
+
+// ---------------------------------------------------------------- weight gradient
+//
+// dW[co][k] is the sum over output positions m of dY[m][co] * im2col(m)[k].  Both operands lie with the
+// reduction m slowest, so stages of 64 positions go into LDS as they are (rows of dY, gathered 16-byte
+// chunks of x) and each MFMA operand is read transposed (ds_read_b64_tr_b16: 4 positions x 16 columns a
+// group of 16 lanes) -- no transposed copy of dY in memory.  Chunks lie at chunk ^ swizzle(row), which spreads
+// the 16 rows of a transposed read over the banks.  The positions are split over blockIdx.z; each split
+// writes its partial sums, which split_sum_kernel adds.  64x32x32x16 positions, 64 -> 128 channels: 0.97 ms
+// (480 TFLOP/s), against 3.1 ms and 1.2 ms for the transposed copy of dY.
+
+struct WeightGrad {
+    Conv c;
+    const bf16_bits* dy;        // [m][co]
+    const bf16_bits* x;
+    float* partial;             // [split][co][kp]
+    int m_total, per_split;
+    Divider by_w, by_h, by_d;
+};
+
+template <int Chunks>
+__device__ __forceinline__ int row_swizzle(int row) {
+    if (Chunks == 16) return 2 * ((row & 3) | (row >> 3 & 1) << 2);
+    if (Chunks == 8) return 2 * ((row >> 1 & 1) | (row >> 3 & 1) << 1);
+    return 2 * (row >> 3 & 1);
+}
+
+// Operand of 16 columns from column `col` (a multiple of 16) and 32 rows from `row` of a [64][Columns] stage.
+template <int Columns>
+__device__ __forceinline__ bf16x8 transposed(const bf16_bits* stage, int row, int col, int lane) {
+    constexpr int Chunks = Columns / 8;
+    const int r = row + (lane >> 4) * 8 + ((lane & 15) >> 2);
+    const int chunk = (col / 8 + ((lane & 3) >> 1)) ^ row_swizzle<Chunks>(r);
+    const bf16_bits* at = stage + r * Columns + chunk * 8 + (lane & 1) * 4;
+    typedef __attribute__((address_space(3))) s4 lds_s4;
+    const s4 low = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)at);
+    const s4 high = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(at + 4 * Columns));
+    const s8 both = __builtin_shufflevector(low, high, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, both);
+}
+
+template <int BC, int BK>
+__global__ __launch_bounds__(256, 2) void weight_grad_kernel(const WeightGrad g) {
+    constexpr int DC = BC / 8, XC = BK / 8;                     // 16-byte chunks of a row
+    constexpr int DI = BC / 32, XI = BK / 32;                   // staging instructions per wave
+    constexpr int WC = BC / 2, WK = BK / 2, CT = WC / 16, KT = WK / 16;
+    constexpr int Stage = 64 * (BC + BK);
+    __shared__ __attribute__((aligned(16))) bf16_bits s0[Stage];
+    __shared__ __attribute__((aligned(16))) bf16_bits s1[Stage];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Conv& c = g.c;
+    const int co0 = blockIdx.x * BC, k0 = blockIdx.y * BK;
+    const int begin = blockIdx.z * g.per_split, end = min(g.m_total, begin + g.per_split);
+    const bf16_bits* const zero = reinterpret_cast<const bf16_bits*>(&kZeroChunk);
+    // The x chunk of each staging instruction: its tap and channel stay for the whole loop.
+    int tap_z[XI], tap_y[XI], tap_x[XI], channel[XI];
+    const int ks = c.ks, kmax = ks * ks * ks * c.ci;
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int row = (wave * XI + i) * (64 / XC) + lane / XC;
+        const int k = k0 + ((lane % XC) ^ row_swizzle<XC>(row)) * 8;
+        const int tap = k / c.ci;
+        channel[i] = k < kmax ? k - tap * c.ci : -1;
+        tap_x[i] = tap % ks - c.pad;
+        tap_y[i] = tap / ks % ks - c.pad;
+        tap_z[i] = tap / (ks * ks) - c.pad;
+    }
+    auto stage = [&](bf16_bits* into, int m0) {
+#pragma unroll
+        for (int i = 0; i < DI; ++i) {
+            const int row = (wave * DI + i) * (64 / DC) + lane / DC;
+            const int col = co0 + ((lane % DC) ^ row_swizzle<DC>(row)) * 8, m = m0 + row;
+            const bf16_bits* from = m < end && col < c.co ? g.dy + (long long)m * c.co + col : zero;
+            chunk_to_lds(from, into + (wave * DI + i) * 512);
+        }
+        bf16_bits* const xs = into + 64 * BC;
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int m = m0 + (wave * XI + i) * (64 / XC) + lane / XC;
+            const unsigned u = divide((unsigned)m, g.by_w), v = divide(u, g.by_h), nb = divide(v, g.by_d);
+            const int x = (m - (int)u * c.wout) * c.stride + tap_x[i], y = (int)(u - v * c.hout) * c.stride + tap_y[i];
+            const int z = (int)(v - nb * c.dout) * c.stride + tap_z[i];
+            const bf16_bits* from = zero;
+            if (m < end && channel[i] >= 0 && (unsigned)x < (unsigned)c.wi && (unsigned)y < (unsigned)c.hi && (unsigned)z < (unsigned)c.di)
+                from = g.x + ((((long long)nb * c.di + z) * c.hi + y) * c.wi + x) * c.ci + channel[i];
+            chunk_to_lds(from, xs + (wave * XI + i) * 512);
+        }
+    };
+    const int wc = (wave & 1) * WC, wk = (wave >> 1) * WK;
+    f4 acc[KT][CT];
+#pragma unroll
+    for (int i = 0; i < KT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const bf16_bits* from) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            bf16x8 d[CT], x[KT];
+#pragma unroll
+            for (int j = 0; j < CT; ++j) d[j] = transposed<BC>(from, 32 * h, wc + 16 * j, lane);
+#pragma unroll
+            for (int i = 0; i < KT; ++i) x[i] = transposed<BK>(from + 64 * BC, 32 * h, wk + 16 * i, lane);
+#pragma unroll
+            for (int i = 0; i < KT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i], d[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    auto arrive = [&] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0): this wave's stage has landed
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (begin < end) stage(s0, begin);
+    for (int m = begin; m < end; m += 128) {
+        arrive();
+        if (m + 64 < end) stage(s1, m + 64);
+        multiply(s0);
+        if (m + 64 >= end) break;
+        arrive();
+        if (m + 128 < end) stage(s0, m + 128);
+        multiply(s1);
+    }
+    float* const out = g.partial + (long long)blockIdx.z * c.co * c.kp;
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+        const int co = co0 + wc + 16 * j + (lane & 15);
+        if (co >= c.co) continue;
+#pragma unroll
+        for (int i = 0; i < KT; ++i) {
+            const int k = k0 + wk + 16 * i + (lane >> 4) * 4;
+            if (k < c.kp) *reinterpret_cast<f4*>(out + (long long)co * c.kp + k) = acc[i][j];
+        }
+    }
+}
+
+// The same for at most 32 values of k (a one-channel input): a wavefront gathers its operands from global
+// memory element by element -- 32 positions of dY rows and of the 27 shifted inputs -- and the four
+// wavefronts of a workgroup add their sums in LDS.  524,288 positions, 1 -> 32 channels: 71 us against
+// 2.2 ms (64 workgroups of gemm_kernel, each gathering 8,192 positions one value at a time).
+constexpr int kNarrowColumns = 32;
+
+__global__ __launch_bounds__(256) void weight_grad_narrow_kernel(const WeightGrad g) {
+    __shared__ float sums[4][kNarrowColumns][33];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Conv& c = g.c;
+    const int co0 = blockIdx.x * kNarrowColumns;
+    const int begin = blockIdx.z * g.per_split, end = min(g.m_total, begin + g.per_split);
+    const int ks = c.ks, kmax = ks * ks * ks * c.ci;
+    int tz[2], ty[2], tx[2], ch[2];
+    for (int i = 0; i < 2; ++i) {
+        const int k = 16 * i + (lane & 15), tap = k / c.ci;
+        ch[i] = k < kmax ? k - tap * c.ci : -1;
+        tx[i] = tap % ks - c.pad;
+        ty[i] = tap / ks % ks - c.pad;
+        tz[i] = tap / (ks * ks) - c.pad;
+    }
+    f4 acc[2][2];
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int m0 = begin + wave * 32; m0 < end; m0 += 128) {
+        s8 x[2], d[2];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int m = m0 + (lane >> 4) * 8 + t;
+            const unsigned u = divide((unsigned)m, g.by_w), v = divide(u, g.by_h), nb = divide(v, g.by_d);
+            const int px = (m - (int)u * c.wout) * c.stride, py = (int)(u - v * c.hout) * c.stride, pz = (int)(v - nb * c.dout) * c.stride;
+            for (int i = 0; i < 2; ++i) {
+                const int xx = px + tx[i], yy = py + ty[i], zz = pz + tz[i];
+                x[i][t] = 0;
+                if (m < end && ch[i] >= 0 && (unsigned)xx < (unsigned)c.wi && (unsigned)yy < (unsigned)c.hi && (unsigned)zz < (unsigned)c.di)
+                    x[i][t] = (short)g.x[((((long long)nb * c.di + zz) * c.hi + yy) * c.wi + xx) * c.ci + ch[i]];
+            }
+            for (int j = 0; j < 2; ++j) {
+                const int co = co0 + 16 * j + (lane & 15);
+                d[j][t] = 0;
+                if (m < end && co < c.co) d[j][t] = (short)g.dy[(long long)m * c.co + co];
+            }
+        }
+        for (int i = 0; i < 2; ++i)
+            for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x[i]), __builtin_bit_cast(bf16x8, d[j]),
+                                                                    acc[i][j], 0, 0, 0);
+    }
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j)
+            for (int e = 0; e < 4; ++e) sums[wave][16 * j + (lane & 15)][16 * i + (lane >> 4) * 4 + e] = acc[i][j][e];
+    __syncthreads();
+    for (int e = tid; e < kNarrowColumns * 32; e += 256) {
+        const int co = e >> 5, k = e & 31;
+        if (co0 + co < c.co)
+            g.partial[((long long)blockIdx.z * c.co + co0 + co) * c.kp + k] =
+                sums[0][co][k] + sums[1][co][k] + sums[2][co][k] + sums[3][co][k];
+    }
+}
+
+// Column tiles and K tiles of the weight gradient; 0 where it is left to gemm_kernel.
+struct WeightGradShape {
+    int bc, bk, splits;
+};
+
+WeightGradShape weight_grad_shape(const tfdtd_conv& d, const Conv& c) {
+    const long long m = (long long)d.n * c.dout * c.hout * c.wout;
+    if (m > 0x7fffffffLL - 256) return {0, 0, 0};
+    long long tiles, least;          // workgroups per split, positions a split takes at least
+    WeightGradShape s{0, 0, 0};
+    if (d.kp == 32) {
+        s.bc = kNarrowColumns; s.bk = 32;
+        tiles = (d.co + s.bc - 1) / s.bc;
+        least = 256;
+    } else if (d.ci % 8 == 0 && d.co % 8 == 0) {
+        s.bc = d.co <= 32 ? 32 : d.co <= 64 ? 64 : 128;
+        s.bk = 128;
+        tiles = (long long)((d.co + s.bc - 1) / s.bc) * ((d.kp + s.bk - 1) / s.bk);
+        least = 256;
+    } else {
+        return s;
+    }
+    // Enough workgroups to fill the chip, and no FP32 sum longer than 12,288 positions (4,096 up to 64 splits).
+    const long long fill = std::min<long long>(768 / tiles, (m + least - 1) / least);
+    const long long precise = std::max<long long>((m + 12287) / 12288, std::min<long long>(64, m / 4096));
+    s.splits = (int)std::max<long long>(1, std::min<long long>(std::max(fill, precise), 512));
+    return s;
+}
+
+// dPre = dY * GELU'(pre) (or dY) in bf16, and its sum over the rows before the rounding: each thread keeps
+// four channels and adds its rows in FP64, the workgroup adds its threads, bias_sum_kernel adds the workgroups.
+// Memory-bound (8 bytes read, 2 written a value): 1.34 GB in 315 us (4.3 TB/s) on 1 M rows of 128; the FP32 copy
+// of dPre and its separate sum took 430 + 168 us.
+constexpr int kBiasBlocks = TFDTD_BIAS_BLOCKS;
+
+typedef __attribute__((ext_vector_type(4))) double d4;
+
+__global__ __launch_bounds__(256) void gelu_backward_rows_kernel(const float* dy, const float* pre, long long rows, int channels,
+                                                                int activation, bf16_bits* dpre16, double* partial) {
+    __shared__ d4 sums[256];
+    const int quads = channels / 4, per = 256 / quads, q = threadIdx.x % quads, r = threadIdx.x / quads;
+    d4 sum = d4{0., 0., 0., 0.};
+    if (r < per)
+        for (long long row = (long long)blockIdx.x * per + r; row < rows; row += (long long)gridDim.x * per) {
+            const long long o = row * channels + 4 * q;
+            const f4 d = *reinterpret_cast<const f4*>(dy + o);
+            f4 v = d;
+            if (activation) {
+                const f4 p = *reinterpret_cast<const f4*>(pre + o);
+                for (int e = 0; e < 4; ++e) v[e] = d[e] * gelu_grad(p[e]);
+            }
+            for (int e = 0; e < 4; ++e) sum[e] += (double)v[e];
+            *reinterpret_cast<uint2*>(dpre16 + o) = make_uint2(float_to_bf16(v[0]) | (unsigned)float_to_bf16(v[1]) << 16,
+                                                              float_to_bf16(v[2]) | (unsigned)float_to_bf16(v[3]) << 16);
+        }
+    sums[threadIdx.x] = sum;
+    __syncthreads();
+    if (r == 0) {
+        for (int k = 1; k < per; ++k) sum += sums[k * quads + q];
+        *reinterpret_cast<d4*>(partial + (long long)blockIdx.x * channels + 4 * q) = sum;
+    }
+}
+
+__global__ __launch_bounds__(1024) void bias_sum_kernel(const double* partial, int blocks, int channels, float* out) {
+    __shared__ double sums[32][32];
+    const int c = blockIdx.x * 32 + (threadIdx.x & 31), part = threadIdx.x >> 5;
+    double s = 0.;
+    if (c < channels)
+#pragma unroll 4
+        for (int b = part; b < blocks; b += 32) s += partial[(long long)b * channels + c];
+    sums[part][threadIdx.x & 31] = s;
+    __syncthreads();
+    if (part == 0 && c < channels) {
+        for (int k = 1; k < 32; ++k) s += sums[k][threadIdx.x];
+        out[c] = (float)s;
+    }
 }
 
 int check_conv(const tfdtd_conv& d) {
@@ -281,6 +1032,13 @@ int tfdtd_conv_forward(const tfdtd_conv* d, const void* x, const void* weight, c
     g.out = pre;
     g.act = static_cast<bf16_bits*>(act);
     if ((long long)d->n * g.c.dout * g.c.hout * g.c.wout > 0x7fffffffLL) return tfdtd_fail(TFDTD_EINVAL, "conv: too many positions");
+    GatherGemm h{};
+    h.c = g.c;
+    h.N = d->co; h.channels = d->ci; h.ldw = d->kp;
+    h.source = g.a; h.weight = g.b;
+    h.bias = bias; h.activation = activation;
+    h.pre = pre; h.act = g.act;
+    if (gather_gemm(h, static_cast<hipStream_t>(stream))) return tfdtd_check_launch("conv forward");
     hipLaunchKernelGGL(gemm_kernel, dim3((g.M + BM - 1) / BM, (g.N + BN - 1) / BN, 1), dim3(256), 0,
                        static_cast<hipStream_t>(stream), g);
     return tfdtd_check_launch("conv forward");
@@ -301,6 +1059,13 @@ int tfdtd_conv_dgrad(const tfdtd_conv* d, const void* dy, const void* weight_t, 
     g.a = static_cast<const bf16_bits*>(dy);
     g.b = static_cast<const bf16_bits*>(weight_t);
     g.out = dx;
+    GatherGemm h{};
+    h.c = g.c;
+    h.dgrad = 1;
+    h.N = d->ci; h.channels = d->co; h.ldw = g.K;
+    h.source = g.a; h.weight = g.b;
+    h.pre = dx;
+    if (gather_gemm(h, static_cast<hipStream_t>(stream))) return tfdtd_check_launch("conv dgrad");
     hipLaunchKernelGGL(gemm_kernel, dim3((g.M + BM - 1) / BM, (g.N + BN - 1) / BN, 1), dim3(256), 0,
                        static_cast<hipStream_t>(stream), g);
     return tfdtd_check_launch("conv dgrad");
@@ -328,8 +1093,117 @@ int tfdtd_conv_wgrad(const tfdtd_conv* d, const void* dy_t, const void* x, int32
     status = tfdtd_check_launch("conv wgrad");
     if (status) return status;
     const long long count = (long long)g.M * g.N;
-    hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, partial, used, count, dw);
+    hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((count + 63) / 64)), dim3(256), 0, s, partial, used, count, dw);
     return tfdtd_check_launch("conv wgrad sum");
+}
+
+int tfdtd_conv_weight_parts(const tfdtd_conv* d) {
+    if (!d || check_conv(*d)) return 0;
+    return d->ks * d->ks * d->ks * ((d->ci + 31) / 32) * ((d->co + 31) / 32);
+}
+
+int tfdtd_conv_weights(const tfdtd_conv* d, const float* weight, void* w16, void* weight_t, int32_t* nonfinite, void* stream) {
+    if (!d || !weight || !w16 || !nonfinite) return tfdtd_fail(TFDTD_EINVAL, "conv weights: null pointer");
+    const int status = check_conv(*d);
+    if (status) return status;
+    const int taps = d->ks * d->ks * d->ks;
+    hipLaunchKernelGGL(weights_kernel, dim3(taps, (d->ci + 31) / 32, (d->co + 31) / 32), dim3(256), 0, static_cast<hipStream_t>(stream), weight, d->co,
+                       d->ci, taps, d->kp, static_cast<bf16_bits*>(w16), static_cast<bf16_bits*>(weight_t), nonfinite);
+    return tfdtd_check_launch("conv weights");
+}
+
+int tfdtd_conv_forward_rows(const tfdtd_conv* d, const void* x, const void* weight, const int32_t* nonfinite, const float* bias,
+                            int32_t activation, float* pre, float* y, void* act, void* stream) {
+    if (!d || !x || !weight || (!pre && !y && !act)) return tfdtd_fail(TFDTD_EINVAL, "conv forward: null pointer");
+    int status = check_conv(*d);
+    if (status) return status;
+    GatherGemm g{};
+    g.c = make_conv(*d);
+    if ((long long)d->n * g.c.dout * g.c.hout * g.c.wout > 0x7fffffffLL) return tfdtd_fail(TFDTD_EINVAL, "conv: too many positions");
+    g.N = d->co; g.channels = d->ci; g.ldw = d->kp;
+    g.source = static_cast<const bf16_bits*>(x);
+    g.weight = static_cast<const bf16_bits*>(weight);
+    g.nonfinite = nonfinite;
+    g.parts = tfdtd_conv_weight_parts(d);
+    g.bias = bias;
+    g.activation = activation;
+    g.pre = pre; g.y = y; g.act = static_cast<bf16_bits*>(act);
+    if (!gather_gemm(g, static_cast<hipStream_t>(stream)))
+        return tfdtd_fail(TFDTD_EUNSUPPORTED, "conv forward: channels or alignment are left to tfdtd_conv_forward");
+    return tfdtd_check_launch("conv forward");
+}
+
+int tfdtd_conv_dgrad_rows(const tfdtd_conv* d, const void* dy, const void* weight_t, const int32_t* nonfinite, float* dx,
+                          void* stream) {
+    if (!d || !dy || !weight_t || !dx) return tfdtd_fail(TFDTD_EINVAL, "conv dgrad: null pointer");
+    int status = check_conv(*d);
+    if (status) return status;
+    GatherGemm g{};
+    g.c = make_conv(*d);
+    g.dgrad = 1;
+    g.N = d->ci; g.channels = d->co; g.ldw = d->ks * d->ks * d->ks * d->co;
+    g.source = static_cast<const bf16_bits*>(dy);
+    g.weight = static_cast<const bf16_bits*>(weight_t);
+    g.nonfinite = nonfinite;
+    g.parts = tfdtd_conv_weight_parts(d);
+    g.pre = dx;
+    if (!gather_gemm(g, static_cast<hipStream_t>(stream)))
+        return tfdtd_fail(TFDTD_EUNSUPPORTED, "conv dgrad: channels or alignment are left to tfdtd_conv_dgrad");
+    return tfdtd_check_launch("conv dgrad");
+}
+
+int tfdtd_conv_wgrad_splits(const tfdtd_conv* d) {
+    if (!d || check_conv(*d)) return 0;
+    return weight_grad_shape(*d, make_conv(*d)).splits;
+}
+
+int tfdtd_conv_wgrad_rows(const tfdtd_conv* d, const void* dy, const void* x, float* partial, float* dw, void* stream) {
+    if (!d || !dy || !x || !partial || !dw) return tfdtd_fail(TFDTD_EINVAL, "conv wgrad: bad arguments");
+    int status = check_conv(*d);
+    if (status) return status;
+    WeightGrad g{};
+    g.c = make_conv(*d);
+    const WeightGradShape shape = weight_grad_shape(*d, g.c);
+    if (shape.splits == 0) return tfdtd_fail(TFDTD_EINVAL, "conv wgrad: channels must be multiples of 8, or at most 32 kernel values");
+    if (d->kp != 32 && (!aligned16(dy) || !aligned16(x) || !aligned16(partial)))
+        return tfdtd_fail(TFDTD_EINVAL, "conv wgrad: operands must be 16-byte aligned");
+    g.dy = static_cast<const bf16_bits*>(dy);
+    g.x = static_cast<const bf16_bits*>(x);
+    g.partial = partial;
+    g.m_total = d->n * g.c.dout * g.c.hout * g.c.wout;
+    g.per_split = (int)(((long long)g.m_total + 64LL * shape.splits - 1) / (64LL * shape.splits) * 64);
+    g.by_w = make_divider((unsigned)g.c.wout);
+    g.by_h = make_divider((unsigned)g.c.hout);
+    g.by_d = make_divider((unsigned)g.c.dout);
+    const int used = (g.m_total + g.per_split - 1) / g.per_split;
+    const dim3 grid((d->co + shape.bc - 1) / shape.bc, (d->kp + shape.bk - 1) / shape.bk, used), block(256);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (d->kp == 32) hipLaunchKernelGGL(weight_grad_narrow_kernel, grid, block, 0, s, g);
+    else if (shape.bc == 32) hipLaunchKernelGGL((weight_grad_kernel<32, 128>), grid, block, 0, s, g);
+    else if (shape.bc == 64) hipLaunchKernelGGL((weight_grad_kernel<64, 128>), grid, block, 0, s, g);
+    else hipLaunchKernelGGL((weight_grad_kernel<128, 128>), grid, block, 0, s, g);
+    status = tfdtd_check_launch("conv wgrad");
+    if (status) return status;
+    const long long count = (long long)d->co * d->kp;
+    hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((count + 63) / 64)), dim3(256), 0, s, partial, used, count, dw);
+    return tfdtd_check_launch("conv wgrad sum");
+}
+
+int tfdtd_gelu_backward_rows(const float* dy, const float* pre, int64_t rows, int32_t channels, int32_t activation, void* dpre16,
+                             double* partial, float* bias_grad, void* stream) {
+    if (!dy || (activation && !pre) || !dpre16 || !partial || !bias_grad || rows < 1 || channels < 4 || channels > 1024 || channels % 4)
+        return tfdtd_fail(TFDTD_EINVAL, "gelu backward rows: bad arguments (channels: a multiple of 4, at most 1024)");
+    if (!aligned16(dy) || !aligned16(pre) || !aligned16(partial) || (reinterpret_cast<uintptr_t>(dpre16) & 7u))
+        return tfdtd_fail(TFDTD_EINVAL, "gelu backward rows: operands must be 16-byte aligned");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int per = 256 / (channels / 4);
+    const int blocks = (int)std::min<int64_t>(kBiasBlocks, (rows + 4LL * per - 1) / (4 * per));
+    hipLaunchKernelGGL(gelu_backward_rows_kernel, dim3(blocks), dim3(256), 0, s, dy, pre, (long long)rows, channels, activation,
+                       static_cast<bf16_bits*>(dpre16), partial);
+    int status = tfdtd_check_launch("gelu backward rows");
+    if (status) return status;
+    hipLaunchKernelGGL(bias_sum_kernel, dim3((channels + 31) / 32), dim3(1024), 0, s, partial, blocks, channels, bias_grad);
+    return tfdtd_check_launch("bias gradient");
 }
 
 int tfdtd_gelu_backward(const float* dy, const float* pre, int64_t count, int32_t activation, float* dpre, void* dpre16,

@@ -218,10 +218,6 @@ struct PlaneAxis {          // CPML rows of one axis, shared by its two terms: l
     unsigned coef, coef_high;   // byte offset of b | c | inv_k of the low side, and what to add for the high side
 };
 
-struct Divider {            // q = (mulhi(m, n) + n) >> s for n < 2^31
-    unsigned m, s;
-};
-
 template <typename real>
 struct PlaneStep {
     int nx, ny, nz, nyz;
@@ -243,8 +239,6 @@ struct PlaneStep {
     long long source_samples;
     const long long* counter;
 };
-
-__device__ __forceinline__ unsigned divide(unsigned n, Divider d) { return (__umulhi(n, d.m) + n) >> d.s; }
 
 // A value at a uniform base plus a 32-bit byte offset of the lane.
 template <typename real>
@@ -446,14 +440,6 @@ __device__ __forceinline__ unsigned wave_item(unsigned block) {
 }
 
 constexpr unsigned kXcdRun = 128;
-
-// Workgroup b runs on XCD b % 8.  Within each run of 8 * xcd workgroups every XCD takes `xcd` consecutive ones.
-__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned blocks, unsigned run) {
-    const unsigned first = b / (8u * run) * (8u * run);
-    if (first + 8u * run > blocks) return b;
-    const unsigned k = b - first;
-    return first + (k & 7u) * run + (k >> 3);
-}
 
 template <typename real, bool forward, int INV, bool FLAT>
 __global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void plane_half_step_kernel(const PlaneStep<real> a) {
@@ -754,12 +740,6 @@ int make_half_step(const tfdtd_half_step* d, HalfStep<real>* a) {
     a->source_samples = d->source_samples;
     a->counter = reinterpret_cast<const long long*>(d->counter);
     return TFDTD_OK;
-}
-
-Divider make_divider(unsigned d) {
-    unsigned s = 0;
-    while ((1ull << s) < d) ++s;
-    return Divider{(unsigned)(((1ull << 32) * ((1ull << s) - d)) / d + 1), s};
 }
 
 // Planes per march: two share the lane's set-up and the plane between them (18.9 against 20.7 us a step on

@@ -50,55 +50,108 @@ def forward_weight(weight):
     return w16
 
 
+def _operands(shape, weight, transposed):
+    """The bf16 operands of a layer: (forward weights, input-gradient weights or None, non-finite parts or None)."""
+    co, ks, ci = weight.shape[0], weight.shape[1], weight.shape[-1]
+    if weight.dtype != torch.float32:
+        return forward_weight(weight), None, None
+    lib = N.library()
+    weight = weight.contiguous()
+    w16 = torch.empty((co, shape.kp), device=weight.device, dtype=torch.bfloat16)
+    wt = torch.empty((ci, ks**3*co), device=weight.device, dtype=torch.bfloat16) if transposed else None
+    parts = torch.empty(lib.tfdtd_conv_weight_parts(ctypes.byref(shape)), device=weight.device, dtype=torch.int32)
+    N.check(lib.tfdtd_conv_weights(ctypes.byref(shape), weight.data_ptr(), w16.data_ptr(), N.address(wt), parts.data_ptr(),
+                                   N.stream_handle()), 'tfdtd_conv_weights')
+    return w16, wt, parts
+
+
+def _forward(shape, x16, w16, parts, bias, activation, pre=None, y=None, act=None):
+    """One layer: x16 -> any of pre (FP32), y (FP32 of the bf16 activation) and act (bf16), each [m, co] or None."""
+    lib, stream = N.library(), N.stream_handle()
+    status = lib.tfdtd_conv_forward_rows(ctypes.byref(shape), x16.data_ptr(), w16.data_ptr(), N.address(parts), bias.data_ptr(),
+                                         int(activation), N.address(pre), N.address(y), N.address(act), stream)
+    if status != N.EUNSUPPORTED:
+        return N.check(status, 'tfdtd_conv_forward_rows')
+    out = next(t for t in (pre, y, act) if t is not None)
+    pre = torch.empty(out.shape, device=out.device, dtype=torch.float32) if pre is None else pre
+    act16 = torch.empty(out.shape, device=out.device, dtype=torch.bfloat16) if act is None else act
+    N.check(lib.tfdtd_conv_forward(ctypes.byref(shape), x16.data_ptr(), w16.data_ptr(), ctypes.c_void_p(bias.data_ptr()),
+                                   int(activation), ctypes.c_void_p(pre.data_ptr()), act16.data_ptr(), stream), 'tfdtd_conv_forward')
+    if y is not None:
+        y.copy_(act16)
+
+
+def _layer_gradients(shape, dy, pre, activation, x16):
+    """(bf16 gradient of the pre-activation, FP32 weight gradient [co][kp], bias gradient) of one layer."""
+    lib, stream = N.library(), N.stream_handle()
+    m, co = pre.shape
+    device = pre.device
+    dpre16 = torch.empty(pre.shape, device=device, dtype=torch.bfloat16)
+    grad_bias = torch.empty(co, device=device, dtype=torch.float32)
+    if co % 4 == 0 and co <= 1024 and dy.data_ptr() % 16 == 0:
+        partial = torch.empty((N.BIAS_BLOCKS, co), device=device, dtype=torch.float64)
+        N.check(lib.tfdtd_gelu_backward_rows(dy.data_ptr(), pre.data_ptr(), m, co, activation, dpre16.data_ptr(),
+                                             partial.data_ptr(), grad_bias.data_ptr(), stream), 'tfdtd_gelu_backward_rows')
+    else:
+        dpre = torch.empty_like(pre)
+        N.check(lib.tfdtd_gelu_backward(ctypes.c_void_p(dy.data_ptr()), ctypes.c_void_p(pre.data_ptr()), m*co, activation,
+                                        ctypes.c_void_p(dpre.data_ptr()), dpre16.data_ptr(), stream), 'tfdtd_gelu_backward')
+        torch.sum(dpre, 0, out=grad_bias)
+    dw = torch.empty((co, shape.kp), device=device, dtype=torch.float32)
+    splits = lib.tfdtd_conv_wgrad_splits(ctypes.byref(shape)) if x16.data_ptr() % 16 == 0 else 0
+    if splits:
+        partial = torch.empty((splits, co, shape.kp), device=device, dtype=torch.float32)
+        N.check(lib.tfdtd_conv_wgrad_rows(ctypes.byref(shape), dpre16.data_ptr(), x16.data_ptr(), partial.data_ptr(),
+                                          dw.data_ptr(), stream), 'tfdtd_conv_wgrad_rows')
+    else:
+        dy_t = dpre16.t().contiguous()
+        splits = max(1, min(64, m//4096))
+        partial = torch.empty((splits, co, shape.kp), device=device, dtype=torch.float32)
+        N.check(lib.tfdtd_conv_wgrad(ctypes.byref(shape), dy_t.data_ptr(), x16.data_ptr(), splits,
+                                     ctypes.c_void_p(partial.data_ptr()), ctypes.c_void_p(dw.data_ptr()), stream), 'tfdtd_conv_wgrad')
+    return dpre16, dw, grad_bias
+
+
+def _input_gradient(shape, dpre16, w16, wt, parts):
+    """FP32 input gradient [m_in, ci] of one layer."""
+    lib, stream = N.library(), N.stream_handle()
+    taps, ci, co = shape.ks**3, shape.ci, shape.co
+    if wt is None:
+        wt = w16[:, :taps*ci].reshape(co, taps, ci).permute(2, 1, 0).contiguous()
+    dx = torch.empty((shape.n*shape.di*shape.hi*shape.wi, ci), device=dpre16.device, dtype=torch.float32)
+    status = lib.tfdtd_conv_dgrad_rows(ctypes.byref(shape), dpre16.data_ptr(), wt.data_ptr(), N.address(parts), dx.data_ptr(), stream)
+    if status == N.EUNSUPPORTED:
+        status = lib.tfdtd_conv_dgrad(ctypes.byref(shape), dpre16.data_ptr(), wt.data_ptr(), ctypes.c_void_p(dx.data_ptr()), stream)
+    N.check(status, 'tfdtd_conv_dgrad')
+    return dx
+
+
 class _Conv(torch.autograd.Function):
     """y = act(conv(x) + b), x and y FP32 channels-last; bf16 operands on MFMA inside."""
 
     @staticmethod
     def forward(ctx, x, weight, bias, stride, pad, activation):
-        lib = N.library()
         co, ks, ci = weight.shape[0], weight.shape[1], weight.shape[-1]
         shape, (do, ho, wo) = conv_shape(tuple(x.shape), ci, co, ks, stride, pad)
         x16 = x.detach().to(torch.bfloat16).contiguous()
-        w16 = forward_weight(weight.detach())
+        w16, wt, parts = _operands(shape, weight.detach(), ctx.needs_input_grad[0])
         m = x.shape[0]*do*ho*wo
         pre = torch.empty((m, co), device=x.device, dtype=torch.float32)
-        act = torch.empty((m, co), device=x.device, dtype=torch.bfloat16)
-        b = bias.detach().float().contiguous()
-        N.check(lib.tfdtd_conv_forward(ctypes.byref(shape), x16.data_ptr(), w16.data_ptr(), ctypes.c_void_p(b.data_ptr()),
-                                       int(activation), ctypes.c_void_p(pre.data_ptr()), act.data_ptr(), N.stream_handle()),
-                'tfdtd_conv_forward')
-        ctx.save_for_backward(x16, w16, pre)
-        ctx.config = (shape, ks, ci, co, int(activation), tuple(x.shape))
-        return act.float().view(x.shape[0], do, ho, wo, co)
+        y = torch.empty((m, co), device=x.device, dtype=torch.float32)
+        _forward(shape, x16, w16, parts, bias.detach().float().contiguous(), activation, pre=pre, y=y)
+        ctx.save_for_backward(x16, w16, wt, parts, pre)
+        ctx.config = (shape, int(activation), tuple(x.shape))
+        return y.view(x.shape[0], do, ho, wo, co)
 
     @staticmethod
     def backward(ctx, grad):
-        lib = N.library()
-        x16, w16, pre = ctx.saved_tensors
-        shape, ks, ci, co, activation, x_shape = ctx.config
-        stream = N.stream_handle()
-        m = pre.shape[0]
-        dpre = torch.empty_like(pre)
-        dpre16 = torch.empty(pre.shape, device=pre.device, dtype=torch.bfloat16)
-        dy = grad.contiguous().view(m, co).float()
-        N.check(lib.tfdtd_gelu_backward(ctypes.c_void_p(dy.data_ptr()), ctypes.c_void_p(pre.data_ptr()), m*co, activation,
-                                        ctypes.c_void_p(dpre.data_ptr()), dpre16.data_ptr(), stream), 'tfdtd_gelu_backward')
-        grad_bias = dpre.sum(0)
-        dy_t = dpre16.t().contiguous()
-        splits = max(1, min(64, m//4096))
-        partial = torch.empty((splits, co, shape.kp), device=pre.device, dtype=torch.float32)
-        dw = torch.empty((co, shape.kp), device=pre.device, dtype=torch.float32)
-        N.check(lib.tfdtd_conv_wgrad(ctypes.byref(shape), dy_t.data_ptr(), x16.data_ptr(), splits,
-                                     ctypes.c_void_p(partial.data_ptr()), ctypes.c_void_p(dw.data_ptr()), stream), 'tfdtd_conv_wgrad')
-        taps = ks**3
-        grad_weight = dw[:, :taps*ci].reshape(co, ks, ks, ks, ci)
-        grad_x = None
-        if ctx.needs_input_grad[0]:
-            wt = w16[:, :taps*ci].reshape(co, taps, ci).permute(2, 1, 0).contiguous()
-            dx = torch.empty((x_shape[0]*x_shape[1]*x_shape[2]*x_shape[3], ci), device=pre.device, dtype=torch.float32)
-            N.check(lib.tfdtd_conv_dgrad(ctypes.byref(shape), dpre16.data_ptr(), wt.data_ptr(), ctypes.c_void_p(dx.data_ptr()),
-                                         stream), 'tfdtd_conv_dgrad')
-            grad_x = dx.view(x_shape)
+        x16, w16, wt, parts, pre = ctx.saved_tensors
+        shape, activation, x_shape = ctx.config
+        dy = grad.contiguous().view(pre.shape).float()
+        dpre16, dw, grad_bias = _layer_gradients(shape, dy, pre, activation, x16)
+        ks, ci = shape.ks, shape.ci
+        grad_weight = dw[:, :ks**3*ci].reshape(shape.co, ks, ks, ks, ci)
+        grad_x = _input_gradient(shape, dpre16, w16, wt, parts).view(x_shape) if ctx.needs_input_grad[0] else None
         return grad_x, grad_weight, grad_bias, None, None, None
 
 
