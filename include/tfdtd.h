@@ -486,11 +486,13 @@ int tfdtd_conv_wgrad(const tfdtd_conv* conv, const void* dy_t, const void* x, in
 int tfdtd_gelu_backward(const float* dy, const float* pre, int64_t count, int32_t activation, float* dpre, void* dpre16,
                         void* stream);
 
-/* The bf16 operands of a layer from its FP32 weights [co][ks^3][ci], in one launch: w16 [co][kp] for the
- * forward, weight_t [ci][ks^3*co] for the input gradient (null: not wanted), and nonfinite
- * int32[tfdtd_conv_weight_parts(conv)], 1 where a part of the weights holds an infinity or NaN. */
+/* The bf16 operands of up to TFDTD_CONV_WEIGHT_JOBS layers from their FP32 weights [co][ks^3][ci], in one launch;
+ * per layer w16 [co][kp] for the forward, weights_t [ci][ks^3*co] for the input gradient (null: not wanted),
+ * and nonfinite int32[tfdtd_conv_weight_parts(conv)], 1 where a part of the weights holds an infinity or NaN. */
+#define TFDTD_CONV_WEIGHT_JOBS 8
 int tfdtd_conv_weight_parts(const tfdtd_conv* conv);
-int tfdtd_conv_weights(const tfdtd_conv* conv, const float* weight, void* w16, void* weight_t, int32_t* nonfinite, void* stream);
+int tfdtd_conv_weights(const tfdtd_conv* convs, int32_t count, const float* const* weights, void* const* w16,
+                       void* const* weights_t, int32_t* const* nonfinite, void* stream);
 /* tfdtd_conv_forward with any of its outputs: pre FP32, y FP32 (the value of the bf16 activation), act bf16.
  * With `nonfinite` (of tfdtd_conv_weights) a tap that is padding for all rows of a workgroup is skipped when every
  * weight is finite.  TFDTD_EUNSUPPORTED where channels (multiples of 8, or kp 32) or the 16-byte alignment

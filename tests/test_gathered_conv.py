@@ -31,7 +31,7 @@ def test_pre_activation_and_gradients_within_the_fp32_bound(gpu, shape, ci, co, 
     b = torch.randn(co, generator=gen)
     s, out = conv_shape((*shape, ci), ci, co, ks, stride, pad)
     m, k = shape[0]*math.prod(out), ks**3*ci
-    w16, wt, parts = _operands(s, w.float().cuda(), True)
+    (w16, wt, parts), = _operands([s], [w.float().cuda()], [True])
     pre = torch.full((m, co), float('nan'), device=gpu)
     act = torch.empty((m, co), device=gpu, dtype=torch.bfloat16)
     _forward(s, x.cuda(), w16, parts, b.cuda(), False, pre=pre, act=act)
@@ -66,3 +66,24 @@ def test_taps_in_the_padding_keep_what_infinite_weights_give(gpu):
     y = conv3d(x, w, b, 1, 1, False)
     assert torch.isnan(y[..., 5]).all()
     assert torch.isfinite(y[..., :5]).all() and torch.isfinite(y[..., 6:]).all()
+
+
+def test_network_equals_its_layers_one_by_one(gpu):
+    """The network's trunk against conv3d after conv3d: the same operations, so equal outputs and gradients."""
+    from torchfdtd_amd.surrogate import SurrogateNet, conv3d, linear
+    net = SurrogateNet(channels=(32, 40, 64), hidden=24, outputs=8, seed=4).to(gpu)
+    gen = torch.Generator().manual_seed(9)
+    rho = torch.rand((3, 18, 13, 9), generator=gen).to(gpu).requires_grad_(True)
+    x = rho.unsqueeze(-1)
+    for w, b in zip(net.weights, net.biases):
+        x = conv3d(x, w, b, stride=2, pad=1, activation=True)
+    x = linear(x.mean(dim=(1, 2, 3)), net.head[0], net.head[1])
+    expected = linear(x, net.head[2], net.head[3], activation=False)
+    parameters = [rho, *net.parameters()]
+    want = torch.autograd.grad(expected.square().sum(), parameters)
+    got = net(rho)
+    assert torch.equal(got, expected)
+    for a, b in zip(torch.autograd.grad(got.square().sum(), parameters), want):
+        assert torch.equal(a, b)
+    with torch.no_grad():
+        assert torch.equal(net(rho), expected)

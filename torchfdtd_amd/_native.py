@@ -121,6 +121,7 @@ class NormGrid(ctypes.Structure):
 
 ADE_MAX_POLES = 16
 BIAS_BLOCKS = 2048
+CONV_WEIGHT_JOBS = 8
 EUNSUPPORTED = 3
 
 
@@ -192,7 +193,7 @@ PROTOTYPES = {
     'tfdtd_conv_dgrad': (i32, [vp, vp, vp, vp, vp]),
     'tfdtd_conv_wgrad': (i32, [vp, vp, vp, i32, vp, vp, vp]),
     'tfdtd_conv_weight_parts': (i32, [vp]),
-    'tfdtd_conv_weights': (i32, [vp, vp, vp, vp, vp, vp]),
+    'tfdtd_conv_weights': (i32, [vp, i32, vp, vp, vp, vp, vp]),
     'tfdtd_conv_forward_rows': (i32, [vp, vp, vp, vp, vp, i32, vp, vp, vp, vp]),
     'tfdtd_conv_dgrad_rows': (i32, [vp, vp, vp, vp, vp, vp]),
     'tfdtd_conv_wgrad_splits': (i32, [vp]),

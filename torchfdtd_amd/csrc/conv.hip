@@ -583,36 +583,55 @@ void launch_gather(GatherGemm g, int classes, hipStream_t stream) {
     else hipLaunchKernelGGL((gather_gemm_kernel<BM, BN, WM, WN, Depth, false>), grid, block, 0, stream, g);
 }
 
-// FP32 weights [co][taps][ci] to the bf16 operands of the forward convolution, [co][kp], and of the input
-// gradient, [ci][taps * co] (transposed through LDS), and per tap and 32 x 32 channels whether a value is not finite.
-__global__ __launch_bounds__(256) void weights_kernel(const float* weight, int co, int ci, int taps, int kp, bf16_bits* w16,
-                                                      bf16_bits* transposed, int* nonfinite) {
+// FP32 weights [co][taps][ci] of several layers to the bf16 operands of the forward convolution, [co][kp],
+// and of the input gradient, [ci][taps * co] (transposed through LDS), and per tap and 32 x 32 channels
+// whether a value is not finite.  One launch for a network's layers: each alone takes the time of a launch.
+struct WeightsJob {
+    const float* weight;
+    bf16_bits* w16;
+    bf16_bits* transposed;      // null: not wanted
+    int* nonfinite;
+    int co, ci, taps, kp, first;    // first: the job's first workgroup
+};
+
+struct WeightsJobs {
+    int count;
+    WeightsJob job[TFDTD_CONV_WEIGHT_JOBS];
+};
+
+__global__ __launch_bounds__(256) void weights_kernel(const WeightsJobs jobs) {
     __shared__ bf16_bits tile[32][33];
     __shared__ int bad;
-    const int tap = blockIdx.x, c0 = blockIdx.y * 32, o0 = blockIdx.z * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    int which = 0;
+    for (int k = 1; k < jobs.count; ++k)
+        if ((int)blockIdx.x >= jobs.job[k].first) which = k;
+    const WeightsJob& j = jobs.job[which];
+    const int co = j.co, ci = j.ci, taps = j.taps, kp = j.kp, part = (int)blockIdx.x - j.first, across = (ci + 31) / 32;
+    const int tap = part % taps, c0 = part / taps % across * 32, o0 = part / (taps * across) * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     if (threadIdx.x == 0) bad = 0;
     __syncthreads();
     bool mine = false;
     for (int r = ty; r < 32; r += 8) {
         const int o = o0 + r, c = c0 + tx;
         if (o < co && c < ci) {
-            const bf16_bits b = float_to_bf16(weight[((long long)o * taps + tap) * ci + c]);
+            const bf16_bits b = float_to_bf16(j.weight[((long long)o * taps + tap) * ci + c]);
             mine |= (b & 0x7f80u) == 0x7f80u;      // infinite or NaN, also a finite value that rounds to infinity
-            w16[(long long)o * kp + tap * ci + c] = b;
+            j.w16[(long long)o * kp + tap * ci + c] = b;
             tile[r][tx] = b;
         }
         if (tap == taps - 1 && o < co && c0 + 32 >= ci)
-            for (int k = taps * ci + tx; k < kp; k += 32) w16[(long long)o * kp + k] = 0;
+            for (int k = taps * ci + tx; k < kp; k += 32) j.w16[(long long)o * kp + k] = 0;
     }
     __syncthreads();
-    if (transposed)
+    if (j.transposed)
         for (int r = ty; r < 32; r += 8) {
             const int c = c0 + r, o = o0 + tx;
-            if (c < ci && o < co) transposed[((long long)c * taps + tap) * co + o] = tile[tx][r];
+            if (c < ci && o < co) j.transposed[((long long)c * taps + tap) * co + o] = tile[tx][r];
         }
     if (mine) bad = 1;
     __syncthreads();
-    if (threadIdx.x == 0) nonfinite[(blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = bad;
+    if (threadIdx.x == 0) j.nonfinite[part] = bad;
 }
 
 // Forward convolution with at most 32 values of K (a one-channel input): no staging pays, a wavefront takes
@@ -1102,13 +1121,24 @@ int tfdtd_conv_weight_parts(const tfdtd_conv* d) {
     return d->ks * d->ks * d->ks * ((d->ci + 31) / 32) * ((d->co + 31) / 32);
 }
 
-int tfdtd_conv_weights(const tfdtd_conv* d, const float* weight, void* w16, void* weight_t, int32_t* nonfinite, void* stream) {
-    if (!d || !weight || !w16 || !nonfinite) return tfdtd_fail(TFDTD_EINVAL, "conv weights: null pointer");
-    const int status = check_conv(*d);
-    if (status) return status;
-    const int taps = d->ks * d->ks * d->ks;
-    hipLaunchKernelGGL(weights_kernel, dim3(taps, (d->ci + 31) / 32, (d->co + 31) / 32), dim3(256), 0, static_cast<hipStream_t>(stream), weight, d->co,
-                       d->ci, taps, d->kp, static_cast<bf16_bits*>(w16), static_cast<bf16_bits*>(weight_t), nonfinite);
+int tfdtd_conv_weights(const tfdtd_conv* convs, int32_t count, const float* const* weights, void* const* w16,
+                       void* const* weights_t, int32_t* const* nonfinite, void* stream) {
+    if (!convs || !weights || !w16 || !nonfinite || count < 1 || count > TFDTD_CONV_WEIGHT_JOBS)
+        return tfdtd_fail(TFDTD_EINVAL, "conv weights: null pointer, or not 1 to %d layers", TFDTD_CONV_WEIGHT_JOBS);
+    WeightsJobs jobs{};
+    jobs.count = count;
+    long long blocks = 0;
+    for (int k = 0; k < count; ++k) {
+        const tfdtd_conv& d = convs[k];
+        const int status = check_conv(d);
+        if (status) return status;
+        if (!weights[k] || !w16[k] || !nonfinite[k]) return tfdtd_fail(TFDTD_EINVAL, "conv weights: layer %d: null pointer", k);
+        jobs.job[k] = WeightsJob{weights[k], static_cast<bf16_bits*>(w16[k]), weights_t ? static_cast<bf16_bits*>(weights_t[k]) : nullptr,
+                                 nonfinite[k], d.co, d.ci, d.ks * d.ks * d.ks, d.kp, (int)blocks};
+        blocks += tfdtd_conv_weight_parts(&d);
+        if (blocks > 0x7fffffffLL) return tfdtd_fail(TFDTD_EINVAL, "conv weights: too many weights for one launch");
+    }
+    hipLaunchKernelGGL(weights_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), jobs);
     return tfdtd_check_launch("conv weights");
 }
 

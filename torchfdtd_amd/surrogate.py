@@ -41,6 +41,11 @@ def conv_shape(x_shape, ci, co, ks, stride, pad):
     return s, tuple(v.value for v in out)
 
 
+def conv_rows(shape):
+    """Output positions of a layer."""
+    return shape.n*math.prod((k+2*shape.pad-shape.ks)//shape.stride+1 for k in (shape.di, shape.hi, shape.wi))
+
+
 def forward_weight(weight):
     """FP32 [co][ks][ks][ks][ci] -> bf16 [co][kp] with zero padding."""
     co = weight.shape[0]
@@ -50,19 +55,21 @@ def forward_weight(weight):
     return w16
 
 
-def _operands(shape, weight, transposed):
-    """The bf16 operands of a layer: (forward weights, input-gradient weights or None, non-finite parts or None)."""
-    co, ks, ci = weight.shape[0], weight.shape[1], weight.shape[-1]
-    if weight.dtype != torch.float32:
-        return forward_weight(weight), None, None
-    lib = N.library()
-    weight = weight.contiguous()
-    w16 = torch.empty((co, shape.kp), device=weight.device, dtype=torch.bfloat16)
-    wt = torch.empty((ci, ks**3*co), device=weight.device, dtype=torch.bfloat16) if transposed else None
-    parts = torch.empty(lib.tfdtd_conv_weight_parts(ctypes.byref(shape)), device=weight.device, dtype=torch.int32)
-    N.check(lib.tfdtd_conv_weights(ctypes.byref(shape), weight.data_ptr(), w16.data_ptr(), N.address(wt), parts.data_ptr(),
-                                   N.stream_handle()), 'tfdtd_conv_weights')
-    return w16, wt, parts
+def _operands(shapes, weights, transposed):
+    """Per layer the bf16 operands (forward weights, input-gradient weights or None, non-finite parts or None);
+    `transposed`: per layer whether the input-gradient weights are wanted."""
+    if len(shapes) > N.CONV_WEIGHT_JOBS or any(w.dtype != torch.float32 for w in weights):
+        return [(forward_weight(w), None, None) for w in weights]
+    lib, count = N.library(), len(shapes)
+    weights = [w.contiguous() for w in weights]
+    out = []
+    for shape, w, want in zip(shapes, weights, transposed):
+        out.append((torch.empty((shape.co, shape.kp), device=w.device, dtype=torch.bfloat16),
+                    torch.empty((shape.ci, shape.ks**3*shape.co), device=w.device, dtype=torch.bfloat16) if want else None,
+                    torch.empty(lib.tfdtd_conv_weight_parts(ctypes.byref(shape)), device=w.device, dtype=torch.int32)))
+    pointers = [(ctypes.c_void_p*count)(*(N.address(t) for t in column)) for column in (weights, *zip(*out))]
+    N.check(lib.tfdtd_conv_weights((ConvShape*count)(*shapes), count, *pointers, N.stream_handle()), 'tfdtd_conv_weights')
+    return out
 
 
 def _forward(shape, x16, w16, parts, bias, activation, pre=None, y=None, act=None):
@@ -134,7 +141,7 @@ class _Conv(torch.autograd.Function):
         co, ks, ci = weight.shape[0], weight.shape[1], weight.shape[-1]
         shape, (do, ho, wo) = conv_shape(tuple(x.shape), ci, co, ks, stride, pad)
         x16 = x.detach().to(torch.bfloat16).contiguous()
-        w16, wt, parts = _operands(shape, weight.detach(), ctx.needs_input_grad[0])
+        (w16, wt, parts), = _operands([shape], [weight.detach()], [ctx.needs_input_grad[0]])
         m = x.shape[0]*do*ho*wo
         pre = torch.empty((m, co), device=x.device, dtype=torch.float32)
         y = torch.empty((m, co), device=x.device, dtype=torch.float32)
@@ -167,6 +174,52 @@ def linear(x, weight, bias, activation=True):
     return y.reshape(x.shape[0], weight.shape[0])
 
 
+class _Trunk(torch.autograd.Function):
+    """A chain of convolutions with GELU, x FP32 channels-last -> FP32 output of the last: what conv3d after conv3d
+    computes, with the activations between the layers kept in the bf16 that the next layer reads.  Without
+    `keep` (no backward will follow) the pre-activations are not stored."""
+
+    @staticmethod
+    def forward(ctx, keep, stride, pad, x, *parameters):
+        weights, biases = [w.detach() for w in parameters[::2]], parameters[1::2]
+        shapes, dims = [], tuple(x.shape)
+        for w in weights:
+            shape, out = conv_shape(dims, w.shape[-1], w.shape[0], w.shape[1], stride, pad)
+            shapes.append(shape)
+            dims = (dims[0], *out, w.shape[0])
+        operands = _operands(shapes, weights, [keep and (k > 0 or ctx.needs_input_grad[3]) for k in range(len(shapes))])
+        inputs, pres = [x.detach().to(torch.bfloat16).contiguous()], []
+        for k, (shape, (w16, _, parts), bias) in enumerate(zip(shapes, operands, biases)):
+            last = k+1 == len(shapes)
+            m = conv_rows(shape)
+            pre = torch.empty((m, shape.co), device=x.device, dtype=torch.float32) if keep else None
+            out = torch.empty((m, shape.co), device=x.device, dtype=torch.float32 if last else torch.bfloat16)
+            _forward(shape, inputs[k], w16, parts, bias.detach().float().contiguous(), True, pre=pre,
+                     **{'y' if last else 'act': out})
+            pres.append(pre)
+            inputs.append(out)
+        if keep:
+            ctx.save_for_backward(*inputs[:-1], *pres, *(t for group in operands for t in group))
+        ctx.config = (shapes, tuple(x.shape))
+        return inputs[-1].view(dims)
+
+    @staticmethod
+    def backward(ctx, grad):
+        shapes, x_shape = ctx.config
+        count = len(shapes)
+        saved = ctx.saved_tensors
+        inputs, pres, operands = saved[:count], saved[count:2*count], saved[2*count:]
+        grads = [None]*(2*count)
+        dy = grad.contiguous().view(pres[-1].shape).float()
+        for k in reversed(range(count)):
+            shape, (w16, wt, parts) = shapes[k], operands[3*k:3*k+3]
+            dpre16, dw, grads[2*k+1] = _layer_gradients(shape, dy, pres[k], 1, inputs[k])
+            grads[2*k] = dw[:, :shape.ks**3*shape.ci].reshape(shape.co, *(shape.ks,)*3, shape.ci)
+            if k > 0 or ctx.needs_input_grad[3]:
+                dy = _input_gradient(shape, dpre16, w16, wt, parts)
+        return (None, None, None, dy.view(x_shape) if ctx.needs_input_grad[3] else None, *grads)
+
+
 class SurrogateNet(nn.Module):
     """rho [n, 64, 64, 8] -> transmission [n, 32]."""
 
@@ -188,8 +241,10 @@ class SurrogateNet(nn.Module):
 
     def forward(self, rho):
         x = rho.unsqueeze(-1).float()
-        for w, b in zip(self.weights, self.biases):
-            x = conv3d(x, w, b, stride=2, pad=1, activation=True)
+        parameters = [p for pair in zip(self.weights, self.biases) for p in pair]
+        if parameters:
+            keep = torch.is_grad_enabled() and any(t.requires_grad for t in (x, *parameters))
+            x = _Trunk.apply(keep, 2, 1, x, *parameters)
         x = x.mean(dim=(1, 2, 3))
         x = linear(x, self.head[0], self.head[1], activation=True)
         return linear(x, self.head[2], self.head[3], activation=False)
