@@ -16,6 +16,7 @@
 
 #include "../../include/tfdtd.h"
 #include "common.h"
+#include "plane_march.h"
 
 namespace {
 
@@ -61,18 +62,6 @@ struct HalfStep {
     long long source_samples;
     const long long* counter;
 };
-
-// The three components of one cell, read as one 12-byte (24-byte) access through a global pointer.
-template <typename real>
-struct Cell {
-    real v[3];
-};
-
-template <typename real>
-__device__ __forceinline__ Cell<real> cell_at(const real* base, long long i) {
-    const auto p = global(base + 3 * i);
-    return Cell<real>{{p[0], p[1], p[2]}};
-}
 
 // One cell.  forward=false: E update from backward differences of H;
 // forward=true: H update from forward differences of E.  The cell and its three neighbours
@@ -211,14 +200,6 @@ __global__ __launch_bounds__(256) void yee_half_step_kernel(const HalfStep<real>
 // on 256^3 (FP32), 30.5 us on 97x83x61 (FP64); the march takes 18.1, 35.7, 106, 286 and 20.9 us.  What
 // bounds it now is the traffic: past the 256 MB cache 5 TB/s of a copy's 5.5, inside it about 6 of 8.2.
 template <typename real>
-struct PlaneAxis {          // CPML rows of one axis, shared by its two terms: low side, then high side
-    int lo[2], hi[2];       // empty: lo == hi == 0
-    unsigned psi[2];        // byte offset of each term's low-side memory in the family's buffer
-    unsigned high[2];       // what to add for the high side
-    unsigned coef, coef_high;   // byte offset of b | c | inv_k of the low side, and what to add for the high side
-};
-
-template <typename real>
 struct PlaneStep {
     int nx, ny, nz, nyz;
     int span, columns;      // planes per march, 64-cell columns of a plane
@@ -239,53 +220,6 @@ struct PlaneStep {
     long long source_samples;
     const long long* counter;
 };
-
-// A value at a uniform base plus a 32-bit byte offset of the lane.
-template <typename real>
-__device__ __forceinline__ real at_byte(const real* base, unsigned off) {
-    return *global(reinterpret_cast<const real*>(reinterpret_cast<const char*>(base) + off));
-}
-
-template <typename real>
-__device__ __forceinline__ void put_byte(real* base, unsigned off, real v) {
-    *global(reinterpret_cast<real*>(reinterpret_cast<char*>(base) + off)) = v;
-}
-
-template <typename real>
-__device__ __forceinline__ Cell<real> cell_at_byte(const real* base, unsigned off) {
-    const auto p = global(reinterpret_cast<const real*>(reinterpret_cast<const char*>(base) + off));
-    return Cell<real>{{p[0], p[1], p[2]}};
-}
-
-// The CPML row of the y or z axis a lane lies in: the memory of its two terms and their coefficients.
-template <typename real>
-struct PlaneHit {
-    bool on;
-    unsigned at[2];     // byte offsets of the two terms' memory in the current plane
-    unsigned stride;    // bytes per x plane
-    real b, c, ik;
-};
-
-// The row k of an axis: w is its slab's width; `on` false leaves the rest unused.
-template <typename real>
-struct AxisRow {
-    bool on;
-    int q, w;
-    unsigned psi[2], coef;
-};
-
-template <typename real>
-__device__ __forceinline__ AxisRow<real> axis_row(const PlaneAxis<real>& p, int k, bool inside) {
-    const int k0 = k - p.lo[0], k1 = k - p.lo[1], w0 = p.hi[0] - p.lo[0], w1 = p.hi[1] - p.lo[1];
-    const bool low = (unsigned)k0 < (unsigned)w0, high = (unsigned)k1 < (unsigned)w1;
-    AxisRow<real> r;
-    r.on = inside & (low | high);
-    r.q = low ? k0 : k1;
-    r.w = low ? w0 : w1;
-    for (int t = 0; t < 2; ++t) r.psi[t] = p.psi[t] + (low ? 0u : p.high[t]);
-    r.coef = p.coef + (low ? 0u : p.coef_high);
-    return r;
-}
 
 template <typename real, bool forward, int INV, bool FLAT>
 __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const unsigned item) {
@@ -433,13 +367,6 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
         dst += plane;
     }
 }
-
-// The wavefront's number among those of its grid, as a scalar.
-__device__ __forceinline__ unsigned wave_item(unsigned block) {
-    return block * 4u + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-}
-
-constexpr unsigned kXcdRun = 128;
 
 template <typename real, bool forward, int INV, bool FLAT>
 __global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void plane_half_step_kernel(const PlaneStep<real> a) {
@@ -741,18 +668,6 @@ int make_half_step(const tfdtd_half_step* d, HalfStep<real>* a) {
     a->counter = reinterpret_cast<const long long*>(d->counter);
     return TFDTD_OK;
 }
-
-// Planes per march: two share the lane's set-up and the plane between them (18.9 against 20.7 us a step on
-// 160x120x40 cells, 12,000 column-planes; 22.2 against 24.7 us on 97x83x61 in FP64, 7,760; four planes:
-// 18.8 and 22.3).  A grid of few wavefronts keeps one, as it needs them all to fill the chip: 7.3 us
-// against 8.5 on 160x120x1, 320 column-planes.
-constexpr long long kSpanItems = 4096;
-
-// Workgroups that one XCD takes in a row: neighbouring rows and planes are then read through one L2.
-// Runs of 1 / 32 / 128 take 40.0 / 36.5 / 35.7 us on 200x160x60 cells, 117.7 / 106.8 / 105.9 us on 192^3 and
-// 292 / 304 / 286 us on 256^3 (384: 299); grids of few workgroups take shorter runs (97x83x61, 970
-// workgroups: 20.9 us with 32, 22.2 with 128) so that every XCD has its share.
-inline unsigned xcd_run(long long blocks) { return (unsigned)std::min<long long>(std::max<long long>(blocks / 32, 1), kXcdRun); }
 
 template <typename real>
 long long plane_blocks(const PlaneStep<real>& a) {
