@@ -237,6 +237,25 @@ int tfdtd_step_fused(const tfdtd_half_step* e_step, const tfdtd_half_step* h_ste
                      const tfdtd_plane* planes, int32_t plane_count,
                      const tfdtd_observe* observe, int32_t n_steps, void* stream);
 
+/* tfdtd_step_fused for one step with its observation folded into the half steps: the E launch copies the
+ * counter to `shadow` (device int64, the caller's scratch), the H launch steps the counter on and records up to
+ * TFDTD_FOLDED_TRACES traces at the cells it updates, and the planes and longer trace tables read the copy.
+ * `cells`, host memory, names the traces of `observe` as values of the grid's own fields (null: the table is
+ * read).  Half steps that the plane march does not take run as tfdtd_step_fused. */
+#define TFDTD_FOLDED_TRACES 16
+typedef struct tfdtd_trace_cell {
+    int64_t element;                /* ((x*ny+y)*nz+z)*3+c */
+    int32_t magnetic;               /* 0 E, 1 H */
+    int32_t reserved;
+} tfdtd_trace_cell;
+
+int tfdtd_step_observed(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_plane* planes,
+                        int32_t plane_count, const tfdtd_observe* observe, const tfdtd_trace_cell* cells, int64_t* shadow,
+                        void* stream);
+
+/* The traces at step *observe->counter (a shadow, after a step), without advancing it. */
+int tfdtd_record_traces(const tfdtd_observe* observe, void* stream);
+
 /* Uneven batches: many grids of any shape advance together, one launch per family.
  * torchfdtd/cuda_batch.py:19-71 (FusedBatchYeeCUDA, identical-topology cohorts) generalised to
  * grids of different shapes, CPML layouts and sources.  tfdtd_batch_pack validates `count`
@@ -248,6 +267,12 @@ size_t tfdtd_batch_table_bytes(int32_t count, int32_t dtype);
 int tfdtd_batch_pack(const tfdtd_half_step* steps, int32_t count, void* host_table, size_t bytes, int32_t* block_prefix);
 int tfdtd_batch_half_step(const void* device_table, const int32_t* device_prefix, int32_t count, int32_t total_blocks,
                           int32_t dtype, int32_t family, void* stream);
+
+/* Both half steps of every grid of a batch that shares one counter: the E launch copies it to `shadow` (device
+ * int64) and the H launch steps it on, so no launch is needed for that.  The E table's descriptors read the
+ * counter; the H table's, and the planes and traces of the step, must read the shadow. */
+int tfdtd_batch_step(const void* e_table, const int32_t* e_prefix, int32_t e_blocks, const void* h_table, const int32_t* h_prefix,
+                     int32_t h_blocks, int32_t count, int32_t dtype, int64_t* counter, int64_t* shadow, void* stream);
 
 /* The one-pass step of many grids (tfdtd_yee_step_march descriptors of one dtype, tile_y and
  * eps_stride): three launches per step -- interior, z-face and boundary tiles -- each covering

@@ -94,3 +94,26 @@ def test_batched_march_and_general_grids_together(gpu):
     for run, single in zip(runs, singles):
         for a, b in zip(state(run), state(single)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('count', [1, 16, 17])
+def test_observed_step_equals_the_separate_launches(gpu, count):
+    """Traces folded into the H launch (up to 16) and read from the table beyond, against E, H, planes, traces and counter
+    as separate launches: the same trace rows and counter, the last steps past the end of the rows."""
+    from torchfdtd_amd import _native as N
+    shape, lib = (13, 12, 17), N.library()
+    runs = [stepper(shape, 'float32', 'cell', {}, 3) for _ in range(2)]
+    last = 3*shape[0]*shape[1]*shape[2]-1
+    flats = [0, last, 5, last-1, *np.random.default_rng(2).integers(0, last, 13).tolist()][:count]
+    for run in runs:
+        run.steps = 6
+        run.set_trace_points([(k % 2 == 1, flat) for k, flat in enumerate(flats)])
+    for _ in range(8):
+        runs[0].step()
+        N.check(lib.tfdtd_step_fused(ctypes.byref(runs[1].e_step), ctypes.byref(runs[1].h_step), runs[1].plane_table, 0,
+                                     ctypes.byref(runs[1].observe), 1, N.stream_handle()), 'separate')
+    torch.cuda.synchronize()
+    assert runs[0].counter.item() == runs[1].counter.item() == 8
+    assert torch.equal(runs[0].traces, runs[1].traces) and bool((runs[0].traces != 0).all())
+    for a, b in zip(state(runs[0]), state(runs[1])):
+        assert torch.equal(a, b)

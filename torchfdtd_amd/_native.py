@@ -85,6 +85,13 @@ class Observe(ctypes.Structure):
     _fields_ = [('dtype', i32), ('count', i32), ('table', vp), ('traces', vp), ('steps', i64), ('counter', vp)]
 
 
+FOLDED_TRACES = 16
+
+
+class TraceCell(ctypes.Structure):
+    _fields_ = [('element', i64), ('magnetic', i32), ('reserved', i32)]
+
+
 class Plane(ctypes.Structure):
     _fields_ = [('dtype', i32), ('spectral', i32), ('points', i64), ('frequencies', i32),
                 ('components', i32), ('electric', i32), ('corners', i32), ('time_downsample', i32),
@@ -171,6 +178,10 @@ PROTOTYPES = {
     'tfdtd_batch_table_bytes': (ctypes.c_size_t, [i32, i32]),
     'tfdtd_batch_pack': (i32, [ctypes.POINTER(HalfStep), i32, vp, ctypes.c_size_t, ctypes.POINTER(i32)]),
     'tfdtd_batch_half_step': (i32, [vp, vp, i32, i32, i32, i32, vp]),
+    'tfdtd_batch_step': (i32, [vp, vp, i32, vp, vp, i32, i32, i32, vp, vp, vp]),
+    'tfdtd_record_traces': (i32, [ctypes.POINTER(Observe), vp]),
+    'tfdtd_step_observed': (i32, [ctypes.POINTER(HalfStep), ctypes.POINTER(HalfStep), ctypes.POINTER(Plane), i32,
+                                  ctypes.POINTER(Observe), ctypes.POINTER(TraceCell), vp, vp]),
     'tfdtd_batch_march_bytes': (ctypes.c_size_t, [i32, i32]),
     'tfdtd_batch_march_pack': (i32, [ctypes.POINTER(March), i32, vp, ctypes.c_size_t, ctypes.POINTER(i32)]),
     'tfdtd_batch_march': (i32, [vp, vp, i32, i32, i32, i32, ctypes.POINTER(i32), vp]),

@@ -208,8 +208,11 @@ class Cohort:
         count = len(self.runs)
         self.e_table, self.e_prefix, e_host = _pack(lambda n: lib.tfdtd_batch_table_bytes(n, self.dtype), lib.tfdtd_batch_pack,
                                                     [run.e_step for run in self.runs], 1, device)
+        # The split step's copy of the counter, which the H launch, the planes and the traces read (the E launch writes
+        # it and the H launch steps the counter on).
+        self.shadow = torch.zeros(1, device=device, dtype=torch.long)
         self.h_table, self.h_prefix, h_host = _pack(lambda n: lib.tfdtd_batch_table_bytes(n, self.dtype), lib.tfdtd_batch_pack,
-                                                    [run.h_step for run in self.runs], 1, device)
+                                                    [self._shadowed(run.h_step) for run in self.runs], 1, device)
         self.e_blocks, self.h_blocks = int(e_host[0, count]), int(h_host[0, count])
         # Point traces of the whole cohort: columns [offset[i], offset[i+1]) belong to run i.
         self.trace_offsets = np.cumsum([0]+[len(run.trace_points) for run in self.runs])
@@ -218,6 +221,8 @@ class Cohort:
         self.trace_table = self._cohort_traces([run.trace_table for run in self.runs])
         self.observe = self._observe(self.trace_table)
         self.planes = self._pack_planes([run.plane_table[k] for run in self.runs for k in range(len(run.planes))])
+        self.planes_s = self._pack_planes([self._shadowed(run.plane_table[k]) for run in self.runs for k in range(len(run.planes))])
+        self.observe_s = self._shadowed(self.observe)
         if one_pass:
             self.march = []
             for k in range(2):
@@ -243,6 +248,12 @@ class Cohort:
         o.steps = self.steps
         o.counter = self.counter.data_ptr()
         return o
+
+    def _shadowed(self, descriptor):
+        """A copy of a descriptor that reads the shadow instead of the counter."""
+        copy = type(descriptor).from_buffer_copy(descriptor)
+        copy.counter = self.shadow.data_ptr()
+        return copy
 
     def _pack_planes(self, descriptors):
         """One batched DFT launch per (field dtype, accumulator precision) group of planes."""
@@ -297,22 +308,24 @@ class Cohort:
             states.extend(s for s in run.states() if s is not run.counter)
         return states
 
-    def _monitors(self, planes, observe, stream):
-        lib = self.lib
+    def _planes_update(self, planes, stream):
         for table, count, blocks, frequencies, dtype, spectral in planes:
-            N.check(lib.tfdtd_batch_dft_update(table.data_ptr(), count, blocks, frequencies, dtype, spectral, stream),
+            N.check(self.lib.tfdtd_batch_dft_update(table.data_ptr(), count, blocks, frequencies, dtype, spectral, stream),
                     'tfdtd_batch_dft_update')
-        N.check(lib.tfdtd_observe_step(ctypes.byref(observe), stream), 'tfdtd_observe_step')
+
+    def _monitors(self, planes, observe, stream):
+        self._planes_update(planes, stream)
+        N.check(self.lib.tfdtd_observe_step(ctypes.byref(observe), stream), 'tfdtd_observe_step')
 
     def step(self):
         """One step of every grid with the split kernels (state in the grids' own buffers)."""
         stream = N.stream_handle()
-        lib, count = self.lib, len(self.runs)
-        N.check(lib.tfdtd_batch_half_step(self.e_table.data_ptr(), self.e_prefix.data_ptr(), count, self.e_blocks,
-                                          self.dtype, N.FAMILY_E, stream), 'tfdtd_batch_half_step E')
-        N.check(lib.tfdtd_batch_half_step(self.h_table.data_ptr(), self.h_prefix.data_ptr(), count, self.h_blocks,
-                                          self.dtype, N.FAMILY_H, stream), 'tfdtd_batch_half_step H')
-        self._monitors(self.planes, self.observe, stream)
+        N.check(self.lib.tfdtd_batch_step(self.e_table.data_ptr(), self.e_prefix.data_ptr(), self.e_blocks, self.h_table.data_ptr(),
+                                          self.h_prefix.data_ptr(), self.h_blocks, len(self.runs), self.dtype,
+                                          self.counter.data_ptr(), self.shadow.data_ptr(), stream), 'tfdtd_batch_step')
+        self._planes_update(self.planes_s, stream)
+        if self.observe_s.count:
+            N.check(self.lib.tfdtd_record_traces(ctypes.byref(self.observe_s), stream), 'tfdtd_record_traces')
 
     def step_pair(self):
         """Two steps with the one-pass kernels: grid buffers -> second set -> grid buffers."""

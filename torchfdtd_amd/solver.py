@@ -275,6 +275,8 @@ class Stepper:
         device, real = g.E.device, g.dtype
         # A batch shares one counter among its grids.
         self.counter = torch.zeros(1, device=device, dtype=torch.long) if counter is None else counter
+        # The split step's copy of the counter: written by its E launch, read by the launches after it.
+        self.shadow = torch.zeros(1, device=device, dtype=torch.long)
         terms = source_terms(p, self.steps)
         self.sources = {'E': [], 'H': []}
         for t in terms:
@@ -435,6 +437,9 @@ class Stepper:
         self.plane_table = self._planes(g.E, g.H)
         self.trace_table = self._trace_table(g.E, g.H)
         self.observe = self._observe(self.trace_table)
+        self.trace_cells = None
+        if 0 < len(self.trace_points) <= N.FOLDED_TRACES:
+            self.trace_cells = (N.TraceCell*len(self.trace_points))(*(N.TraceCell(flat, int(m), 0) for m, flat in self.trace_points))
         if self.one_pass:
             if self.materials is not None:
                 self.materials.refresh()     # the permittivity may have been replaced (a widened layout)
@@ -612,8 +617,9 @@ class Stepper:
             self._dispersive_step(stream)
             return
         if self.kernel == 'hip':
-            N.check(self.lib.tfdtd_step_fused(ctypes.byref(self.e_step), ctypes.byref(self.h_step), self.plane_table,
-                                              len(self.planes), ctypes.byref(self.observe), 1, stream), 'tfdtd_step_fused')
+            N.check(self.lib.tfdtd_step_observed(ctypes.byref(self.e_step), ctypes.byref(self.h_step), self.plane_table,
+                                                 len(self.planes), ctypes.byref(self.observe), self.trace_cells,
+                                                 self.shadow.data_ptr(), stream), 'tfdtd_step_observed')
             return
         g = self.grid
         g.update_E()
