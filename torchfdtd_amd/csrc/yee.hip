@@ -526,11 +526,14 @@ __device__ __forceinline__ void phases(const Plane<real, spec>& a, long long ste
     p[3] = er * hi + ei * hr;
 }
 
-// Interpolated sample of (point, component) i at step n, times the window.
+// n % d of a step number, in 32 bits where it fits (a 64-bit remainder takes some 150 instructions).
+__device__ __forceinline__ int step_mod(long long n, int d) {
+    return (n >> 31) == 0 ? (int)((unsigned)n % (unsigned)d) : (int)(n % d);
+}
+
+// Interpolated sample of (point p, component c) at step n, times the window.
 template <typename real, typename spec>
-__device__ __forceinline__ real plane_sample(const Plane<real, spec>& a, long long i, long long n) {
-    const int c = (int)(i % a.nc);
-    const long long p = i / a.nc;
+__device__ __forceinline__ real plane_sample(const Plane<real, spec>& a, long long p, int c, long long n) {
     const bool electric = c < a.ne;
     const auto field = global(electric ? a.E : a.H);
     const auto idx = global(a.indices[c]);
@@ -560,9 +563,14 @@ __device__ __forceinline__ real plane_sample(const Plane<real, spec>& a, long lo
 }
 
 // Accumulate the staged samples of steps [lo, hi) (one block at most): the phases of those steps go
-// to LDS, each thread sums its sample's products in FP64 and adds the sum to its accumulators.
+// to LDS, each thread sums its sample's products in FP64 and adds the sum to its accumulators.  The
+// staged values are read once per kFlushGroup frequencies and the remainders of the step numbers formed
+// once (a pair of 64-bit remainders per step and frequency made the flush of 29,376 samples x 8
+// frequencies x 32 steps take 90 us, twice a step's half steps).
+constexpr int kFlushGroup = 4;
+
 template <typename real, typename spec>
-__device__ __forceinline__ void flush_range(const Plane<real, spec>& a, long long i, long long lo, long long hi) {
+__device__ __forceinline__ void flush_range(const Plane<real, spec>& a, long long i, int c, long long lo, long long hi) {
     extern __shared__ unsigned char lds_raw[];
     spec* phase = reinterpret_cast<spec*>(lds_raw);
     const int count = (int)(hi - lo);
@@ -570,21 +578,46 @@ __device__ __forceinline__ void flush_range(const Plane<real, spec>& a, long lon
     __syncthreads();
     const long long samples = a.points * a.nc;
     if (i >= samples) return;
-    const int o = (int)(i % a.nc) < a.ne ? 0 : 2;
-    for (int f = 0; f < a.nf; ++f) {
-        double sr = 0., si = 0.;
+    const int o = c < a.ne ? 0 : 2;
+    const int slot = step_mod(lo, a.block), skip = step_mod(lo, a.downsample);
+    for (int f = 0; f < a.nf; f += kFlushGroup) {
+        double sr[kFlushGroup], si[kFlushGroup];
+#pragma unroll
+        for (int g = 0; g < kFlushGroup; ++g) sr[g] = si[g] = 0.;
+        int s = slot, m = skip;
         for (int j = 0; j < count; ++j) {
-            const long long step = lo + j;
-            if (step % a.downsample) continue;
-            const spec v = (spec)global(a.stage)[(step % a.block) * samples + i];
-            const spec* p = phase + 4 * (j * a.nf + f) + o;
-            sr += (double)(p[0] * v);
-            si += (double)(p[1] * v);
+            if (m == 0) {
+                const spec v = (spec)global(a.stage)[s * samples + i];
+#pragma unroll
+                for (int g = 0; g < kFlushGroup; ++g) {
+                    const spec* p = phase + 4 * (j * a.nf + min(f + g, a.nf - 1)) + o;
+                    sr[g] += (double)(p[0] * v);
+                    si[g] += (double)(p[1] * v);
+                }
+            }
+            if (++s == a.block) s = 0;
+            if (++m == a.downsample) m = 0;
         }
-        const auto out = global(a.value + 2 * ((long long)f * samples + i));
-        out[0] = out[0] + (spec)sr;
-        out[1] = out[1] + (spec)si;
+#pragma unroll
+        for (int g = 0; g < kFlushGroup; ++g)
+            if (f + g < a.nf) {
+                const auto out = global(a.value + 2 * ((long long)(f + g) * samples + i));
+                out[0] = out[0] + (spec)sr[g];
+                out[1] = out[1] + (spec)si[g];
+            }
     }
+}
+
+// The component of sample i, and its point.
+template <typename real, typename spec>
+__device__ __forceinline__ int sample_component(const Plane<real, spec>& a, long long i, long long* point) {
+    if (a.points * a.nc < 0x7fffffffLL) {
+        const unsigned p = (unsigned)i / (unsigned)a.nc;
+        *point = p;
+        return (int)((unsigned)i - p * (unsigned)a.nc);
+    }
+    *point = i / a.nc;
+    return (int)(i - *point * a.nc);
 }
 
 // One thread per (point, component) sample.  Per-step accumulation (block <= 1): the block first
@@ -598,21 +631,25 @@ __device__ __forceinline__ void dft_plane_block(const Plane<real, spec>& a, long
     if (n >= a.samples) return;
     const long long samples = a.points * a.nc;
     const long long i = block * blockDim.x + threadIdx.x;
+    long long point;
+    const int c = sample_component(a, i, &point);
+    const bool taken = a.downsample == 1 || step_mod(n, a.downsample) == 0;
     if (a.block > 1) {
-        if (n % a.downsample == 0 && i < samples) global(a.stage)[(n % a.block) * samples + i] = plane_sample(a, i, n);
-        if ((n + 1) % a.block == 0 || n + 1 == a.samples) {
-            const long long first = n - n % a.block;
+        const int slot = step_mod(n, a.block);
+        if (taken && i < samples) global(a.stage)[slot * samples + i] = plane_sample(a, point, c, n);
+        if (slot + 1 == a.block || n + 1 == a.samples) {
+            const long long first = n - slot;
             const long long flushed = *global(a.flushed);
-            flush_range(a, i, first > flushed ? first : flushed, n + 1);
+            flush_range(a, i, c, first > flushed ? first : flushed, n + 1);
         }
         return;
     }
-    if (n % a.downsample) return;
+    if (!taken) return;
     for (int f = threadIdx.x; f < a.nf; f += blockDim.x) phases(a, n, f, phase + 4 * f);
     __syncthreads();
     if (i >= samples) return;
-    const spec sv = (spec)plane_sample(a, i, n);
-    const int o = (int)(i % a.nc) < a.ne ? 0 : 2;
+    const spec sv = (spec)plane_sample(a, point, c, n);
+    const int o = c < a.ne ? 0 : 2;
     for (int f = 0; f < a.nf; ++f) {
         const auto out = global(a.value + 2 * ((long long)f * samples + i));
         out[0] = out[0] + phase[4 * f + o] * sv;
@@ -625,10 +662,13 @@ template <typename real, typename spec>
 __global__ __launch_bounds__(256) void dft_flush_kernel(const Plane<real, spec> a) {
     const long long n = *a.counter < a.samples ? *a.counter : a.samples;
     if (a.block <= 1 || n == a.samples) return;     // a finished window was accumulated by its last step
-    const long long first = n - n % a.block;
+    const long long first = n - step_mod(n, a.block);
     const long long lo = first > *a.flushed ? first : *a.flushed;
     if (lo >= n) return;
-    flush_range(a, (long long)blockIdx.x * blockDim.x + threadIdx.x, lo, n);
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    long long point;
+    const int c = sample_component(a, i, &point);
+    flush_range(a, i, c, lo, n);
 }
 
 __global__ void set_flushed_kernel(const long long* counter, long long samples, long long* flushed) {
