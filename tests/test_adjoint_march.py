@@ -41,3 +41,24 @@ def test_gradient_of_marched_grids_matches_the_oracle(gpu, shape, precision, fac
     _, part, _ = engine_gradient(project, eps, weights, AdjointOptions(design_box=box))
     inside = tuple(slice(a, b) for a, b in box)
     assert np.array_equal(part[inside], got[inside])
+
+
+def test_plane_observers_are_numbered_as_they_first_appear(gpu):
+    from torchfdtd_amd.adjoint import COMPONENTS, DifferentiablePlaneSimulation
+    from torchfdtd_amd.models import FieldMonitor, SpectrumSettings
+    from torchfdtd_amd.monitors import interpolation_map
+    spectrum = SpectrumSettings(sampling='wavelength', frequency_points=2, wavelength_start=1, wavelength_stop=2, apodization='none')
+    planes = [('x', (.2, 0, 0), (0, .8, .8)), ('x', (.23, .1, 0), (0, .5, .6)), ('y', (0, .1, 0), (.7, 0, .6))]
+    project = Project(region=Region(dimension='3d', size=(1.7, 1.6, 1.9), mesh=.1, pml_cells=3, steps=20), sources=[Source(id='s')],
+                      monitors=[FieldMonitor(id=f'm{i}', normal=n, center=c, size=s, spectrum=spectrum) for i, (n, c, s) in enumerate(planes)])
+    model = DifferentiablePlaneSimulation(project)
+    expected = []
+    for _, _, plan, maps in model.plans:
+        for component, (numbers, _) in zip(COMPONENTS, maps):
+            indices, _ = interpolation_map(project.region, component, plan['points_um'])
+            for flat, number in zip(indices.reshape(-1).tolist(), numbers.reshape(-1).tolist()):
+                if number == len(expected):
+                    expected.append((component[0] == 'H', flat))
+                assert expected[number] == (component[0] == 'H', flat)
+    assert model.observers == expected and len(set(expected)) == len(expected)
+    assert model.components == tuple('H' if m else 'E' for m, _ in expected)

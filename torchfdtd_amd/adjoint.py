@@ -38,7 +38,7 @@ from .models import Project
 from .monitors import interpolation_map, plane_plan
 from .planning import index_at, periodic_axes
 from .plan import resolve_plan
-from .solver import Stepper
+from .solver import Stepper, TracePoints
 
 COMPONENTS = ('Ex', 'Ey', 'Ez', 'Hx', 'Hy', 'Hz')
 
@@ -241,7 +241,7 @@ class _Engine:
         self.reverse_counter = torch.zeros(1, device=g.device, dtype=torch.long)
         # Seeds: one target per observer (the observers are distinct elements).
         points = run.trace_points
-        targets = np.array([(int(m), flat) for m, flat in points], dtype=np.int64).reshape(-1, 2)
+        targets = np.stack([points.magnetic.astype(np.int64), points.flat], axis=1)
         self.seed_targets = torch.as_tensor(targets, device=g.device)
         self.seed_offsets = torch.arange(len(points)+1, device=g.device, dtype=torch.int32)
         self.seed_columns = torch.arange(len(points), device=g.device, dtype=torch.int32)
@@ -264,7 +264,7 @@ class _Engine:
                 bars = self.psi_bar[forward]
                 setattr(d, name, march_family(g, forward, bars[parity], bars[1-parity]))
             d.nseed = len(points)
-            if points:
+            if len(points):
                 d.seed_targets, d.seed_offsets = self.seed_targets.data_ptr(), self.seed_offsets.data_ptr()
                 d.seed_columns, d.seeds = self.seed_columns.data_ptr(), self.seeds.data_ptr()
                 d.seed_width, d.seed_rows = len(points), self.seeds.shape[0]
@@ -443,7 +443,8 @@ class DifferentiablePlaneSimulation(torch.nn.Module):
         if not active or any(m.kind != 'field' for m in active):
             raise ValueError('DifferentiablePlaneSimulation requires enabled field monitors only.')
         r = self.project.region
-        self.plans, observers, lookup = [], [], {}
+        # The observers: every field element an interpolation reads, once, numbered in the order they first appear.
+        self.plans, parts, lookup, count = [], [], {}, 0
         for raw in active:
             monitor = self.project.resolved_monitor(raw)
             if monitor.time_downsample != 1 or monitor.spectrum.apodization != 'none':
@@ -452,19 +453,28 @@ class DifferentiablePlaneSimulation(torch.nn.Module):
             maps = []
             for component in COMPONENTS:
                 indices, weights = interpolation_map(r, component, plan['points_um'])
-                flat = indices.reshape(-1)
-                numbers = np.empty(flat.shape, dtype=np.int64)
-                known = lookup.setdefault(component, {})
-                for k, index in enumerate(flat.tolist()):
-                    number = known.get(index)
-                    if number is None:
-                        number = known[index] = len(observers)
-                        observers.append((component[0] == 'H', index))
-                    numbers[k] = number
-                maps.append((numbers.reshape(indices.shape), weights))
+                values, first, inverse = np.unique(indices.reshape(-1), return_index=True, return_inverse=True)
+                known, known_numbers = lookup.get(component, (np.empty(0, np.int64), np.empty(0, np.int64)))
+                at = np.searchsorted(known, values)
+                seen = np.zeros(len(values), dtype=bool)
+                if len(known):
+                    seen = known[np.minimum(at, len(known)-1)] == values
+                numbers = np.empty(len(values), dtype=np.int64)
+                numbers[seen] = known_numbers[at[seen]]
+                fresh = np.flatnonzero(~seen)
+                fresh = fresh[np.argsort(first[fresh], kind='stable')]
+                numbers[fresh] = count+np.arange(len(fresh))
+                count += len(fresh)
+                parts.append((component[0] == 'H', values[fresh]))
+                merged = np.concatenate([known, values[fresh]])
+                order = np.argsort(merged, kind='stable')
+                lookup[component] = (merged[order], np.concatenate([known_numbers, numbers[fresh]])[order])
+                maps.append((numbers[inverse].reshape(indices.shape), weights))
             self.plans.append((monitor.id, monitor.normal, plan, maps))
-        self.observers = observers
-        self.components = tuple(('H' if m else 'E') for m, _ in observers)
+        magnetic = np.concatenate([np.full(len(flat), m) for m, flat in parts])
+        self._points = TracePoints.of(magnetic, np.concatenate([flat for _, flat in parts]))
+        self.observers = list(self._points)
+        self.components = tuple(np.where(magnetic, 'H', 'E').tolist())
 
     @property
     def plan(self):
@@ -480,14 +490,14 @@ class DifferentiablePlaneSimulation(torch.nn.Module):
     def forward(self, epsilon, frequency_hz):
         _check_epsilon(epsilon, self.project.region)
         r = self.project.region
-        engine = _Engine(_internal_project(self.project), epsilon.detach(), self.observers, self.options)
+        engine = _Engine(_internal_project(self.project), epsilon.detach(), self._points, self.options)
         signals = _Simulate.apply(epsilon, engine).to(torch.float64)
         device = signals.device
         f = torch.as_tensor(frequency_hz, device=device, dtype=torch.float64).reshape(-1)
         if not bool(torch.isfinite(f).all()) or bool((f <= 0).any()) or bool((f*r.time_step >= .5).any()):
             raise ValueError('Frequencies must be finite, positive and below temporal Nyquist.')
         t = (torch.arange(signals.shape[0], device=device, dtype=torch.float64)+1)*r.time_step
-        magnetic = torch.as_tensor([c == 'H' for c in self.components], device=device)
+        magnetic = torch.as_tensor(self._points.magnetic, device=device)
         spectra = torch.zeros((f.numel(), signals.shape[1]), device=device, dtype=torch.complex128)
         for family in (False, True):
             columns = torch.nonzero(magnetic == family).flatten()

@@ -14,6 +14,7 @@ import json
 import math
 import threading
 import time
+from collections.abc import Sequence
 from dataclasses import dataclass, field
 from functools import cached_property
 from pathlib import Path
@@ -250,6 +251,36 @@ def dispersive_materials(project, grid, ownership):
     return states
 
 
+class TracePoints(Sequence):
+    """The recorded points of a run, (magnetic, flat element index) pairs, held as two arrays: a plane objective has
+    tens of thousands of them, and tables are made from the arrays at once."""
+
+    def __init__(self, points):
+        if isinstance(points, TracePoints):
+            self.magnetic, self.flat = points.magnetic, points.flat
+            return
+        points = list(points)
+        self.magnetic = np.fromiter((bool(m) for m, _ in points), dtype=bool, count=len(points))
+        self.flat = np.fromiter((int(f) for _, f in points), dtype=np.int64, count=len(points))
+
+    @classmethod
+    def of(cls, magnetic, flat):
+        out = cls(())
+        out.magnetic, out.flat = np.asarray(magnetic, dtype=bool), np.asarray(flat, dtype=np.int64)
+        return out
+
+    def __len__(self):
+        return len(self.flat)
+
+    def __getitem__(self, k):
+        if isinstance(k, slice):
+            return list(zip(self.magnetic[k].tolist(), self.flat[k].tolist()))
+        return bool(self.magnetic[k]), int(self.flat[k])
+
+    def __iter__(self):
+        return iter(zip(self.magnetic.tolist(), self.flat.tolist()))
+
+
 class Stepper:
     """Device state of one resident run and its step (the reference's closure, solver.py:776-797)."""
 
@@ -282,11 +313,12 @@ class Stepper:
         for t in terms:
             self.sources[t.family].append((t.comp, t.box, torch.as_tensor(t.values, device=device)))
         self.point_monitors = [p.resolved_monitor(m) for m in p.monitors if m.enabled and m.kind == 'point']
-        self.trace_points = []
+        points = []
         for m in self.point_monitors:
             loc = index_at(m.center, r, m.component)
             flat = ((loc[0]*r.shape[1]+loc[1])*r.shape[2]+loc[2])*3+'xyz'.index(m.component[1].lower())
-            self.trace_points.append((m.component[0] == 'H', flat))
+            points.append((m.component[0] == 'H', flat))
+        self.trace_points = TracePoints(points)
         self.traces = torch.zeros((self.steps, len(self.trace_points)), device=device, dtype=real)
         self.planes = [FrequencyPlane(g, p.resolved_monitor(m)) for m in p.monitors if m.enabled and m.kind == 'field']
         if self.kernel == 'torch':
@@ -397,15 +429,16 @@ class Stepper:
 
     def set_trace_points(self, points):
         """Replace the recorded traces by `points`: (magnetic, flat element index) pairs."""
-        self.trace_points = [(bool(m), int(flat)) for m, flat in points]
+        self.trace_points = TracePoints(points)
         self.traces = torch.zeros((self.steps, len(self.trace_points)), device=self.grid.device, dtype=self.grid.dtype)
         self.two_step = self.two_step and self._two_step_allowed()   # the traces may widen the snapshot
         self._describe()
 
     def _trace_table(self, E, H):
         """int64 (address, element index) of every point trace in the fields E, H."""
-        rows = [((H if magnetic else E).data_ptr(), flat) for magnetic, flat in self.trace_points]
-        return torch.as_tensor(np.array(rows, dtype=np.int64).reshape(-1, 2), device=E.device)
+        points = self.trace_points
+        fields = np.where(points.magnetic, np.int64(H.data_ptr()), np.int64(E.data_ptr()))
+        return torch.as_tensor(np.stack([fields, points.flat], axis=1), device=E.device)
 
     def _observe(self, table):
         g = self.grid
@@ -481,8 +514,7 @@ class Stepper:
                     for k, plane in enumerate(self.planes):
                         self.plane_table_s[k] = plane.descriptor(self.counter, self.snap_e, self.snap_h,
                                                                  indices=self.snap_indices[k])
-                    flats = self._snapshot_index(torch.as_tensor([flat for _, flat in self.trace_points], dtype=torch.long,
-                                                                 device=g.E.device), boxes).tolist()
+                    flats = self._snapshot_index(torch.as_tensor(self.trace_points.flat, device=g.E.device), boxes).tolist()
                     rows = [((self.snap_h if magnetic else self.snap_e).data_ptr(), f)
                             for (magnetic, _), f in zip(self.trace_points, flats)]
                     self.trace_table_s = torch.as_tensor(np.array(rows, dtype=np.int64).reshape(-1, 2), device=g.E.device)
