@@ -197,8 +197,10 @@ __global__ __launch_bounds__(256) void yee_half_step_kernel(const HalfStep<real>
 // costs little more than its own arithmetic.  One thread per cell of the whole grid (half_step_cell) was
 // bound by its 64-bit divisions, per-term slab tests and dependent descriptor loads: a step of both
 // families plus its trace took 26.5 us on 160x120x40 cells, 49.1 us on 200x160x60, 124 us on 192^3, 325 us
-// on 256^3 (FP32), 30.5 us on 97x83x61 (FP64); the march takes 18.1, 35.7, 106, 286 and 20.9 us.  What
-// bounds it now is the traffic: past the 256 MB cache 5 TB/s of a copy's 5.5, inside it about 6 of 8.2.
+// on 256^3 (FP32), 30.5 us on 97x83x61 (FP64); the march takes 16.7, 33.6, 108, 285 and 18.9 us.  A cell of a
+// wavefront without slab rows executes about 45 vector instructions (with the lanes' 64-bit address sums and
+// the slabs' arithmetic left to every wavefront: 110, and 18.1, 35.7, 106, 286 and 20.9 us).  What bounds it
+// now is the traffic: past the 256 MB cache 5.3 TB/s of a copy's 5.5, inside it 6.4 of 8.2.
 constexpr int kPlaneTraces = TFDTD_FOLDED_TRACES;
 
 struct PlaneTrace {         // a point trace: its cell and value, and its column among the run's traces
@@ -210,7 +212,7 @@ struct PlaneStep {
     int nx, ny, nz, nyz;
     int span, columns;      // planes per march, 64-cell columns of a plane
     Divider by_nz, by_columns;
-    int xcd, spare;         // workgroups an XCD takes in a row
+    int xcd, chunks;        // workgroups an XCD takes in a row, marches along x
     const real* src;
     real* dst;
     const real* inverse;
@@ -245,19 +247,20 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
     constexpr unsigned W = sizeof(real);
     const int nx = a.nx, ny = a.ny, nz = FLAT ? 1 : a.nz, nyz = a.nyz;
     // Spare lanes of the last column and spare wavefronts of the last workgroup repeat a cell and store nothing.
-    const unsigned chunks = (unsigned)(nx + a.span - 1) / (unsigned)a.span;
-    const unsigned xchunk = min(divide(item, a.by_columns), chunks - 1u);
+    const unsigned xchunk = min(divide(item, a.by_columns), (unsigned)a.chunks - 1u);
     const unsigned cell = (item - xchunk * a.columns) * 64u + (threadIdx.x & 63u);
     const bool owned = cell < (unsigned)nyz;
     const unsigned r = min(cell, (unsigned)nyz - 1u);
     const int xa = (int)xchunk * a.span, xb = min(nx, xa + a.span);
     const int y = FLAT ? (int)r : (int)divide(r, a.by_nz), z = FLAT ? 0 : (int)(r - (unsigned)y * nz);
-    const unsigned off = r * (3 * W);
+    unsigned off = r * (3 * W), line = r * W;
     const bool iny = forward ? y < ny - 1 : y > 0, inz = !FLAT && (forward ? z < nz - 1 : z > 0);
     const bool wrapx = a.periodic_mask & 1, wrapy = a.periodic_mask & 2, wrapz = !FLAT && (a.periodic_mask & 4);
     const unsigned rowb = (unsigned)nz * (3 * W), lasty = (unsigned)(ny - 1) * rowb, lastz = (unsigned)(nz - 1) * (3 * W);
-    const unsigned offy = forward ? (iny ? off + rowb : wrapy ? off - lasty : off) : (iny ? off - rowb : wrapy ? off + lasty : off);
-    const unsigned offz = forward ? (inz ? off + 3 * W : wrapz ? off - lastz : off) : (inz ? off - 3 * W : wrapz ? off + lastz : off);
+    // The neighbour across y or z: the wrapped cell of a periodic axis, else the cell itself at its end.
+    const unsigned endy = wrapy ? (forward ? 0u - lasty : lasty) : 0u, endz = wrapz ? (forward ? 0u - lastz : lastz) : 0u;
+    unsigned offy = off + (iny ? (forward ? rowb : 0u - rowb) : endy);
+    unsigned offz = off + (inz ? (forward ? 3 * W : 0u - 3 * W) : endz);
     const long long plane = 3LL * nyz;
     const real* src = a.src + xa * plane;
     real* dst = a.dst + xa * plane;
@@ -292,15 +295,23 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
         }
     }
     const bool source = owned && a.nsrc > 0 && y >= a.box_lo[1] && y < a.box_hi[1] && z >= a.box_lo[2] && z < a.box_hi[2];
+    const bool sources = __builtin_amdgcn_ballot_w64(source) != 0;
+    real courant = a.courant;
+    asm volatile("" : "+s"(courant));   // read once, before the loop
+    // A wavefront without slab rows of an axis skips that axis's memory.
+    const bool anyy = __builtin_amdgcn_ballot_w64(hy.on) != 0, anyz = !FLAT && __builtin_amdgcn_ballot_w64(hz.on) != 0;
     real* const psi = a.psi;
     for (int x = xa; x < xb; ++x) {
+        // The lane offsets stay 32-bit values of the loop: widened once before it, every access would add them
+        // to its base in 64-bit vector arithmetic.
+        asm volatile("" : "+v"(off), "+v"(offy), "+v"(offz), "+v"(line));
         const bool inx = forward ? x < nx - 1 : x > 0;
         if (forward) side = cell_at_byte(inx ? src + plane : wrapx ? a.src : src, off);
         const Cell<real> old = cell_at_byte(dst, off);
         Cell<real> inv;
         if (INV == 3) inv = cell_at_byte(a.inverse + x * plane, off);
         else {
-            const real v = INV == 1 ? at_byte(a.inverse + (long long)x * nyz, r * W) : one;
+            const real v = INV == 1 ? at_byte(a.inverse + (long long)x * nyz, line) : one;
             inv = Cell<real>{{v, v, v}};
         }
         const Cell<real> nby = cell_at_byte(src, offy);
@@ -312,15 +323,15 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
         real mx[2], my[2], mz[2];
         const AxisRow<real> rx = axis_row(a.axis[0], x, inx);
         real bx = real(0), cx = real(0), ikx = real(0);
-        unsigned atx[2] = {0u, 0u};
+        real* psix[2] = {psi, psi};
         if (rx.on) {
-            const unsigned wide = (unsigned)rx.w * W, k = rx.coef + (unsigned)rx.q * W, e = ((unsigned)rx.q * nyz + r) * W;
+            const unsigned wide = (unsigned)rx.w * W, k = rx.coef + (unsigned)rx.q * W, e = (unsigned)rx.q * (unsigned)nyz * W;
             bx = at_byte(a.coef, k);
             cx = at_byte(a.coef, k + wide);
             ikx = at_byte(a.coef, k + 2 * wide);
             for (int t = 0; t < 2; ++t) {
-                atx[t] = rx.psi[t] + e;
-                mx[t] = at_byte(psi, atx[t]);
+                psix[t] = reinterpret_cast<real*>(reinterpret_cast<char*>(psi) + rx.psi[t] + e);
+                mx[t] = at_byte(psix[t], line);
             }
         }
         if (hy.on)
@@ -328,48 +339,58 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
         if (hz.on)
             for (int t = 0; t < 2; ++t) mz[t] = at_byte(psi, hz.at[t]);
         real curl[3] = {real(0), real(0), real(0)};
-        // The two terms of one axis: difference, CPML row, sum into the curl in term order.
-        auto axis_terms = [&](auto axis_tag, bool in, bool wrap, const Cell<real>& nb, bool hit, real b, real c, real ik, real* m) {
+        // The two terms of one axis: difference, CPML row (`any`: the wavefront has one), sum into the curl in
+        // term order.
+        auto axis_terms = [&](auto axis_tag, bool in, bool wrap, const Cell<real>& nb, bool any, bool hit, real b, real c, real ik, real* m) {
             constexpr int axis = decltype(axis_tag)::value;
-            const real pec = forward && ((a.pec_mask >> axis) & 1) ? -a.pec_factor[axis] : real(0);
             const bool pecs = forward && ((a.pec_mask >> axis) & 1);
+            const real pec = pecs ? -a.pec_factor[axis] : real(0);
+            real d[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int ic = term_in(2 * axis + k);
+                d[k] = forward ? nb.v[ic] - here.v[ic] : here.v[ic] - nb.v[ic];
+            }
+            if (any) {
+                asm volatile("");       // a branch: the rows' arithmetic is not run for every wavefront
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    m[k] = m[k] * b + c * d[k];
+                    const real stretched = d[k] * ik + m[k];
+                    d[k] = hit ? stretched : d[k];
+                }
+            }
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 const int t = 2 * axis + k, ic = term_in(t), oc = term_out(t);
-                real d = forward ? nb.v[ic] - here.v[ic] : here.v[ic] - nb.v[ic];
-                if (hit) {
-                    m[k] = m[k] * b + c * d;
-                    d = d * ik + m[k];
-                }
-                if (!in && !wrap) d = pecs ? pec * here.v[ic] : real(0);
-                curl[oc] = term_sign(t) > 0 ? curl[oc] + d : curl[oc] - d;
+                if (!in && !wrap) d[k] = pecs ? pec * here.v[ic] : real(0);
+                curl[oc] = term_sign(t) > 0 ? curl[oc] + d[k] : curl[oc] - d[k];
             }
         };
-        axis_terms(std::integral_constant<int, 0>{}, inx, wrapx, side, rx.on, bx, cx, ikx, mx);
-        axis_terms(std::integral_constant<int, 1>{}, iny, wrapy, nby, hy.on, hy.b, hy.c, hy.ik, my);
-        if (!FLAT) axis_terms(std::integral_constant<int, 2>{}, inz, wrapz, nbz, hz.on, hz.b, hz.c, hz.ik, mz);
+        axis_terms(std::integral_constant<int, 0>{}, inx, wrapx, side, rx.on, rx.on, bx, cx, ikx, mx);
+        axis_terms(std::integral_constant<int, 1>{}, iny, wrapy, nby, anyy, hy.on, hy.b, hy.c, hy.ik, my);
+        if (!FLAT) axis_terms(std::integral_constant<int, 2>{}, inz, wrapz, nbz, anyz, hz.on, hz.b, hz.c, hz.ik, mz);
         real out[3];
 #pragma unroll
         for (int m = 0; m < 3; ++m) {
-            const real coefficient = a.courant * inv.v[m];
+            const real coefficient = courant * inv.v[m];
             out[m] = forward ? old.v[m] - coefficient * curl[m] : old.v[m] + coefficient * curl[m];
         }
-        if (source && x >= a.box_lo[0] && x < a.box_hi[0]) {
+        if (sources && x >= a.box_lo[0] && x < a.box_hi[0]) {
             const long long n = *global(a.counter);
             for (int k = 0; k < a.nsrc && n < a.source_samples; ++k) {
                 const Source<real>& box = a.srcs[k];
-                if (x >= box.lo[0] && x < box.hi[0] && y >= box.lo[1] && y < box.hi[1] && z >= box.lo[2] &&
-                    z < box.hi[2]) {
-                    const real v = global(box.values)[n];
-                    if (box.comp == 0) out[0] = out[0] + v;
-                    else if (box.comp == 1) out[1] = out[1] + v;
-                    else out[2] = out[2] + v;
-                }
+                if (x < box.lo[0] || x >= box.hi[0]) continue;
+                const bool in = owned & (y >= box.lo[1]) & (y < box.hi[1]) & (z >= box.lo[2]) & (z < box.hi[2]);
+                const real v = global(box.values)[n];
+#pragma unroll
+                for (int m = 0; m < 3; ++m)
+                    if (box.comp == m && in) out[m] = out[m] + v;
             }
         }
         if (owned) {
             if (rx.on)
-                for (int t = 0; t < 2; ++t) put_byte(psi, atx[t], mx[t]);
+                for (int t = 0; t < 2; ++t) put_byte(psix[t], line, mx[t]);
             if (hy.on)
                 for (int t = 0; t < 2; ++t) put_byte(psi, hy.at[t], my[t]);
             if (hz.on)
@@ -392,7 +413,10 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
             }
         if (!forward) { side = here; here = ahead; }
         else here = side;
-        for (int t = 0; t < 2; ++t) { hy.at[t] += hy.stride; hz.at[t] += hz.stride; }
+        if (anyy)
+            for (int t = 0; t < 2; ++t) hy.at[t] += hy.stride;
+        if (anyz)
+            for (int t = 0; t < 2; ++t) hz.at[t] += hz.stride;
         src += plane;
         dst += plane;
     }
@@ -400,8 +424,8 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
 
 template <typename real, bool forward, int INV, bool FLAT>
 __global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void plane_half_step_kernel(const PlaneStep<real> a) {
-    carry_counter(a.counter, a.counter_to, a.counter_add);
     march_half_step<real, forward, INV, FLAT>(a, wave_item(xcd_block(blockIdx.x, gridDim.x, a.xcd)));
+    carry_counter(a.counter, a.counter_to, a.counter_add);
 }
 
 // One grid of a batched half step: its plane march where `march` is set, else the general step.
@@ -744,7 +768,7 @@ int make_half_step(const tfdtd_half_step* d, HalfStep<real>* a) {
 
 template <typename real>
 long long plane_blocks(const PlaneStep<real>& a) {
-    return ((long long)a.columns * ((a.nx + a.span - 1) / a.span) + 3) / 4;
+    return ((long long)a.columns * a.chunks + 3) / 4;
 }
 
 // The plane march of a half step: true when the grid's layout allows it.  The two terms of an axis must
@@ -801,7 +825,8 @@ bool make_plane_step(const HalfStep<real>& h, bool forward, PlaneStep<real>* out
     a.span = (long long)a.columns * h.nx < kSpanItems ? 1 : 2;
     a.by_nz = make_divider((unsigned)h.nz);
     a.by_columns = make_divider((unsigned)a.columns);
-    const long long items = (long long)a.columns * ((h.nx + a.span - 1) / a.span);
+    a.chunks = (h.nx + a.span - 1) / a.span;
+    const long long items = (long long)a.columns * a.chunks;
     if (items > 0x7ffffff0LL) return false;
     a.xcd = (int)xcd_run(plane_blocks(a));
     a.src = h.src; a.dst = h.dst; a.inverse = h.inverse;
