@@ -87,3 +87,26 @@ def test_network_equals_its_layers_one_by_one(gpu):
         assert torch.equal(a, b)
     with torch.no_grad():
         assert torch.equal(net(rho), expected)
+
+
+@pytest.mark.parametrize('ci,co,ks', [(1, 6, 1), (5, 32, 1), (31, 36, 1), (32, 64, 1), (1, 33, 3)])
+def test_narrow_layers_find_their_taps_and_round_as_torch(gpu, ci, co, ks):
+    """At most 32 values of K, split into taps and channels; bf16 values of ties, overflow, infinities and NaN."""
+    from torchfdtd_amd.surrogate import _forward, _operands, conv_shape
+    gen = torch.Generator().manual_seed(ci+co)
+    shape = (3, 5, 4, 7)
+    x, w = torch.randn((*shape, ci), generator=gen).bfloat16(), torch.randn((co, ks, ks, ks, ci), generator=gen).bfloat16()
+    b = torch.randn(co, generator=gen)
+    b[:5] = torch.tensor([math.inf, -math.inf, math.nan, 3.4e38, 1+2**-8])
+    s, out = conv_shape((*shape, ci), ci, co, ks, 1, ks // 2)
+    m, k = shape[0]*math.prod(out), ks**3*ci
+    (w16, _, parts), = _operands([s], [w.float().cuda()], [False])
+    pre, act = torch.empty((m, co), device=gpu), torch.empty((m, co), device=gpu, dtype=torch.bfloat16)
+    _forward(s, x.cuda(), w16, parts, b.cuda(), False, pre=pre, act=act)
+    expected = direct(x.double(), w.double(), b.double(), 1, ks // 2).reshape(m, co)
+    magnitude = direct(x.double().abs(), w.double().abs(), b.double().abs(), 1, ks // 2).reshape(m, co)
+    got = pre.cpu().double()
+    assert bool(((got-expected).abs() <= (k+1)*2**-24*magnitude)[:, 3:].all())
+    assert torch.equal(got[:, :2], expected[:, :2]) and bool(got[:, 2].isnan().all())
+    assert torch.equal(act.cpu().nan_to_num(7.), pre.cpu().bfloat16().nan_to_num(7.))
+    assert torch.equal(act.cpu().isnan(), pre.cpu().isnan())

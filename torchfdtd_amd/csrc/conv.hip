@@ -32,12 +32,9 @@ typedef short s8 __attribute__((ext_vector_type(8)));
 
 constexpr int BM = 64, BN = 64, BK = 32, LDK = BK + 8;   // LDS rows padded by 16 bytes
 
-// Round to nearest even (finite inputs), as torch's float -> bfloat16 conversion.
-__device__ __forceinline__ bf16_bits float_to_bf16(float f) {
-    const unsigned u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (bf16_bits)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-    return (bf16_bits)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
+// Round to nearest even, infinities and NaN kept, as torch's float -> bfloat16 conversion: one instruction on
+// gfx950 (two values at a time where the caller converts neighbours).
+__device__ __forceinline__ bf16_bits float_to_bf16(float f) { return __builtin_bit_cast(bf16_bits, (__bf16)f); }
 
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
@@ -286,8 +283,18 @@ struct GatherGemm {
     bf16_bits* act;             // forward: activation (may be null)
 };
 
+// The bias of four consecutive columns, read once per workgroup tile: behind the outputs' stores each row would
+// wait for it again.
+__device__ __forceinline__ f4 column_bias(const GatherGemm& g, int col) {
+    f4 b = f4{0.f, 0.f, 0.f, 0.f};
+    if (!g.dgrad && g.bias)
+        for (int e = 0; e < 4; ++e)
+            if (col + e < g.N) b[e] = g.bias[col + e];
+    return b;
+}
+
 // Four consecutive columns of a row to the outputs: bias, pre-activation, activation; the input gradient as it is.
-__device__ __forceinline__ void finish_columns(const GatherGemm& g, long long cell, int col, f4 v) {
+__device__ __forceinline__ void finish_columns(const GatherGemm& g, long long cell, int col, f4 v, f4 bias) {
     if (col + 3 < g.N && g.N % 4 == 0) {
         const long long o = cell * g.N + col;
         if (g.dgrad) {
@@ -295,7 +302,7 @@ __device__ __forceinline__ void finish_columns(const GatherGemm& g, long long ce
             return;
         }
         if (g.bias)
-            for (int e = 0; e < 4; ++e) v[e] += g.bias[col + e];
+            for (int e = 0; e < 4; ++e) v[e] += bias[e];
         if (g.pre) *reinterpret_cast<f4*>(g.pre + o) = v;
         bf16_bits b[4];
         for (int e = 0; e < 4; ++e) b[e] = float_to_bf16(g.activation ? gelu(v[e]) : v[e]);
@@ -311,7 +318,7 @@ __device__ __forceinline__ void finish_columns(const GatherGemm& g, long long ce
         if (col + e >= g.N) continue;
         const long long o = cell * g.N + col + e;
         float f = v[e];
-        if (!g.dgrad && g.bias) f += g.bias[col + e];
+        if (!g.dgrad && g.bias) f += bias[e];
         if (g.pre) g.pre[o] = f;
         if (g.dgrad) continue;
         const bf16_bits b = float_to_bf16(g.activation ? gelu(f) : f);
@@ -550,6 +557,9 @@ __global__ __launch_bounds__(256) void gather_gemm_kernel(const GatherGemm g) {
         }
     }
     // A lane holds four consecutive columns of one row per tile.
+    f4 bias[CT];
+#pragma unroll
+    for (int i = 0; i < CT; ++i) bias[i] = column_bias(g, col0 + wn + 16 * i + fc * 4);
 #pragma unroll
     for (int j = 0; j < RT; ++j) {
         const int row = row0 + wm + 16 * j + fr;
@@ -565,7 +575,7 @@ __global__ __launch_bounds__(256) void gather_gemm_kernel(const GatherGemm g) {
 #pragma unroll
         for (int i = 0; i < CT; ++i) {
             const int col = col0 + wn + 16 * i + fc * 4;
-            finish_columns(g, cell, col, acc[i][j]);
+            finish_columns(g, cell, col, acc[i][j], bias[i]);
         }
     }
 }
@@ -636,49 +646,69 @@ __global__ __launch_bounds__(256) void weights_kernel(const WeightsJobs jobs) {
 
 // Forward convolution with at most 32 values of K (a one-channel input): no staging pays, a wavefront takes
 // 64 rows, gathers each row's K values into the MFMA operand and keeps the weights of its columns in
-// registers.  Bound by its outputs: 524,288 rows x 32 columns, pre-activation and value in FP32: 57 us
-// against 107 for gemm_kernel and the conversion pass.
+// registers.  Bound by its vector instructions, of which the activation is nearly half: 2,097,152 rows x 32
+// columns to bf16 take 108 us (128 with a division and three comparisons per value, the bias read again behind
+// every row's stores and the rounding in integer instructions); 524,288 rows with the FP32 pre-activation took
+// 107 us in gemm_kernel and its conversion pass.
+// n / d for n, d <= 32: (n * small_reciprocal(d)) >> 10 (the excess n * (d - 1) stays below 1024).
+__host__ __device__ constexpr int small_reciprocal(int d) { return (1023 + d) / d; }
+
+struct NarrowSplit {
+    Divider by_w, by_h, by_d;
+    int per_ci, per_ks, per_ks2;    // small_reciprocal of ci, ks and ks * ks
+};
+
 template <int CT>
-__global__ __launch_bounds__(256) void narrow_forward_kernel(const GatherGemm g, int rows, Divider by_w, Divider by_h, Divider by_d) {
+__global__ __launch_bounds__(256) void narrow_forward_kernel(const GatherGemm g, int rows, const NarrowSplit split) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Conv& c = g.c;
     const int col0 = blockIdx.y * CT * 16, fr = lane & 15, fc = lane >> 4;
     bf16x8 w[CT];
+    f4 bias[CT];
 #pragma unroll
     for (int i = 0; i < CT; ++i) {
+        bias[i] = column_bias(g, col0 + 16 * i + fc * 4);
         s8 v = {0, 0, 0, 0, 0, 0, 0, 0};
         const int col = col0 + 16 * i + fr;
         if (col < g.N) v = *reinterpret_cast<const s8*>(g.weight + (long long)col * 32 + fc * 8);
         w[i] = __builtin_bit_cast(bf16x8, v);
     }
+    // A lane's 8 values of K: the tap of each (31: none, the padding of K), and its elements from the row's position.
     const int ks = c.ks, kmax = ks * ks * ks * c.ci;
-    int tz[8], ty[8], tx[8], at[8];
+    int tap[8], at[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-        const int k = fc * 8 + t, tap = k / c.ci;
-        tx[t] = k < kmax ? tap % ks - c.pad : -0x40000000;      // never inside
-        ty[t] = tap / ks % ks - c.pad;
-        tz[t] = tap / (ks * ks) - c.pad;
-        at[t] = ((tz[t] * c.hi + ty[t]) * c.wi + (tap % ks - c.pad)) * c.ci + (k - tap * c.ci);
+        const int k = fc * 8 + t, own = k * split.per_ci >> 10, z = own * split.per_ks2 >> 10, line = own * split.per_ks >> 10;
+        const int y = line - z * ks, x = own - line * ks;
+        tap[t] = k < kmax ? own : 31;
+        at[t] = (((z - c.pad) * c.hi + y - c.pad) * c.wi + x - c.pad) * c.ci + (k - own * c.ci);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int row = (blockIdx.x * 4 + wave) * 64 + 16 * j + fr;
-        const unsigned u = divide((unsigned)row, by_w), v = divide(u, by_h), nb = divide(v, by_d);
+        const unsigned u = divide((unsigned)row, split.by_w), v = divide(u, split.by_h), nb = divide(v, split.by_d);
         const int x = (row - (int)u * c.wout) * c.stride, y = (int)(u - v * c.hout) * c.stride, z = (int)(v - nb * c.dout) * c.stride;
-        const bf16_bits* const from = g.source + ((((long long)nb * c.di + z) * c.hi + y) * c.wi + x) * c.ci;
+        const int from = ((((int)nb * c.di + z) * c.hi + y) * c.wi + x) * c.ci;
+        // A bit per tap that lies inside the input.
+        unsigned inside = 0u;
+        for (int kd = 0; kd < ks; ++kd)
+            for (int kh = 0; kh < ks; ++kh) {
+                if ((unsigned)(z + kd - c.pad) >= (unsigned)c.di || (unsigned)(y + kh - c.pad) >= (unsigned)c.hi) continue;
+                for (int kw = 0; kw < ks; ++kw)
+                    if ((unsigned)(x + kw - c.pad) < (unsigned)c.wi) inside |= 1u << ((kd * ks + kh) * ks + kw);
+            }
+        if (row >= rows) inside = 0u;
         s8 taken;
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             taken[t] = 0;
-            if (row < rows && (unsigned)(x + tx[t]) < (unsigned)c.wi && (unsigned)(y + ty[t]) < (unsigned)c.hi &&
-                (unsigned)(z + tz[t]) < (unsigned)c.di)
-                taken[t] = (short)from[at[t]];
+            if (inside >> tap[t] & 1u)
+                taken[t] = *global(reinterpret_cast<const short*>(reinterpret_cast<const char*>(g.source) + (unsigned)(from + at[t]) * 2u));
         }
 #pragma unroll
         for (int i = 0; i < CT; ++i) {
             const f4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], __builtin_bit_cast(bf16x8, taken), f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            if (row < rows) finish_columns(g, row, col0 + 16 * i + fc * 4, sum);
+            if (row < rows) finish_columns(g, row, col0 + 16 * i + fc * 4, sum, bias[i]);
         }
     }
 }
@@ -688,12 +718,13 @@ bool gather_gemm(GatherGemm g, hipStream_t stream) {
     const long long inside = (long long)g.c.di * g.c.hi * g.c.wi, outside = (long long)g.c.dout * g.c.hout * g.c.wout;
     if (g.c.n * inside > 0x7fffffffLL || inside * g.channels > 0x7fffffffLL || outside * g.channels > 0x7fffffffLL) return false;
     if (g.N % 4 == 0 && (!aligned16(g.pre) || !aligned16(g.y) || (reinterpret_cast<uintptr_t>(g.act) & 7u))) return false;
-    if (!g.dgrad && g.ldw == 32 && aligned16(g.weight)) {
+    if (!g.dgrad && g.ldw == 32 && aligned16(g.weight) && g.c.n * inside * g.c.ci <= 0x7fffffffLL) {     // 32-bit byte offsets
         const int rows = g.c.n * g.c.dout * g.c.hout * g.c.wout, columns = g.N <= 32 ? 2 : 4;
         const dim3 grid((rows + 255) / 256, (g.N + columns * 16 - 1) / (columns * 16)), block(256);
-        const Divider w = make_divider((unsigned)g.c.wout), h = make_divider((unsigned)g.c.hout), d = make_divider((unsigned)g.c.dout);
-        if (columns == 2) hipLaunchKernelGGL(narrow_forward_kernel<2>, grid, block, 0, stream, g, rows, w, h, d);
-        else hipLaunchKernelGGL(narrow_forward_kernel<4>, grid, block, 0, stream, g, rows, w, h, d);
+        const NarrowSplit split{make_divider((unsigned)g.c.wout), make_divider((unsigned)g.c.hout), make_divider((unsigned)g.c.dout),
+                                small_reciprocal(g.c.ci), small_reciprocal(g.c.ks), small_reciprocal(g.c.ks * g.c.ks)};
+        if (columns == 2) hipLaunchKernelGGL(narrow_forward_kernel<2>, grid, block, 0, stream, g, rows, split);
+        else hipLaunchKernelGGL(narrow_forward_kernel<4>, grid, block, 0, stream, g, rows, split);
         return true;
     }
     if (g.channels % 8 || !aligned16(g.source) || !aligned16(g.weight) || g.ldw % 8) return false;
