@@ -7,10 +7,12 @@ Here a cohort only needs a common step count and precision: every grid keeps its
 shape, CPML layout, sources, traces and planes, and each kernel launch covers every
 grid of the cohort through a device table of per-grid descriptors.
 
-Per step (split kernels): one E launch, one H launch, one plane-DFT launch and one
-trace/counter launch for the whole cohort.  Per pair of steps (one-pass kernels):
-three tile launches (interior, z-face, boundary) for each step, plus the DFT and
-trace launches.  The step loop is captured in HIP graphs exactly as for one run.
+Per step (split kernels): one E launch, one H launch (which steps the counter on) and
+one plane-DFT launch for the whole cohort, and one for its traces if it has any.  A
+cohort larger than the memory-side cache takes a block of steps in groups of grids
+that stay in it.  Per pair of steps (one-pass kernels): three tile launches (interior,
+z-face, boundary) for each step, plus the DFT and trace launches.  The step loop is
+captured in HIP graphs exactly as for one run.
 
 Entry points mirror the reference: run_tensor_batch (tensor_batch.py:44-113),
 plan_grouped_batch / run_grouped_batch (grouped_batch.py:80-146) and
@@ -42,6 +44,15 @@ from .models import Project
 from .diagnostics import StateNorms
 from .run_control import RunMonitor, check_count
 from .solver import ENGINE_LOCK, DisplaySlice, Result, Stepper, pack_table as _pack, run_signature, run_summary
+
+
+# A split cohort whose state (fields, 1/eps, CPML memory) exceeds WHOLE_BYTES no longer stays in the 256 MB
+# memory-side cache from step to step; it then takes a block of steps in groups of at most GROUP_BYTES.  Uneven
+# grids of about 22 MB, 128 steps with their planes, whole against grouped: 8 grids 10.1 / 12.1 ms (smaller
+# launches fill the chip less well), 11 grids 15.4 / 16.2, 12 grids 19.1 / 17.3, 16 grids 30.2 / 24.4, 20 grids
+# 37.5 / 31.7, 40 grids 74.7 / 65.6; 28 grids in groups of 160 MB 44.5, of 213 MB 49.2.
+WHOLE_BYTES = 232 << 20
+GROUP_BYTES = 208 << 20
 
 
 @dataclass
@@ -223,6 +234,7 @@ class Cohort:
         self.planes = self._pack_planes([run.plane_table[k] for run in self.runs for k in range(len(run.planes))])
         self.planes_s = self._pack_planes([self._shadowed(run.plane_table[k]) for run in self.runs for k in range(len(run.planes))])
         self.observe_s = self._shadowed(self.observe)
+        self.groups = [] if one_pass else self._resident_groups()
         if one_pass:
             self.march = []
             for k in range(2):
@@ -232,6 +244,32 @@ class Cohort:
             self.trace_table_b = self._cohort_traces([run.trace_table_b for run in self.runs])
             self.observe_b = self._observe(self.trace_table_b)
             self.planes_b = self._pack_planes([run.plane_table_b[k] for run in self.runs for k in range(len(run.planes))])
+
+    def _resident_groups(self):
+        """Runs of consecutive grids whose state stays in the memory-side cache, each with tables of its own
+        ([] where the whole cohort fits, or has traces, whose rows hold every grid of the cohort)."""
+        if self.observe.count:
+            return []
+        sizes = [sum(t.numel()*t.element_size() for t in (g.E, g.H, g.inverse_permittivity, *g.psi_buffers.values()))
+                 for g in self.grids]
+        total = sum(sizes)
+        if total <= WHOLE_BYTES:
+            return []
+        count = -(-total//GROUP_BYTES)
+        # Groups of near-equal size: a grid belongs to the one that its middle lies in.
+        middles = np.cumsum(sizes)-np.array(sizes)/2
+        members = [part for k in range(count) if (part := np.flatnonzero((middles*count/total).astype(int) == k).tolist())]
+        groups = []
+        for part in members:
+            runs = [self.runs[i] for i in part]
+            tables = []
+            for descriptors in ([run.e_step for run in runs], [self._shadowed(run.h_step) for run in runs]):
+                table, prefix, host = _pack(lambda n: self.lib.tfdtd_batch_table_bytes(n, self.dtype), self.lib.tfdtd_batch_pack,
+                                            descriptors, 1, self.counter.device)
+                tables += [table, prefix, int(host[0, len(runs)])]
+            planes = self._pack_planes([self._shadowed(run.plane_table[k]) for run in runs for k in range(len(run.planes))])
+            groups.append((tables, len(runs), planes))
+        return groups
 
     def _cohort_traces(self, tables):
         tables = [t for t in tables if t.numel()]
@@ -327,6 +365,23 @@ class Cohort:
         if self.observe_s.count:
             N.check(self.lib.tfdtd_record_traces(ctypes.byref(self.observe_s), stream), 'tfdtd_record_traces')
 
+    def step_block(self, count):
+        """`count` steps of every grid with the split kernels.  A cohort larger than the memory-side cache advances
+        its resident groups one after the other, each by all the steps, the counter set back in between."""
+        if not self.groups or count < 2:
+            for _ in range(count):
+                self.step()
+            return
+        stream = N.stream_handle()
+        for k, ((e, e_prefix, e_blocks, h, h_prefix, h_blocks), grids, planes) in enumerate(self.groups):
+            if k:
+                self.counter.sub_(count)
+            for _ in range(count):
+                N.check(self.lib.tfdtd_batch_step(e.data_ptr(), e_prefix.data_ptr(), e_blocks, h.data_ptr(), h_prefix.data_ptr(),
+                                                  h_blocks, grids, self.dtype, self.counter.data_ptr(), self.shadow.data_ptr(),
+                                                  stream), 'tfdtd_batch_step')
+                self._planes_update(planes, stream)
+
     def step_pair(self):
         """Two steps with the one-pass kernels: grid buffers -> second set -> grid buffers."""
         self.refresh_materials()
@@ -346,12 +401,12 @@ class Cohort:
             if count % 2:
                 self.step()
         else:
-            for _ in range(count):
-                self.step()
+            self.step_block(count)
 
     def graphs(self, width=1):
         return StepGraphs(self.step, self.states(), self.steps, width, pair=self.step_pair if self.one_pass else None,
-                          prepare=self.refresh_materials if self.one_pass else None)
+                          prepare=self.refresh_materials if self.one_pass else None,
+                          block=None if self.one_pass else self.step_block)
 
     def traces_of(self, i, completed):
         return self.traces[:completed, int(self.trace_offsets[i]):int(self.trace_offsets[i+1])].cpu().numpy().copy()

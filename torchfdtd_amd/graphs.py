@@ -39,9 +39,10 @@ class StepGraphs:
     before every replay (e.g. Stepper.refresh_materials, which follows permittivity changes).
     """
 
-    def __init__(self, step, states, steps, width=1, warmup=3, pair=None, prepare=None, quad=None, widths=()):
+    def __init__(self, step, states, steps, width=1, warmup=3, pair=None, prepare=None, quad=None, widths=(), block=None):
         """`widths`: further step counts to capture a graph of each (<= 64), for callers that advance
-        by counts other than 1 and `width` (a checkpoint segment and its remainder)."""
+        by counts other than 1 and `width` (a checkpoint segment and its remainder).  `block(n)`, when given,
+        takes n steps at once in place of n calls of `step`."""
         self.prepare = prepare
         self.width = min(validate_graph_steps(width), steps)
         states = list(states)
@@ -54,6 +55,8 @@ class StepGraphs:
                 pair()      # the pair's first launches happen outside capture too
             if quad is not None and steps >= 4:
                 quad()
+            if block is not None and steps >= 2:
+                block(2)
             for value in states:
                 value.zero_()
         torch.cuda.current_stream().wait_stream(stream)
@@ -83,8 +86,11 @@ class StepGraphs:
                         step()
                         made['split'] = 1
                 else:
-                    for _ in range(count):
-                        step()
+                    if block is not None:
+                        block(count)
+                    else:
+                        for _ in range(count):
+                            step()
                     made['split'] = count
                 graph.capture_end()
             self.composition[count] = made
