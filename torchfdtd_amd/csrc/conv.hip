@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void gelu_backward_kernel(const float* dy, con
 // output positions (forward) or, for the input gradient, the input positions of one parity class of a
 // strided layer: rows of one class see the same taps, so no tap is multiplied that the stride rules out.
 //
-// A workgroup (4 waves) computes BM rows x BN columns over K in stages of 64: source rows and weight rows
+// A workgroup (4 waves, 8 at 128 x 128) computes BM rows x BN columns over K in stages of 64: source rows and weight rows
 // go from global memory straight into LDS (16 bytes a lane, no registers), `Depth` - 1 stages ahead of the
 // stage being multiplied.  A lane keeps its rows' addresses and a bit per tap (inside or padding) for the
 // whole loop, so a stage costs it one offset and a select; padding reads a chunk of zeros.  A row's 16-byte
@@ -253,10 +253,12 @@ __global__ __launch_bounds__(256) void gelu_backward_kernel(const float* dy, con
 // so results are equal bit for bit; a tap that is padding for every row of the workgroup is skipped when the
 // weights are finite (it would add zeros).
 //
-// 64x32x32x16 positions, 64 -> 128 channels, 3x3x3 (0.46 TFLOP): forward 2.72 -> 0.97 ms (480 TFLOP/s), input
-// gradient 3.5 -> 0.75 ms (620).  gemm_kernel gathered through registers with a division chain per chunk and
-// two barriers per 32 of K; here the staged bytes bound it (32 KB a stage and workgroup, 27 taps of x through
-// L2: about 7 TB/s), the matrix cores are busy a fifth to a quarter of the time.
+// 64x32x32x16 positions, 64 -> 128 channels, 3x3x3 (0.46 TFLOP): forward 2.72 -> 0.88 ms (530 TFLOP/s), input
+// gradient 3.5 -> 0.76 ms (610).  gemm_kernel gathered through registers with a division chain per chunk and
+// two barriers per 32 of K.  The forward layer's matrix instructions take a quarter of its cycles and its epilogue
+// (GELU, two FP32 outputs) a fifth; the rest is the latency of the stages, which is why eight waves per tile
+// beat four (0.95 ms with the same stages) and why fewer, larger stages do not help (256 x 128 tiles, two or three
+// stages deep: 0.99 ms; 128 x 128 three deep, one workgroup per CU: 1.5 ms).
 typedef __attribute__((address_space(3))) void lds_void;
 
 __device__ const uint4 kZeroChunk = {0u, 0u, 0u, 0u};
@@ -375,8 +377,10 @@ struct Pieces {
 // `Whole`: the channels are a multiple of 32, so a piece of 32 has one tap; otherwise (a multiple of 8) each
 // 16-byte chunk finds its own.
 template <int BM, int BN, int WM, int WN, int Depth, bool Whole>
-__global__ __launch_bounds__(256) void gather_gemm_kernel(const GatherGemm g) {
-    constexpr int XI = BM / 32, WI = BN / 32;          // staging instructions per wave
+__global__ __launch_bounds__(BM / WM * (BN / WN) * 64) void gather_gemm_kernel(const GatherGemm g) {
+    constexpr int Waves = BM / WM * (BN / WN);
+    constexpr int XI = BM / (8 * Waves), WI = BN / (8 * Waves);         // staging instructions per wave
+    static_assert(XI * 8 * Waves == BM && WI * 8 * Waves == BN, "whole staging instructions");
     constexpr int RT = WM / 16, CT = WN / 16;          // 16-row and 16-column tiles per wave
     constexpr int Stage = (BM + BN) * 64;
     __shared__ __attribute__((aligned(16))) bf16_bits s0[Stage];
@@ -431,7 +435,7 @@ __global__ __launch_bounds__(256) void gather_gemm_kernel(const GatherGemm g) {
     unsigned todo = taps == 32 ? ~0u : (1u << taps) - 1u;
     if (Whole && g.nonfinite) {
         int bad = 0;
-        for (int i = tid; i < g.parts; i += 256) bad |= g.nonfinite[i];
+        for (int i = tid; i < g.parts; i += 64 * Waves) bad |= g.nonfinite[i];
         atomicOr(&s_mask, any);
         if (bad) s_bad = 1u;
         __syncthreads();
@@ -458,41 +462,63 @@ __global__ __launch_bounds__(256) void gather_gemm_kernel(const GatherGemm g) {
         }
     int staged = 0;
     const bf16_bits* const zero = reinterpret_cast<const bf16_bits*>(&kZeroChunk);
+    // Whole: a lane's chunk places of its rows and weight rows are fixed, so a stage adds one offset per half to
+    // pointers formed here.  Weight rows past the last repeat it and K past the last piece repeats the first:
+    // neither is used.
+    const bf16_bits* weight_at[WI];
+    if (Whole) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) row_at[i] += (chunk_of[i & 1] & 3) * 8;
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            const int r = (wave * WI + i) * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7);
+            weight_at[i] = g.weight + (long long)min(col0 + r, g.N - 1) * g.ldw + (chunk & 3) * 8;
+        }
+    }
+    const int odd_weights = wave * WI & 1;
+    const bool upper[2] = {(chunk_of[0] >> 2) != 0, (chunk_of[1] >> 2) != 0};       // which half of a stage, by parity
+    const bool upper_weights[2] = {(((lane & 7) ^ (((lane >> 4) + 4 * odd_weights) & 7)) >> 2) != 0,
+                                   (((lane & 7) ^ (((lane >> 4) + 4 * (odd_weights ^ 1)) & 7)) >> 2) != 0};
     auto stage = [&](bf16_bits* into) {
-        int offset[2] = {0, 0};
-        unsigned bit[2] = {0u, 0u};
-        int k[2] = {0, 0};
+        bf16_bits* const weights = into + BM * 64;
         if (Whole) {
+            int offset[2], k[2];
+            unsigned bit[2];
             for (int h = 0; h < 2; ++h) {
-                if (at.more) {
-                    offset[h] = tap_offset(at.tap) + at.c;
-                    bit[h] = 1u << at.tap;
-                    k[h] = at.tap * C + at.c;
-                } else {
-                    k[h] = -1;
-                }
+                offset[h] = at.more ? tap_offset(at.tap) + at.c : 0;
+                bit[h] = at.more ? 1u << at.tap : 0u;
+                k[h] = at.more ? at.tap * C + at.c : 0;
                 at.next(C);
             }
+            int mine[2], ours[2];
+            unsigned need[2];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                mine[v] = upper[v] ? offset[1] : offset[0];
+                need[v] = upper[v] ? bit[1] : bit[0];
+                ours[v] = upper_weights[v] ? k[1] : k[0];
+            }
+#pragma unroll
+            for (int i = 0; i < XI; ++i)
+                chunk_to_lds(row_taps[i] & need[i & 1] ? row_at[i] + mine[i & 1] : zero, into + (wave * XI + i) * 512);
+#pragma unroll
+            for (int i = 0; i < WI; ++i) chunk_to_lds(weight_at[i] + ours[i & 1], weights + (wave * WI + i) * 512);
+            ++staged;
+            return;
         }
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
-            const int chunk = chunk_of[i & 1], half = chunk >> 2, within = (chunk & 3) * 8;
             const bf16_bits* from = zero;
-            if (Whole) {
-                if (row_taps[i] & (half ? bit[1] : bit[0])) from = row_at[i] + (half ? offset[1] : offset[0]) + within;
-            } else if (own_tap[i & 1] < taps && (row_taps[i] >> own_tap[i & 1] & 1u)) {
+            if (own_tap[i & 1] < taps && (row_taps[i] >> own_tap[i & 1] & 1u))
                 from = row_at[i] + tap_offset(own_tap[i & 1]) + own_c[i & 1];
-            }
             chunk_to_lds(from, into + (wave * XI + i) * 512);
         }
-        bf16_bits* const weights = into + BM * 64;
 #pragma unroll
         for (int i = 0; i < WI; ++i) {
             const int r = (wave * WI + i) * 8 + (lane >> 3);
-            const int chunk = (lane & 7) ^ ((r >> 1) & 7), half = chunk >> 2, within = (chunk & 3) * 8;
-            const int kk = Whole ? (half ? k[1] : k[0]) : staged * 64 + half * 32;
+            const int chunk = (lane & 7) ^ ((r >> 1) & 7), kk = staged * 64 + chunk * 8;
             const bf16_bits* from = zero;
-            if (col0 + r < g.N && kk >= 0 && kk + within < g.ldw) from = g.weight + (long long)(col0 + r) * g.ldw + kk + within;
+            if (col0 + r < g.N && kk < g.ldw) from = g.weight + (long long)(col0 + r) * g.ldw + kk;
             chunk_to_lds(from, weights + (wave * WI + i) * 512);
         }
         ++staged;
@@ -588,7 +614,7 @@ constexpr unsigned kRowRun = 64;
 template <int BM, int BN, int WM, int WN, int Depth>
 void launch_gather(GatherGemm g, int classes, hipStream_t stream) {
     g.run = kRowRun;
-    const dim3 grid((g.rows_max + BM - 1) / BM, (g.N + BN - 1) / BN, classes), block(256);
+    const dim3 grid((g.rows_max + BM - 1) / BM, (g.N + BN - 1) / BN, classes), block(BM / WM * (BN / WN) * 64);
     if (g.channels % 32 == 0) hipLaunchKernelGGL((gather_gemm_kernel<BM, BN, WM, WN, Depth, true>), grid, block, 0, stream, g);
     else hipLaunchKernelGGL((gather_gemm_kernel<BM, BN, WM, WN, Depth, false>), grid, block, 0, stream, g);
 }
@@ -743,7 +769,7 @@ bool gather_gemm(GatherGemm g, hipStream_t stream) {
         if (blocks(128, 32) >= 512) launch_gather<128, 32, 32, 32, 2>(g, classes, stream);
         else launch_gather<32, 32, 16, 16, 3>(g, classes, stream);
     } else if (g.N > 64 && blocks(128, 128) >= 512) {
-        launch_gather<128, 128, 64, 64, 2>(g, classes, stream);
+        launch_gather<128, 128, 64, 32, 2>(g, classes, stream);     // 64 columns: four waves 0.76 ms, eight 0.83
     } else if (blocks(128, 64) >= 512) {
         launch_gather<128, 64, 64, 32, 2>(g, classes, stream);
     } else if (blocks(64, 64) >= 512) {
