@@ -110,3 +110,22 @@ def test_narrow_layers_find_their_taps_and_round_as_torch(gpu, ci, co, ks):
     assert torch.equal(got[:, :2], expected[:, :2]) and bool(got[:, 2].isnan().all())
     assert torch.equal(act.cpu().nan_to_num(7.), pre.cpu().bfloat16().nan_to_num(7.))
     assert torch.equal(act.cpu().isnan(), pre.cpu().isnan())
+
+
+@pytest.mark.parametrize('shape,ci,co,ks,stride,pad', [((9, 2, 3, 2), 64, 72, 3, 1, 1), ((40, 3, 2, 5), 8, 64, 3, 2, 1), ((2, 17, 13, 11), 32, 32, 3, 2, 0),
+                                                       ((70, 1, 2, 1), 16, 136, 3, 1, 1), ((3, 1, 1, 65), 40, 24, 1, 2, 0), ((1, 66, 1, 1), 24, 64, 3, 1, 1),
+                                                       ((2, 64, 4, 3), 8, 32, 3, 1, 0), ((5, 3, 64, 3), 16, 128, 3, 1, 1)])
+def test_weight_gradient_walks_every_position(gpu, shape, ci, co, ks, stride, pad):
+    """Positions move on by 64 with carries: axes of 1 to 66, several samples a stage, ends inside a stage, splits."""
+    from torchfdtd_amd.surrogate import _layer_gradients, conv_shape
+    s, out = conv_shape((*shape, ci), ci, co, ks, stride, pad)
+    gen = torch.Generator().manual_seed(ci+co)
+    m, k = shape[0]*math.prod(out), ks**3*ci
+    x, dy = torch.randn((*shape, ci), generator=gen).bfloat16(), torch.randn((m, co), generator=gen).bfloat16()
+    _, dw, _ = _layer_gradients(s, dy.float().cuda(), torch.zeros((m, co), device=gpu), 0, x.cuda())
+
+    def direct_gradient(a, b):
+        w = torch.zeros((co, ks, ks, ks, ci), dtype=torch.float64, requires_grad=True)
+        return torch.autograd.grad(direct(a, w, None, stride, pad).reshape(m, co), w, b)[0]
+    want, size = direct_gradient(x.double(), dy.double()), direct_gradient(x.double().abs(), dy.double().abs())
+    assert bool(((dw.cpu()[:, :k].reshape(want.shape).double()-want).abs() <= (m+1)*2**-24*size).all())

@@ -787,8 +787,9 @@ bool gather_gemm(GatherGemm g, hipStream_t stream) {
 // chunks of x) and each MFMA operand is read transposed (ds_read_b64_tr_b16: 4 positions x 16 columns a
 // group of 16 lanes) -- no transposed copy of dY in memory.  Chunks lie at chunk ^ swizzle(row), which spreads
 // the 16 rows of a transposed read over the banks.  The positions are split over blockIdx.z; each split
-// writes its partial sums, which split_sum_kernel adds.  64x32x32x16 positions, 64 -> 128 channels: 0.97 ms
-// (480 TFLOP/s), against 3.1 ms and 1.2 ms for the transposed copy of dY.
+// writes its partial sums, which split_sum_kernel adds.  64x32x32x16 positions, 64 -> 128 channels: 0.75 ms
+// (620 TFLOP/s), against 3.1 ms and 1.2 ms for the transposed copy of dY; 0.99 ms while each chunk's position
+// was found by division in every stage, 0.78 ms with four wavefronts a tile.
 
 struct WeightGrad {
     Conv c;
@@ -797,6 +798,10 @@ struct WeightGrad {
     float* partial;             // [split][co][kp]
     int m_total, per_split;
     Divider by_w, by_h, by_d;
+    // 64 output positions on, without carries: input cells along x, y and z, and chunks of 8 channels in all; a
+    // carry of an axis moves `carry` chunks more.
+    int step[3];
+    unsigned on, carry[3];
 };
 
 template <int Chunks>
@@ -820,11 +825,12 @@ __device__ __forceinline__ bf16x8 transposed(const bf16_bits* stage, int row, in
     return __builtin_bit_cast(bf16x8, both);
 }
 
-template <int BC, int BK>
-__global__ __launch_bounds__(256, 2) void weight_grad_kernel(const WeightGrad g) {
+template <int BC, int BK, int Waves>
+__global__ __launch_bounds__(64 * Waves, Waves / 2) void weight_grad_kernel(const WeightGrad g) {
     constexpr int DC = BC / 8, XC = BK / 8;                     // 16-byte chunks of a row
-    constexpr int DI = BC / 32, XI = BK / 32;                   // staging instructions per wave
-    constexpr int WC = BC / 2, WK = BK / 2, CT = WC / 16, KT = WK / 16;
+    constexpr int DI = DC / Waves, XI = XC / Waves;             // staging instructions per wave
+    constexpr int WC = BC / 2, WK = BK / (Waves / 2), CT = WC / 16, KT = WK / 16;
+    static_assert(DI * Waves == DC && XI * Waves == XC, "whole staging instructions");
     constexpr int Stage = 64 * (BC + BK);
     __shared__ __attribute__((aligned(16))) bf16_bits s0[Stage];
     __shared__ __attribute__((aligned(16))) bf16_bits s1[Stage];
@@ -834,38 +840,61 @@ __global__ __launch_bounds__(256, 2) void weight_grad_kernel(const WeightGrad g)
     const int co0 = blockIdx.x * BC, k0 = blockIdx.y * BK;
     const int begin = blockIdx.z * g.per_split, end = min(g.m_total, begin + g.per_split);
     const bf16_bits* const zero = reinterpret_cast<const bf16_bits*>(&kZeroChunk);
-    // The x chunk of each staging instruction: its tap and channel stay for the whole loop.
-    int tap_z[XI], tap_y[XI], tap_x[XI], channel[XI];
-    const int ks = c.ks, kmax = ks * ks * ks * c.ci;
+    // The x chunk of each staging instruction: its tap and channel stay for the whole loop, its input cell moves on
+    // by 64 output positions a stage, axis by axis with carries -- finding it anew took three divisions and
+    // 64-bit products per chunk, more than the matrix instructions.  `at` counts chunks of 8 channels.
+    int tx[XI], ty[XI], tz[XI], end_x[XI], end_y[XI], end_z[XI], row_of[XI];
+    unsigned at[XI];
+    const int ks = c.ks, kmax = ks * ks * ks * c.ci, wide = c.wout * c.stride, high = c.hout * c.stride, deep = c.dout * c.stride;
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
         const int row = (wave * XI + i) * (64 / XC) + lane / XC;
         const int k = k0 + ((lane % XC) ^ row_swizzle<XC>(row)) * 8;
-        const int tap = k / c.ci;
-        channel[i] = k < kmax ? k - tap * c.ci : -1;
-        tap_x[i] = tap % ks - c.pad;
-        tap_y[i] = tap / ks % ks - c.pad;
-        tap_z[i] = tap / (ks * ks) - c.pad;
+        const int tap = k / c.ci, kx = tap % ks - c.pad, ky = tap / ks % ks - c.pad, kz = tap / (ks * ks) - c.pad;
+        row_of[i] = k < kmax ? row : 0x7fffffff;
+        const unsigned m = (unsigned)(begin + row), u = divide(m, g.by_w), v = divide(u, g.by_h), nb = divide(v, g.by_d);
+        tx[i] = (int)(m - u * c.wout) * c.stride + kx;
+        ty[i] = (int)(u - v * c.hout) * c.stride + ky;
+        tz[i] = (int)(v - nb * c.dout) * c.stride + kz;
+        end_x[i] = wide + kx;
+        end_y[i] = high + ky;
+        end_z[i] = deep + kz;
+        at[i] = (unsigned)((((((long long)nb * c.di + tz[i]) * c.hi + ty[i]) * c.wi + tx[i]) * c.ci + (k - tap * c.ci)) >> 3);
     }
+    const bf16_bits* dy_at[DI];
+#pragma unroll
+    for (int i = 0; i < DI; ++i) {
+        const int row = (wave * DI + i) * (64 / DC) + lane / DC;
+        dy_at[i] = g.dy + (long long)(begin + row) * c.co + co0 + ((lane % DC) ^ row_swizzle<DC>(row)) * 8;
+    }
+    const long long dy_on = 64LL * c.co;
     auto stage = [&](bf16_bits* into, int m0) {
+        const int left = end - m0;
 #pragma unroll
         for (int i = 0; i < DI; ++i) {
-            const int row = (wave * DI + i) * (64 / DC) + lane / DC;
-            const int col = co0 + ((lane % DC) ^ row_swizzle<DC>(row)) * 8, m = m0 + row;
-            const bf16_bits* from = m < end && col < c.co ? g.dy + (long long)m * c.co + col : zero;
-            chunk_to_lds(from, into + (wave * DI + i) * 512);
+            const int row = (wave * DI + i) * (64 / DC) + lane / DC, col = co0 + ((lane % DC) ^ row_swizzle<DC>(row)) * 8;
+            chunk_to_lds(row < left && col < c.co ? dy_at[i] : zero, into + (wave * DI + i) * 512);
+            dy_at[i] += dy_on;
         }
         bf16_bits* const xs = into + 64 * BC;
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
-            const int m = m0 + (wave * XI + i) * (64 / XC) + lane / XC;
-            const unsigned u = divide((unsigned)m, g.by_w), v = divide(u, g.by_h), nb = divide(v, g.by_d);
-            const int x = (m - (int)u * c.wout) * c.stride + tap_x[i], y = (int)(u - v * c.hout) * c.stride + tap_y[i];
-            const int z = (int)(v - nb * c.dout) * c.stride + tap_z[i];
-            const bf16_bits* from = zero;
-            if (m < end && channel[i] >= 0 && (unsigned)x < (unsigned)c.wi && (unsigned)y < (unsigned)c.hi && (unsigned)z < (unsigned)c.di)
-                from = g.x + ((((long long)nb * c.di + z) * c.hi + y) * c.wi + x) * c.ci + channel[i];
-            chunk_to_lds(from, xs + (wave * XI + i) * 512);
+            const bool inside = (row_of[i] < left) & ((unsigned)tx[i] < (unsigned)c.wi) & ((unsigned)ty[i] < (unsigned)c.hi) &
+                                ((unsigned)tz[i] < (unsigned)c.di);
+            chunk_to_lds(inside ? g.x + (long long)at[i] * 8 : zero, xs + (wave * XI + i) * 512);
+            at[i] += g.on;
+            tx[i] += g.step[0];
+            const bool cx = tx[i] >= end_x[i];
+            tx[i] -= cx ? wide : 0;
+            at[i] += cx ? g.carry[0] : 0u;
+            ty[i] += cx ? g.step[1] + c.stride : g.step[1];
+            const bool cy = ty[i] >= end_y[i];
+            ty[i] -= cy ? high : 0;
+            at[i] += cy ? g.carry[1] : 0u;
+            tz[i] += cy ? g.step[2] + c.stride : g.step[2];
+            const bool cz = tz[i] >= end_z[i];
+            tz[i] -= cz ? deep : 0;
+            at[i] += cz ? g.carry[2] : 0u;
         }
     };
     const int wc = (wave & 1) * WC, wk = (wave >> 1) * WK;
@@ -991,7 +1020,7 @@ WeightGradShape weight_grad_shape(const tfdtd_conv& d, const Conv& c) {
         s.bc = kNarrowColumns; s.bk = 32;
         tiles = (d.co + s.bc - 1) / s.bc;
         least = 256;
-    } else if (d.ci % 8 == 0 && d.co % 8 == 0) {
+    } else if (d.ci % 8 == 0 && d.co % 8 == 0 && (long long)d.n * d.di * d.hi * d.wi <= 0xffffffffLL / (d.ci / 8)) {
         s.bc = d.co <= 32 ? 32 : d.co <= 64 ? 64 : 128;
         s.bk = 128;
         tiles = (long long)((d.co + s.bc - 1) / s.bc) * ((d.kp + s.bk - 1) / s.bk);
@@ -1262,13 +1291,20 @@ int tfdtd_conv_wgrad_rows(const tfdtd_conv* d, const void* dy, const void* x, fl
     g.by_w = make_divider((unsigned)g.c.wout);
     g.by_h = make_divider((unsigned)g.c.hout);
     g.by_d = make_divider((unsigned)g.c.dout);
+    const int x64 = 64 % g.c.wout, u64 = 64 / g.c.wout, y64 = u64 % g.c.hout, v64 = u64 / g.c.hout, z64 = v64 % g.c.dout;
+    const long long chunk = d->ci / 8, line = chunk * d->wi, page = line * d->hi;
+    g.step[0] = x64 * d->stride; g.step[1] = y64 * d->stride; g.step[2] = z64 * d->stride;
+    g.on = (unsigned)(g.step[0] * chunk + g.step[1] * line + g.step[2] * page + v64 / g.c.dout * (page * d->di));
+    g.carry[0] = (unsigned)(d->stride * (line - g.c.wout * chunk));
+    g.carry[1] = (unsigned)(d->stride * (page - g.c.hout * line));
+    g.carry[2] = (unsigned)(page * d->di - (long long)d->stride * g.c.dout * page);
     const int used = (g.m_total + g.per_split - 1) / g.per_split;
-    const dim3 grid((d->co + shape.bc - 1) / shape.bc, (d->kp + shape.bk - 1) / shape.bk, used), block(256);
+    const dim3 grid((d->co + shape.bc - 1) / shape.bc, (d->kp + shape.bk - 1) / shape.bk, used), block(256), wide(512);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (d->kp == 32) hipLaunchKernelGGL(weight_grad_narrow_kernel, grid, block, 0, s, g);
-    else if (shape.bc == 32) hipLaunchKernelGGL((weight_grad_kernel<32, 128>), grid, block, 0, s, g);
-    else if (shape.bc == 64) hipLaunchKernelGGL((weight_grad_kernel<64, 128>), grid, block, 0, s, g);
-    else hipLaunchKernelGGL((weight_grad_kernel<128, 128>), grid, block, 0, s, g);
+    else if (shape.bc == 32) hipLaunchKernelGGL((weight_grad_kernel<32, 128, 4>), grid, block, 0, s, g);
+    else if (shape.bc == 64) hipLaunchKernelGGL((weight_grad_kernel<64, 128, 8>), grid, wide, 0, s, g);
+    else hipLaunchKernelGGL((weight_grad_kernel<128, 128, 8>), grid, wide, 0, s, g);
     status = tfdtd_check_launch("conv wgrad");
     if (status) return status;
     const long long count = (long long)d->co * d->kp;
