@@ -253,6 +253,17 @@ int tfdtd_step_observed(const tfdtd_half_step* e_step, const tfdtd_half_step* h_
                         int32_t plane_count, const tfdtd_observe* observe, const tfdtd_trace_cell* cells, int64_t* shadow,
                         void* stream);
 
+/* `n_steps` (two or more) whole steps of one grid of one z plane, several to a launch, with its traces and counter: the
+ * state ends in the grid's own buffers by way of `second`, a set of the same sizes whose contents do not matter.
+ * Results are those of n_steps calls of tfdtd_step_observed.  TFDTD_EUNSUPPORTED where the grid has more planes, the
+ * half steps do not take the plane march, or the traces are not given by `cells`; n_steps 0 only asks that. */
+typedef struct tfdtd_flat_buffers {
+    void *e, *h, *psi_e, *psi_h;
+} tfdtd_flat_buffers;
+
+int tfdtd_flat_steps(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_observe* observe,
+                     const tfdtd_trace_cell* cells, const tfdtd_flat_buffers* second, int64_t* shadow, int32_t n_steps, void* stream);
+
 /* The traces at step *observe->counter (a shadow, after a step), without advancing it. */
 int tfdtd_record_traces(const tfdtd_observe* observe, void* stream);
 

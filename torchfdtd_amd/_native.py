@@ -92,6 +92,10 @@ class TraceCell(ctypes.Structure):
     _fields_ = [('element', i64), ('magnetic', i32), ('reserved', i32)]
 
 
+class FlatBuffers(ctypes.Structure):
+    _fields_ = [('e', vp), ('h', vp), ('psi_e', vp), ('psi_h', vp)]
+
+
 class Plane(ctypes.Structure):
     _fields_ = [('dtype', i32), ('spectral', i32), ('points', i64), ('frequencies', i32),
                 ('components', i32), ('electric', i32), ('corners', i32), ('time_downsample', i32),
@@ -182,6 +186,8 @@ PROTOTYPES = {
     'tfdtd_record_traces': (i32, [ctypes.POINTER(Observe), vp]),
     'tfdtd_step_observed': (i32, [ctypes.POINTER(HalfStep), ctypes.POINTER(HalfStep), ctypes.POINTER(Plane), i32,
                                   ctypes.POINTER(Observe), ctypes.POINTER(TraceCell), vp, vp]),
+    'tfdtd_flat_steps': (i32, [ctypes.POINTER(HalfStep), ctypes.POINTER(HalfStep), ctypes.POINTER(Observe), ctypes.POINTER(TraceCell),
+                               ctypes.POINTER(FlatBuffers), vp, i32, vp]),
     'tfdtd_batch_march_bytes': (ctypes.c_size_t, [i32, i32]),
     'tfdtd_batch_march_pack': (i32, [ctypes.POINTER(March), i32, vp, ctypes.c_size_t, ctypes.POINTER(i32)]),
     'tfdtd_batch_march': (i32, [vp, vp, i32, i32, i32, i32, ctypes.POINTER(i32), vp]),

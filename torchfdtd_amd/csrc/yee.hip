@@ -428,6 +428,207 @@ __global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void plane_half_ste
     carry_counter(a.counter, a.counter_to, a.counter_add);
 }
 
+// ---------------------------------------------------------------- several steps of a flat grid in one launch
+//
+// A grid of one z plane with few cells is bound by its launches: two of 3 us a step, whatever its cells.  A workgroup here loads a 32 x 32 patch of cells, a lane each, with their CPML memory and
+// coefficients, takes `steps` steps with the fields exchanged through LDS, and stores the cells that are right:
+// a step spoils one more row on each side, so the patch owns its inner (32 - 2 steps)^2 cells and its
+// neighbours compute the rest again.  Fields and memory go from one buffer set to the other (neighbours still read
+// the old state).  Every cell's arithmetic is the half steps' in their order, so results are equal bit for bit.
+//
+// us per step in a graph, half steps and patches: 160x120 6.2 -> 1.34 (FP64 6.3 -> 1.82), 256x256 5.6 -> 1.4, 400x400
+// 6.8 -> 2.4, 800x800 11.4 -> 5.5 (FP64 17.5 -> 10.2), 1500x1500 27.6 -> 14, 3000x3000 85 -> 48 (FP64 274 -> 109).  A small
+// grid is bound by one patch's chain (two barriers and two rounds through LDS a step, its load and store), a large
+// one by the cells computed twice.
+constexpr int kFlatTile = 32, kFlatSteps = 8;
+
+// Steps per launch.  More steps share the load, the store and the launch, but own fewer cells of the patch (64% at
+// 3, 56% at 4, 39% at 6, 25% at 8).  8 while all patches run at once, two to a CU (256x256: 1.41 us a step, 1.63 with
+// 6); 6 up to four such rounds (400x400: 2.43, 2.69 with 8 and 2.74 with 4; 800x800: 5.5, 6.4 and 5.9); 4 beyond (1500x1500:
+// 14.0, 14.8 with 6 and 19.0 with 2; 3000x3000: 48, 55 and 69).
+inline long long flat_tiles(int nx, int ny, int steps) {
+    const int own = kFlatTile - 2 * steps;
+    return (long long)((nx + own - 1) / own) * ((ny + own - 1) / own);
+}
+
+inline int flat_depth(int nx, int ny) { return flat_tiles(nx, ny, kFlatSteps) <= 512 ? kFlatSteps : flat_tiles(nx, ny, 6) <= 2048 ? 6 : 4; }
+
+template <typename real>
+struct FlatSet {            // one buffer set: fields and each family's CPML memory
+    real *e, *h, *psi_e, *psi_h;
+};
+
+template <typename real>
+struct FlatPass {
+    PlaneStep<real> e, h;
+    FlatSet<real> in, out;
+    int steps, tiles_y;
+    const long long* counter;
+    long long* counter_to;  // takes the counter after the steps
+};
+
+// A cell's CPML rows of one family: the memory of the two terms of the x and the y axis and their coefficients.
+template <typename real>
+struct FlatRows {
+    bool on[2];
+    unsigned at[2][2];
+    real b[2], c[2], ik[2], m[2][2];
+};
+
+template <typename real, bool forward>
+__device__ __forceinline__ FlatRows<real> flat_rows(const PlaneStep<real>& a, const real* psi, int x, int y, bool live) {
+    constexpr unsigned W = sizeof(real);
+    FlatRows<real> out;
+#pragma unroll
+    for (int ax = 0; ax < 2; ++ax) {
+        const int k = ax ? y : x, n = ax ? a.ny : a.nx;
+        const AxisRow<real> r = axis_row(a.axis[ax], k, live && (forward ? k < n - 1 : k > 0));
+        out.on[ax] = r.on;
+        out.b[ax] = out.c[ax] = out.ik[ax] = out.m[ax][0] = out.m[ax][1] = real(0);
+        out.at[ax][0] = out.at[ax][1] = 0u;
+        if (!r.on) continue;
+        const unsigned wide = (unsigned)r.w * W, coef = r.coef + (unsigned)r.q * W;
+        const unsigned cell = ax ? (unsigned)x * wide + (unsigned)r.q * W : ((unsigned)r.q * a.ny + y) * W;
+        out.b[ax] = at_byte(a.coef, coef);
+        out.c[ax] = at_byte(a.coef, coef + wide);
+        out.ik[ax] = at_byte(a.coef, coef + 2 * wide);
+        for (int t = 0; t < 2; ++t) {
+            out.at[ax][t] = r.psi[t] + cell;
+            out.m[ax][t] = at_byte(psi, out.at[ax][t]);
+        }
+    }
+    return out;
+}
+
+template <typename real, bool forward>
+__device__ __forceinline__ void flat_half(const PlaneStep<real>& a, const real (*from)[kFlatTile * kFlatTile], const int next[2],
+                                          const Cell<real>& here, Cell<real>& field, const Cell<real>& coefficient,
+                                          FlatRows<real>& rows, const bool any[2], int x, int y, bool source, bool sources, long long n) {
+    real curl[3] = {real(0), real(0), real(0)};
+#pragma unroll
+    for (int ax = 0; ax < 2; ++ax) {
+        const int k = ax ? y : x, last = (ax ? a.ny : a.nx) - 1;
+        const bool in = forward ? k < last : k > 0, wrap = (a.periodic_mask >> ax) & 1;
+        const bool pecs = forward && ((a.pec_mask >> ax) & 1);
+        const real pec = pecs ? -a.pec_factor[ax] : real(0);
+        real d[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int ic = term_in(2 * ax + j);
+            const real nb = from[ic][next[ax]];
+            d[j] = forward ? nb - here.v[ic] : here.v[ic] - nb;
+        }
+        if (any[ax]) {
+            asm volatile("");       // a branch, as in march_half_step
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const real m = rows.m[ax][j] * rows.b[ax] + rows.c[ax] * d[j];
+                const real stretched = d[j] * rows.ik[ax] + m;
+                rows.m[ax][j] = m;
+                d[j] = rows.on[ax] ? stretched : d[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int t = 2 * ax + j, ic = term_in(t), oc = term_out(t);
+            if (!in && !wrap) d[j] = pecs ? pec * here.v[ic] : real(0);
+            curl[oc] = term_sign(t) > 0 ? curl[oc] + d[j] : curl[oc] - d[j];
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        const real change = coefficient.v[m] * curl[m];
+        field.v[m] = forward ? field.v[m] - change : field.v[m] + change;
+    }
+    if (sources)
+        for (int k = 0; k < a.nsrc && n < a.source_samples; ++k) {
+            const Source<real>& box = a.srcs[k];
+            const bool hit = source & (x >= box.lo[0]) & (x < box.hi[0]) & (y >= box.lo[1]) & (y < box.hi[1]);
+            const real v = global(box.values)[n];
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+                if (box.comp == m && hit) field.v[m] = field.v[m] + v;
+        }
+}
+
+template <typename real, int INV>
+__global__ __launch_bounds__(kFlatTile * kFlatTile, sizeof(real) == 8 ? 4 : 8) void flat_steps_kernel(const FlatPass<real> a) {
+    constexpr int T = kFlatTile;
+    __shared__ real se[3][T * T], sh[3][T * T];
+    const int nx = a.e.nx, ny = a.e.ny, tid = threadIdx.x, ly = tid & (T - 1), lx = tid / T;
+    const int own = T - 2 * a.steps, bx = blockIdx.x / a.tiles_y, by = blockIdx.x - bx * a.tiles_y;
+    int x = bx * own - a.steps + lx, y = by * own - a.steps + ly;
+    const bool owned = lx >= a.steps && lx < T - a.steps && ly >= a.steps && ly < T - a.steps && x < nx && y < ny;
+    // A periodic axis continues with its other end's cells; elsewhere lanes beyond the grid hold zeros that no cell reads.
+    if (a.e.periodic_mask & 1) { x %= nx; x += x < 0 ? nx : 0; }
+    if (a.e.periodic_mask & 2) { y %= ny; y += y < 0 ? ny : 0; }
+    const bool live = x >= 0 && x < nx && y >= 0 && y < ny;
+    const long long cell = live ? (long long)x * ny + y : 0;
+    Cell<real> e{{real(0), real(0), real(0)}}, h = e, ce = e, ch = e;
+    if (live) {
+        e = cell_at(a.in.e, cell);
+        h = cell_at(a.in.h, cell);
+        if (INV == 3) ce = cell_at(a.e.inverse, cell);
+        else ce.v[0] = ce.v[1] = ce.v[2] = global(a.e.inverse)[cell];
+    }
+    const real one = global(a.h.inverse)[0];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+        ce.v[m] = a.e.courant * ce.v[m];
+        ch.v[m] = a.h.courant * one;
+    }
+    FlatRows<real> re = flat_rows<real, false>(a.e, a.in.psi_e, x, y, live);
+    FlatRows<real> rh = flat_rows<real, true>(a.h, a.in.psi_h, x, y, live);
+    const long long n0 = *global(a.counter);
+    auto any = [](bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; };
+    const bool rows_e[2] = {any(re.on[0]), any(re.on[1])}, rows_h[2] = {any(rh.on[0]), any(rh.on[1])};
+    const bool srcs_e = any(live && a.e.nsrc > 0 && x >= a.e.box_lo[0] && x < a.e.box_hi[0] && y >= a.e.box_lo[1] && y < a.e.box_hi[1]);
+    const bool srcs_h = any(live && a.h.nsrc > 0 && x >= a.h.box_lo[0] && x < a.h.box_hi[0] && y >= a.h.box_lo[1] && y < a.h.box_hi[1]);
+    bool trace = false;
+    for (int k = 0; k < a.h.ntraces; ++k) trace |= owned && a.h.trace[k].x == x && a.h.trace[k].cell == y;
+    const bool traces = any(trace);
+    // Neighbours of lanes at the patch's edge lie outside it: those lanes read themselves, and their cells are spoilt.
+    const int low[2] = {lx > 0 ? tid - T : tid, ly > 0 ? tid - 1 : tid};
+    const int high[2] = {lx < T - 1 ? tid + T : tid, ly < T - 1 ? tid + 1 : tid};
+#pragma unroll
+    for (int m = 0; m < 3; ++m) sh[m][tid] = h.v[m];
+    __syncthreads();
+    for (int s = 0; s < a.steps; ++s) {
+        flat_half<real, false>(a.e, sh, low, h, e, ce, re, rows_e, x, y, live, srcs_e, n0 + s);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) se[m][tid] = e.v[m];
+        __syncthreads();
+        flat_half<real, true>(a.h, se, high, e, h, ch, rh, rows_h, x, y, live, srcs_h, n0 + s);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) sh[m][tid] = h.v[m];
+        if (traces && trace && n0 + s < a.h.trace_steps)
+            for (int k = 0; k < a.h.ntraces; ++k) {
+                const PlaneTrace& t = a.h.trace[k];
+                if (t.x != x || t.cell != y) continue;
+                const real fe = t.component == 0 ? e.v[0] : t.component == 1 ? e.v[1] : e.v[2];
+                const real fh = t.component == 0 ? h.v[0] : t.component == 1 ? h.v[1] : h.v[2];
+                global(a.h.traces)[(n0 + s) * a.h.ntraces + k] = t.magnetic ? fh : fe;
+            }
+        __syncthreads();
+    }
+    if (owned) {
+        const auto to_e = global(a.out.e + 3 * cell), to_h = global(a.out.h + 3 * cell);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            to_e[m] = e.v[m];
+            to_h[m] = h.v[m];
+        }
+#pragma unroll
+        for (int ax = 0; ax < 2; ++ax)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (re.on[ax]) put_byte(a.out.psi_e, re.at[ax][t], re.m[ax][t]);
+                if (rh.on[ax]) put_byte(a.out.psi_h, rh.at[ax][t], rh.m[ax][t]);
+            }
+    }
+    if (blockIdx.x == 0 && tid == 0) *global(a.counter_to) = n0 + a.steps;
+}
+
 // One grid of a batched half step: its plane march where `march` is set, else the general step.
 template <typename real>
 struct BatchStep {
@@ -1115,6 +1316,26 @@ int batch_half_step(const void* device_table, const int32_t* device_prefix, int 
     return check_launch("batch_half_step");
 }
 
+// The traces of a step at the cells its H launch updates, where they are few enough.
+template <typename real>
+int fold_traces(const tfdtd_observe* obs, const tfdtd_trace_cell* cells, PlaneStep<real>* h, bool* folded) {
+    *folded = cells && obs->count > 0 && obs->count <= kPlaneTraces;
+    if (!*folded) return TFDTD_OK;
+    h->ntraces = obs->count;
+    h->traces = static_cast<real*>(obs->traces);
+    h->trace_steps = (long long)obs->steps;
+    h->trace_lo = h->nx;
+    const long long values = 3LL * h->nx * h->nyz;
+    for (int k = 0; k < obs->count; ++k) {
+        if (cells[k].element < 0 || cells[k].element >= values) return fail(TFDTD_EINVAL, "trace %d lies outside the grid", k);
+        const long long cell = cells[k].element / 3;
+        h->trace[k] = PlaneTrace{(int)(cell / h->nyz), (int)(cell % h->nyz), (int)(cells[k].element % 3), cells[k].magnetic};
+        h->trace_lo = std::min(h->trace_lo, h->trace[k].x);
+        h->trace_hi = std::max(h->trace_hi, h->trace[k].x + 1);
+    }
+    return TFDTD_OK;
+}
+
 // One step of a grid whose half steps both march: E (copying the counter to `shadow`), H (stepping the counter on and
 // recording up to TFDTD_FOLDED_TRACES traces), planes and further traces, which read the copy.  A launch of its own
 // for the traces and the counter cost 0.9 us a step on 160x120x40 cells (930 -> 884 us for 50 steps), 1.1 us
@@ -1136,21 +1357,9 @@ int observed_step(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, 
     ph.counter = shadow;
     ph.counter_to = counter;
     ph.counter_add = 1;
-    const bool folded = cells && obs->count > 0 && obs->count <= kPlaneTraces;
-    if (folded) {
-        ph.ntraces = obs->count;
-        ph.traces = static_cast<real*>(obs->traces);
-        ph.trace_steps = (long long)obs->steps;
-        ph.trace_lo = ph.nx;
-        const long long values = 3LL * ph.nx * ph.nyz;
-        for (int k = 0; k < obs->count; ++k) {
-            if (cells[k].element < 0 || cells[k].element >= values) return fail(TFDTD_EINVAL, "trace %d lies outside the grid", k);
-            const long long cell = cells[k].element / 3;
-            ph.trace[k] = PlaneTrace{(int)(cell / ph.nyz), (int)(cell % ph.nyz), (int)(cells[k].element % 3), cells[k].magnetic};
-            ph.trace_lo = std::min(ph.trace_lo, ph.trace[k].x);
-            ph.trace_hi = std::max(ph.trace_hi, ph.trace[k].x + 1);
-        }
-    }
+    bool folded = false;
+    status = fold_traces(obs, cells, &ph, &folded);
+    if (status) return status;
     launch_plane_step(pe, false, e_step->inverse_stride, stream);
     status = check_launch("yee_half_step");
     if (status) return status;
@@ -1159,6 +1368,46 @@ int observed_step(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, 
     if (!status) status = planes(p, plane_count, stream, shadow);
     if (!status && obs->count > 0 && !folded) status = record_traces(obs, shadow, stream);
     return status;
+}
+
+// Passes of a flat run of `n` steps: an even number, so the state returns to its buffers, of nearly equal steps.
+template <typename real>
+int flat_steps(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_observe* obs, const tfdtd_trace_cell* cells,
+               const FlatSet<real>& second, long long* shadow, int n, hipStream_t stream) {
+    HalfStep<real> e, h;
+    int status = make_half_step(e_step, &e);
+    if (!status) status = make_half_step(h_step, &h);
+    if (status) return status;
+    FlatPass<real> a;
+    if (e.nz != 1 || e.nx != h.nx || e.ny != h.ny || e.nz != h.nz || e.src != h.dst || e.dst != h.src ||
+        e.periodic_mask != h.periodic_mask || !make_plane_step(e, false, &a.e) || !make_plane_step(h, true, &a.h))
+        return fail(TFDTD_EUNSUPPORTED, "flat_steps needs one grid of one z plane that the plane march takes");
+    bool folded = false;
+    status = fold_traces(obs, cells, &a.h, &folded);
+    if (status) return status;
+    if (obs->count > 0 && !folded) return fail(TFDTD_EUNSUPPORTED, "flat_steps records at most %d traces", kPlaneTraces);
+    if (n == 0) return TFDTD_OK;
+    long long* const counter = reinterpret_cast<long long*>(obs->counter);
+    const FlatSet<real> own{a.e.dst, a.h.dst, a.e.psi, a.h.psi};
+    const int depth = flat_depth(a.e.nx, a.e.ny), passes = (n + 2 * depth - 1) / (2 * depth) * 2;
+    for (int k = 0; k < passes; ++k) {
+        const bool back = k & 1;
+        a.in = back ? second : own;
+        a.out = back ? own : second;
+        a.counter = back ? shadow : counter;
+        a.counter_to = back ? counter : shadow;
+        a.steps = n / passes + (k < n % passes);
+        const int width = kFlatTile - 2 * a.steps;
+        a.tiles_y = (a.e.ny + width - 1) / width;
+        const long long tiles = flat_tiles(a.e.nx, a.e.ny, a.steps);
+        if (tiles > 0x7fffffffLL) return fail(TFDTD_EINVAL, "grid too large for one launch");
+        const dim3 grid((unsigned)tiles), block(kFlatTile * kFlatTile);
+        if (e_step->inverse_stride == 1) hipLaunchKernelGGL((flat_steps_kernel<real, 1>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((flat_steps_kernel<real, 3>), grid, block, 0, stream, a);
+        status = check_launch("flat_steps");
+        if (status) return status;
+    }
+    return TFDTD_OK;
 }
 
 }  // namespace
@@ -1315,6 +1564,26 @@ int tfdtd_step_observed(const tfdtd_half_step* e_step, const tfdtd_half_step* h_
     else return fail(TFDTD_EINVAL, "dtype must be float32 or float64");
     if (status || done) return status;
     return tfdtd_step_fused(e_step, h_step, p, plane_count, obs, 1, stream);
+}
+
+int tfdtd_flat_steps(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_observe* obs,
+                     const tfdtd_trace_cell* cells, const tfdtd_flat_buffers* second, int64_t* shadow, int32_t n_steps, void* stream) {
+    if (!e_step || !h_step || e_step->family != TFDTD_FAMILY_E || h_step->family != TFDTD_FAMILY_H || e_step->dtype != h_step->dtype)
+        return fail(TFDTD_EINVAL, "flat_steps needs an E and an H descriptor of one dtype");
+    if (!obs || !obs->counter) return fail(TFDTD_EINVAL, "flat_steps needs the observe descriptor and its counter");
+    if (obs->count < 0 || (obs->count > 0 && (!obs->table || !obs->traces)))
+        return fail(TFDTD_EINVAL, "observe: trace table and traces are required");
+    if (n_steps < 0 || n_steps == 1) return fail(TFDTD_EINVAL, "flat_steps takes two steps or more (0: asks whether it takes the grid)");
+    if (n_steps > 0 && (!shadow || !second || !second->e || !second->h || !second->psi_e || !second->psi_h))
+        return fail(TFDTD_EINVAL, "flat_steps needs a second buffer set and the shadow");
+    const tfdtd_flat_buffers b = second ? *second : tfdtd_flat_buffers{};
+    long long* const copy = reinterpret_cast<long long*>(shadow);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (e_step->dtype == TFDTD_F32)
+        return flat_steps<float>(e_step, h_step, obs, cells, {(float*)b.e, (float*)b.h, (float*)b.psi_e, (float*)b.psi_h}, copy, n_steps, s);
+    if (e_step->dtype == TFDTD_F64)
+        return flat_steps<double>(e_step, h_step, obs, cells, {(double*)b.e, (double*)b.h, (double*)b.psi_e, (double*)b.psi_h}, copy, n_steps, s);
+    return fail(TFDTD_EINVAL, "dtype must be float32 or float64");
 }
 
 int tfdtd_record_traces(const tfdtd_observe* d, void* stream) {

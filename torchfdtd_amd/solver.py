@@ -308,6 +308,7 @@ class Stepper:
         self.counter = torch.zeros(1, device=device, dtype=torch.long) if counter is None else counter
         # The split step's copy of the counter: written by its E launch, read by the launches after it.
         self.shadow = torch.zeros(1, device=device, dtype=torch.long)
+        self.flat_set = None        # second buffer set of `block`
         terms = source_terms(p, self.steps)
         self.sources = {'E': [], 'H': []}
         for t in terms:
@@ -662,6 +663,32 @@ class Stepper:
             N.check(self.lib.tfdtd_dft_update(self.plane_table, len(self.planes), stream), 'tfdtd_dft_update')
         N.check(self.lib.tfdtd_observe_step(ctypes.byref(self.observe), stream), 'tfdtd_observe_step')
 
+    def flat(self):
+        """Whether `block` takes this grid: one z plane, at most `FOLDED_TRACES` traces, no plane monitors, no ADE.
+        Allocates its second buffer set (on the caller's stream, outside any capture)."""
+        if self.kernel != 'hip' or self.dispersive or self.planes or self.grid.Nz != 1:
+            return False
+        status = self.lib.tfdtd_flat_steps(ctypes.byref(self.e_step), ctypes.byref(self.h_step), ctypes.byref(self.observe),
+                                           self.trace_cells, None, None, 0, None)
+        if status == N.EUNSUPPORTED:
+            return False
+        N.check(status, 'tfdtd_flat_steps')
+        if self.flat_set is None:
+            g = self.grid
+            self.flat_set = [torch.empty_like(t) for t in (g.E, g.H, g.psi_buffers[False], g.psi_buffers[True])]
+        return True
+
+    def block(self, count):
+        """`count` steps of a grid that is `flat`, several to a launch; bit for bit `count` calls of step."""
+        if count < 2:
+            for _ in range(count):
+                self.step()
+            return
+        second = N.FlatBuffers(*(t.data_ptr() for t in self.flat_set))
+        N.check(self.lib.tfdtd_flat_steps(ctypes.byref(self.e_step), ctypes.byref(self.h_step), ctypes.byref(self.observe),
+                                          self.trace_cells, ctypes.byref(second), self.shadow.data_ptr(), count,
+                                          N.stream_handle(self.grid.device)), 'tfdtd_flat_steps')
+
     def _dispersive_step(self, stream):
         """The reference's order with MaterialADE (cuda_kernels.py:355-362, solver.py:785-797): save E at
         the owned samples, E update, ADE correction, E sources, H update and sources, planes, traces."""
@@ -714,7 +741,7 @@ class Simulation:
                    if control.auto_shutoff or control.divergence_check else None)
         graph = (StepGraphs(run.step, run.states(), r.steps, cuda_graph_steps, pair=run.step_pair if run.one_pass else None,
                             prepare=run.refresh_materials if run.one_pass else None,
-                            quad=run.quad if run.two_step else None)
+                            quad=run.quad if run.two_step else None, block=run.block if run.flat() else None)
                  if cuda_graph else None)
         view = DisplaySlice(p)
         plane_index = view.index
