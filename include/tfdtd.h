@@ -450,6 +450,12 @@ typedef struct tfdtd_curl_record {
 
 int tfdtd_record_curl(const tfdtd_curl_record* record, void* stream);
 
+/* tfdtd_record_curl, then tfdtd_step_observed; the record is made by the E launch where the plane march takes the
+ * step and the record reads the step's own H, memory and counter. */
+int tfdtd_step_recorded(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_plane* planes,
+                        int32_t plane_count, const tfdtd_observe* observe, const tfdtd_trace_cell* cells, int64_t* shadow,
+                        const tfdtd_curl_record* record, void* stream);
+
 /* One step of the discrete adjoint, backwards (torchfdtd/differentiable.py:496-519 and
  * torchfdtd/cuda_adjoint.py:218-234, FusedAdjointCUDA.step): for t = *counter,
  *   e_bar/h_bar[target k] += sum of seeds[t][seed_columns[seed_offsets[k] .. seed_offsets[k+1])]

@@ -186,6 +186,8 @@ PROTOTYPES = {
     'tfdtd_record_traces': (i32, [ctypes.POINTER(Observe), vp]),
     'tfdtd_step_observed': (i32, [ctypes.POINTER(HalfStep), ctypes.POINTER(HalfStep), ctypes.POINTER(Plane), i32,
                                   ctypes.POINTER(Observe), ctypes.POINTER(TraceCell), vp, vp]),
+    'tfdtd_step_recorded': (i32, [ctypes.POINTER(HalfStep), ctypes.POINTER(HalfStep), ctypes.POINTER(Plane), i32,
+                                  ctypes.POINTER(Observe), ctypes.POINTER(TraceCell), vp, ctypes.POINTER(CurlRecord), vp]),
     'tfdtd_flat_steps': (i32, [ctypes.POINTER(HalfStep), ctypes.POINTER(HalfStep), ctypes.POINTER(Observe), ctypes.POINTER(TraceCell),
                                ctypes.POINTER(FlatBuffers), vp, i32, vp]),
     'tfdtd_batch_march_bytes': (ctypes.c_size_t, [i32, i32]),

@@ -200,8 +200,7 @@ class _Engine:
 
     # ------------------------------------------------------------------ forward
     def _step(self):
-        N.check(self.lib.tfdtd_record_curl(ctypes.byref(self.records[0]), N.stream_handle()), 'tfdtd_record_curl')
-        self.run.step()
+        self.run.step(self.records[0])
 
     def _pair(self):
         run, lib, stream = self.run, self.lib, N.stream_handle()

@@ -338,12 +338,6 @@ __device__ __forceinline__ void write_memory(real* psi, const MarchRow<real>& ro
         for (int k = 0; k < 2; ++k) put_byte(psi, row.at[k] + x * row.stride, row.b * m[k]);
 }
 
-// t % modulus, in 32 bits where both fit.
-__device__ __forceinline__ long long slot_of(long long t, long long modulus) {
-    if (((t | modulus) >> 31) == 0) return (long long)((unsigned)t % (unsigned)modulus);
-    return t % modulus;
-}
-
 template <typename real, int INV, bool FLAT>
 __global__ __launch_bounds__(256, sizeof(real) == 8 ? 3 : 5) void h_transpose_march_kernel(const AdjointMarch<real> a) {
     constexpr unsigned W = sizeof(real);

@@ -83,6 +83,12 @@ __device__ __forceinline__ unsigned wave_item(unsigned block) {
     return block * 4u + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
+// t % modulus, in 32 bits where both fit.
+__device__ __forceinline__ long long slot_of(long long t, long long modulus) {
+    if (((t | modulus) >> 31) == 0) return (long long)((unsigned)t % (unsigned)modulus);
+    return t % modulus;
+}
+
 constexpr unsigned kXcdRun = 128;
 
 // Planes per march: two share the lane's set-up and the plane between them (18.9 against 20.7 us a step on

@@ -242,8 +242,20 @@ __device__ __forceinline__ void carry_counter(const long long* from, long long* 
     if (to && blockIdx.x == 0 && threadIdx.x == 0) *global(to) = *global(from) + add;
 }
 
-template <typename real, bool forward, int INV, bool FLAT>
-__device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const unsigned item) {
+// The adjoint's record folded into the E step: the curl that the update of a box cell adds, in slot
+// counter % modulus.
+template <typename real>
+struct CurlBox {
+    int lo[3], hi[3];
+    long long modulus;
+    real* record;
+};
+
+struct NoBox {};
+
+template <typename real, bool forward, int INV, bool FLAT, typename Box>
+__device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const unsigned item, const Box& box) {
+    constexpr bool recorded = !std::is_same<Box, NoBox>::value;
     constexpr unsigned W = sizeof(real);
     const int nx = a.nx, ny = a.ny, nz = FLAT ? 1 : a.nz, nyz = a.nyz;
     // Spare lanes of the last column and spare wavefronts of the last workgroup repeat a cell and store nothing.
@@ -301,6 +313,17 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
     // A wavefront without slab rows of an axis skips that axis's memory.
     const bool anyy = __builtin_amdgcn_ballot_w64(hy.on) != 0, anyz = !FLAT && __builtin_amdgcn_ballot_w64(hz.on) != 0;
     real* const psi = a.psi;
+    bool boxed = false;
+    real* record = nullptr;     // the box's plane of this x, and the lane's byte offset in it
+    unsigned record_at = 0u;
+    long long record_plane = 0;
+    if constexpr (recorded) {
+        const int by = box.hi[1] - box.lo[1], bz = box.hi[2] - box.lo[2];
+        boxed = owned & (y >= box.lo[1]) & (y < box.hi[1]) & (z >= box.lo[2]) & (z < box.hi[2]);
+        record_at = (unsigned)((y - box.lo[1]) * bz + z - box.lo[2]) * (3 * W);
+        record_plane = 3LL * by * bz;
+        record = box.record + (slot_of(*global(a.counter), box.modulus) * (box.hi[0] - box.lo[0]) + xa - box.lo[0]) * record_plane;
+    }
     for (int x = xa; x < xb; ++x) {
         // The lane offsets stay 32-bit values of the loop: widened once before it, every access would add them
         // to its base in 64-bit vector arithmetic.
@@ -388,6 +411,15 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
                     if (box.comp == m && in) out[m] = out[m] + v;
             }
         }
+        if constexpr (recorded) {
+            if (boxed && x >= box.lo[0] && x < box.hi[0]) {
+                const auto to = global(reinterpret_cast<real*>(reinterpret_cast<char*>(record) + record_at));
+                to[0] = curl[0];
+                to[1] = curl[1];
+                to[2] = curl[2];
+            }
+            record += record_plane;
+        }
         if (owned) {
             if (rx.on)
                 for (int t = 0; t < 2; ++t) put_byte(psix[t], line, mx[t]);
@@ -424,7 +456,15 @@ __device__ __forceinline__ void march_half_step(const PlaneStep<real>& a, const 
 
 template <typename real, bool forward, int INV, bool FLAT>
 __global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void plane_half_step_kernel(const PlaneStep<real> a) {
-    march_half_step<real, forward, INV, FLAT>(a, wave_item(xcd_block(blockIdx.x, gridDim.x, a.xcd)));
+    march_half_step<real, forward, INV, FLAT>(a, wave_item(xcd_block(blockIdx.x, gridDim.x, a.xcd)), NoBox{});
+    carry_counter(a.counter, a.counter_to, a.counter_add);
+}
+
+// The E step with the adjoint's record.  A launch of its own for the record read H and the CPML memory again and
+// took 4.7-4.9 us on a 50x50x6 box or a 71x66x37 grid, and its gap.
+template <typename real, int INV, bool FLAT>
+__global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void recorded_half_step_kernel(const PlaneStep<real> a, const CurlBox<real> box) {
+    march_half_step<real, false, INV, FLAT>(a, wave_item(xcd_block(blockIdx.x, gridDim.x, a.xcd)), box);
     carry_counter(a.counter, a.counter_to, a.counter_add);
 }
 
@@ -660,14 +700,14 @@ __global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void batch_half_ste
         const unsigned item = wave_item((unsigned)(b - prefix[lo]));
         const bool flat = t.plane.nz == 1;
         if (forward) {
-            if (flat) march_half_step<real, true, 0, true>(t.plane, item);
-            else march_half_step<real, true, 0, false>(t.plane, item);
+            if (flat) march_half_step<real, true, 0, true>(t.plane, item, NoBox{});
+            else march_half_step<real, true, 0, false>(t.plane, item, NoBox{});
         } else if (t.inverse_stride == 1) {
-            if (flat) march_half_step<real, false, 1, true>(t.plane, item);
-            else march_half_step<real, false, 1, false>(t.plane, item);
+            if (flat) march_half_step<real, false, 1, true>(t.plane, item, NoBox{});
+            else march_half_step<real, false, 1, false>(t.plane, item, NoBox{});
         } else {
-            if (flat) march_half_step<real, false, 3, true>(t.plane, item);
-            else march_half_step<real, false, 3, false>(t.plane, item);
+            if (flat) march_half_step<real, false, 3, true>(t.plane, item, NoBox{});
+            else march_half_step<real, false, 3, false>(t.plane, item, NoBox{});
         }
         return;
     }
@@ -1316,6 +1356,38 @@ int batch_half_step(const void* device_table, const int32_t* device_prefix, int 
     return check_launch("batch_half_step");
 }
 
+// The record of an E step as part of it: true where it reads what the step reads (the step's own H, memory and
+// counter, every slab applied).
+template <typename real>
+bool make_curl_box(const tfdtd_curl_record& d, const tfdtd_half_step& e, const tfdtd_observe& obs, const PlaneStep<real>& step, CurlBox<real>* box) {
+    if (d.dtype != e.dtype || d.nx != e.nx || d.ny != e.ny || d.nz != e.nz || d.H != e.src || d.counter != obs.counter ||
+        (d.periodic_mask & 7) != step.periodic_mask || !d.record || d.modulus < 1)
+        return false;
+    if (step.psi && d.e.psi_in != step.psi) return false;
+    const int n[3] = {d.nx, d.ny, d.nz};
+    for (int k = 0; k < 3; ++k) {
+        if (d.box_lo[k] < 0 || d.box_hi[k] <= d.box_lo[k] || d.box_hi[k] > n[k]) return false;
+        box->lo[k] = d.box_lo[k];
+        box->hi[k] = d.box_hi[k];
+    }
+    box->modulus = d.modulus;
+    box->record = static_cast<real*>(d.record);
+    return true;
+}
+
+template <typename real>
+void launch_recorded_step(const PlaneStep<real>& a, const CurlBox<real>& box, int inverse_stride, hipStream_t stream) {
+    const dim3 grid((unsigned)plane_blocks(a)), block(256);
+    const bool flat = a.nz == 1;
+    if (inverse_stride == 1) {
+        if (flat) hipLaunchKernelGGL((recorded_half_step_kernel<real, 1, true>), grid, block, 0, stream, a, box);
+        else hipLaunchKernelGGL((recorded_half_step_kernel<real, 1, false>), grid, block, 0, stream, a, box);
+    } else {
+        if (flat) hipLaunchKernelGGL((recorded_half_step_kernel<real, 3, true>), grid, block, 0, stream, a, box);
+        else hipLaunchKernelGGL((recorded_half_step_kernel<real, 3, false>), grid, block, 0, stream, a, box);
+    }
+}
+
 // The traces of a step at the cells its H launch updates, where they are few enough.
 template <typename real>
 int fold_traces(const tfdtd_observe* obs, const tfdtd_trace_cell* cells, PlaneStep<real>* h, bool* folded) {
@@ -1342,7 +1414,8 @@ int fold_traces(const tfdtd_observe* obs, const tfdtd_trace_cell* cells, PlaneSt
 // on 160x120x1.
 template <typename real>
 int observed_step(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_plane* p, int plane_count,
-                  const tfdtd_observe* obs, const tfdtd_trace_cell* cells, long long* shadow, hipStream_t stream, bool* done) {
+                  const tfdtd_observe* obs, const tfdtd_trace_cell* cells, long long* shadow, const tfdtd_curl_record* record,
+                  hipStream_t stream, bool* done) {
     *done = false;
     HalfStep<real> e, h;
     int status = make_half_step(e_step, &e);
@@ -1350,6 +1423,8 @@ int observed_step(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, 
     if (status) return status;
     PlaneStep<real> pe, ph;
     if (!make_plane_step(e, false, &pe) || !make_plane_step(h, true, &ph)) return TFDTD_OK;
+    CurlBox<real> box;
+    if (record && !make_curl_box(*record, *e_step, *obs, pe, &box)) return TFDTD_OK;
     *done = true;
     long long* const counter = reinterpret_cast<long long*>(obs->counter);
     pe.counter = counter;
@@ -1360,7 +1435,8 @@ int observed_step(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, 
     bool folded = false;
     status = fold_traces(obs, cells, &ph, &folded);
     if (status) return status;
-    launch_plane_step(pe, false, e_step->inverse_stride, stream);
+    if (record) launch_recorded_step(pe, box, e_step->inverse_stride, stream);
+    else launch_plane_step(pe, false, e_step->inverse_stride, stream);
     status = check_launch("yee_half_step");
     if (status) return status;
     launch_plane_step(ph, true, h_step->inverse_stride, stream);
@@ -1549,6 +1625,12 @@ int tfdtd_step_fused(const tfdtd_half_step* e_step, const tfdtd_half_step* h_ste
 
 int tfdtd_step_observed(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_plane* p, int32_t plane_count,
                         const tfdtd_observe* obs, const tfdtd_trace_cell* cells, int64_t* shadow, void* stream) {
+    return tfdtd_step_recorded(e_step, h_step, p, plane_count, obs, cells, shadow, nullptr, stream);
+}
+
+int tfdtd_step_recorded(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, const tfdtd_plane* p, int32_t plane_count,
+                        const tfdtd_observe* obs, const tfdtd_trace_cell* cells, int64_t* shadow, const tfdtd_curl_record* record,
+                        void* stream) {
     if (!e_step || !h_step || e_step->family != TFDTD_FAMILY_E || h_step->family != TFDTD_FAMILY_H)
         return fail(TFDTD_EINVAL, "step_observed needs an E and an H descriptor");
     if (!obs || !obs->counter || !shadow) return fail(TFDTD_EINVAL, "step_observed needs the observe descriptor, its counter and the shadow");
@@ -1559,10 +1641,11 @@ int tfdtd_step_observed(const tfdtd_half_step* e_step, const tfdtd_half_step* h_
     long long* const copy = reinterpret_cast<long long*>(shadow);
     bool done = false;
     int status;
-    if (e_step->dtype == TFDTD_F32) status = observed_step<float>(e_step, h_step, p, plane_count, obs, cells, copy, s, &done);
-    else if (e_step->dtype == TFDTD_F64) status = observed_step<double>(e_step, h_step, p, plane_count, obs, cells, copy, s, &done);
+    if (e_step->dtype == TFDTD_F32) status = observed_step<float>(e_step, h_step, p, plane_count, obs, cells, copy, record, s, &done);
+    else if (e_step->dtype == TFDTD_F64) status = observed_step<double>(e_step, h_step, p, plane_count, obs, cells, copy, record, s, &done);
     else return fail(TFDTD_EINVAL, "dtype must be float32 or float64");
     if (status || done) return status;
+    if (record && (status = tfdtd_record_curl(record, stream))) return status;
     return tfdtd_step_fused(e_step, h_step, p, plane_count, obs, 1, stream);
 }
 

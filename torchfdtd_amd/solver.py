@@ -644,15 +644,19 @@ class Stepper:
             for _ in range(count):
                 self.step()
 
-    def step(self):
+    def step(self, record=None):
+        """One step; `record` (a CurlRecord) has its E update's curl recorded."""
         stream = N.stream_handle(self.grid.device)
+        if self.kernel == 'hip' and not self.dispersive:
+            N.check(self.lib.tfdtd_step_recorded(ctypes.byref(self.e_step), ctypes.byref(self.h_step), self.plane_table,
+                                                 len(self.planes), ctypes.byref(self.observe), self.trace_cells,
+                                                 self.shadow.data_ptr(), None if record is None else ctypes.byref(record),
+                                                 stream), 'tfdtd_step_recorded')
+            return
+        if record is not None:
+            N.check(self.lib.tfdtd_record_curl(ctypes.byref(record), stream), 'tfdtd_record_curl')
         if self.dispersive:
             self._dispersive_step(stream)
-            return
-        if self.kernel == 'hip':
-            N.check(self.lib.tfdtd_step_observed(ctypes.byref(self.e_step), ctypes.byref(self.h_step), self.plane_table,
-                                                 len(self.planes), ctypes.byref(self.observe), self.trace_cells,
-                                                 self.shadow.data_ptr(), stream), 'tfdtd_step_observed')
             return
         g = self.grid
         g.update_E()
