@@ -173,6 +173,7 @@ class Adjoint(ctypes.Structure):
 
 
 _lib = None
+_gpu_found = False
 
 PROTOTYPES = {
     'tfdtd_yee_step_march': (i32, [ctypes.POINTER(March), vp]),
@@ -258,10 +259,14 @@ def load_library(path=None):
 
 
 def library():
-    """The loaded library, with a GPU present; raises otherwise (no CPU fallback)."""
-    import torch
-    if not torch.cuda.is_available():
-        raise RuntimeError('torchfdtd_amd runs on an AMD GPU (gfx950); no GPU is visible')
+    """The loaded library, with a GPU present; raises otherwise (no CPU fallback).  The GPU is looked for until it is
+    found: each look costs 3 us, and a training step of the surrogate comes here 15 times."""
+    global _gpu_found
+    if not _gpu_found:
+        import torch
+        if not torch.cuda.is_available():
+            raise RuntimeError('torchfdtd_amd runs on an AMD GPU (gfx950); no GPU is visible')
+        _gpu_found = True
     return load_library()
 
 
@@ -283,5 +288,10 @@ def address(tensor):
 
 
 def stream_handle(device=None):
+    """The current stream's handle, without the 4 us of a torch Stream object."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = None if device is None else torch.device(device).index
+    if index is None:
+        index = torch.cuda.current_device()
+    torch.cuda.init()
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(index))
