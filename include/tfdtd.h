@@ -536,10 +536,12 @@ int tfdtd_conv_weight_parts(const tfdtd_conv* conv);
 int tfdtd_conv_weights(const tfdtd_conv* convs, int32_t count, const float* const* weights, void* const* w16,
                        void* const* weights_t, int32_t* const* nonfinite, void* stream);
 /* tfdtd_conv_forward with any of its outputs: pre FP32, y FP32 (the value of the bf16 activation), act bf16.
+ * x is bf16 (x_dtype TFDTD_CONV_BF16), or FP32 (TFDTD_F32) for layers of kp 32, which round it as they read it.
  * With `nonfinite` (of tfdtd_conv_weights) a tap that is padding for all rows of a workgroup is skipped when every
  * weight is finite.  TFDTD_EUNSUPPORTED where channels (multiples of 8, or kp 32) or the 16-byte alignment
  * of the operands leave the layer to tfdtd_conv_forward; likewise tfdtd_conv_dgrad_rows to tfdtd_conv_dgrad. */
-int tfdtd_conv_forward_rows(const tfdtd_conv* conv, const void* x, const void* weight, const int32_t* nonfinite, const float* bias,
+#define TFDTD_CONV_BF16 2
+int tfdtd_conv_forward_rows(const tfdtd_conv* conv, const void* x, int32_t x_dtype, const void* weight, const int32_t* nonfinite, const float* bias,
                             int32_t activation, float* pre, float* y, void* act, void* stream);
 int tfdtd_conv_dgrad_rows(const tfdtd_conv* conv, const void* dy, const void* weight_t, const int32_t* nonfinite, float* dx,
                           void* stream);

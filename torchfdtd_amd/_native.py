@@ -134,6 +134,7 @@ ADE_MAX_POLES = 16
 BIAS_BLOCKS = 2048
 CONV_WEIGHT_JOBS = 8
 EUNSUPPORTED = 3
+CONV_BF16 = 2
 
 
 class Ade(ctypes.Structure):
@@ -214,7 +215,7 @@ PROTOTYPES = {
     'tfdtd_conv_wgrad': (i32, [vp, vp, vp, i32, vp, vp, vp]),
     'tfdtd_conv_weight_parts': (i32, [vp]),
     'tfdtd_conv_weights': (i32, [vp, i32, vp, vp, vp, vp, vp]),
-    'tfdtd_conv_forward_rows': (i32, [vp, vp, vp, vp, vp, i32, vp, vp, vp, vp]),
+    'tfdtd_conv_forward_rows': (i32, [vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, vp]),
     'tfdtd_conv_dgrad_rows': (i32, [vp, vp, vp, vp, vp, vp]),
     'tfdtd_conv_wgrad_splits': (i32, [vp]),
     'tfdtd_conv_wgrad_rows': (i32, [vp, vp, vp, vp, vp, vp]),

@@ -271,6 +271,7 @@ __device__ __forceinline__ void chunk_to_lds(const void* from, bf16_bits* to) {
 struct GatherGemm {
     Conv c;
     int dgrad;                  // 0 forward, 1 input gradient
+    int wide;                   // 1: the source is FP32, rounded to bf16 as it is read (narrow forward)
     int rows_max;               // rows of the largest class
     unsigned run;               // row tiles an XCD takes in a row
     int N, channels, ldw;       // columns, source channels, weight row length
@@ -672,10 +673,12 @@ __global__ __launch_bounds__(256) void weights_kernel(const WeightsJobs jobs) {
 
 // Forward convolution with at most 32 values of K (a one-channel input): no staging pays, a wavefront takes
 // 64 rows, gathers each row's K values into the MFMA operand and keeps the weights of its columns in
-// registers.  Bound by its vector instructions, of which the activation is nearly half: 2,097,152 rows x 32
-// columns to bf16 take 108 us (128 with a division and three comparisons per value, the bias read again behind
-// every row's stores and the rounding in integer instructions); 524,288 rows with the FP32 pre-activation took
-// 107 us in gemm_kernel and its conversion pass.
+// registers.  Bound by its vector instructions, of which the activation is nearly half, and its scattered 2- or
+// 4-byte loads: 524,288 rows x 32 columns to FP32 and bf16 take 39 us (107 in gemm_kernel and its conversion pass; 41
+// with the taps' mask formed tap by tap instead of axis by axis), 2,097,152 rows to bf16 from bf16 108 us (128 with a
+// division and three comparisons per value, the bias read again behind every row's stores and the rounding in
+// integer instructions).  An FP32 source (`Wide`) is rounded as it is read: 113 us, where the conversion pass before it
+// took 20.
 // n / d for n, d <= 32: (n * small_reciprocal(d)) >> 10 (the excess n * (d - 1) stays below 1024).
 __host__ __device__ constexpr int small_reciprocal(int d) { return (1023 + d) / d; }
 
@@ -684,7 +687,7 @@ struct NarrowSplit {
     int per_ci, per_ks, per_ks2;    // small_reciprocal of ci, ks and ks * ks
 };
 
-template <int CT>
+template <int CT, bool Wide>
 __global__ __launch_bounds__(256) void narrow_forward_kernel(const GatherGemm g, int rows, const NarrowSplit split) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Conv& c = g.c;
@@ -715,21 +718,26 @@ __global__ __launch_bounds__(256) void narrow_forward_kernel(const GatherGemm g,
         const unsigned u = divide((unsigned)row, split.by_w), v = divide(u, split.by_h), nb = divide(v, split.by_d);
         const int x = (row - (int)u * c.wout) * c.stride, y = (int)(u - v * c.hout) * c.stride, z = (int)(v - nb * c.dout) * c.stride;
         const int from = ((((int)nb * c.di + z) * c.hi + y) * c.wi + x) * c.ci;
-        // A bit per tap that lies inside the input.
-        unsigned inside = 0u;
-        for (int kd = 0; kd < ks; ++kd)
-            for (int kh = 0; kh < ks; ++kh) {
-                if ((unsigned)(z + kd - c.pad) >= (unsigned)c.di || (unsigned)(y + kh - c.pad) >= (unsigned)c.hi) continue;
-                for (int kw = 0; kw < ks; ++kw)
-                    if ((unsigned)(x + kw - c.pad) < (unsigned)c.wi) inside |= 1u << ((kd * ks + kh) * ks + kw);
-            }
+        // A bit per tap that lies inside the input, from a bit per axis and offset.
+        auto axis_bits = [&](int at, int n) {
+            unsigned bits = 0u;
+            for (int k = 0; k < ks; ++k) bits |= (unsigned)(at + k - c.pad) < (unsigned)n ? 1u << k : 0u;
+            return bits;
+        };
+        const unsigned bx = axis_bits(x, c.wi), by = axis_bits(y, c.hi), bz = axis_bits(z, c.di);
+        unsigned line = 0u, inside = 0u;
+        for (int k = 0; k < ks; ++k) line |= by >> k & 1u ? bx << k * ks : 0u;
+        for (int k = 0; k < ks; ++k) inside |= bz >> k & 1u ? line << k * ks * ks : 0u;
         if (row >= rows) inside = 0u;
         s8 taken;
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             taken[t] = 0;
-            if (inside >> tap[t] & 1u)
-                taken[t] = *global(reinterpret_cast<const short*>(reinterpret_cast<const char*>(g.source) + (unsigned)(from + at[t]) * 2u));
+            if (inside >> tap[t] & 1u) {
+                const unsigned element = (unsigned)(from + at[t]);
+                if (Wide) taken[t] = (short)float_to_bf16(*global(reinterpret_cast<const float*>(reinterpret_cast<const char*>(g.source) + element * 4u)));
+                else taken[t] = *global(reinterpret_cast<const short*>(reinterpret_cast<const char*>(g.source) + element * 2u));
+            }
         }
 #pragma unroll
         for (int i = 0; i < CT; ++i) {
@@ -744,15 +752,21 @@ bool gather_gemm(GatherGemm g, hipStream_t stream) {
     const long long inside = (long long)g.c.di * g.c.hi * g.c.wi, outside = (long long)g.c.dout * g.c.hout * g.c.wout;
     if (g.c.n * inside > 0x7fffffffLL || inside * g.channels > 0x7fffffffLL || outside * g.channels > 0x7fffffffLL) return false;
     if (g.N % 4 == 0 && (!aligned16(g.pre) || !aligned16(g.y) || (reinterpret_cast<uintptr_t>(g.act) & 7u))) return false;
-    if (!g.dgrad && g.ldw == 32 && aligned16(g.weight) && g.c.n * inside * g.c.ci <= 0x7fffffffLL) {     // 32-bit byte offsets
+    if (!g.dgrad && g.ldw == 32 && aligned16(g.weight) && g.c.n * inside * g.c.ci <= (g.wide ? 0x3fffffffLL : 0x7fffffffLL)) {     // 32-bit byte offsets
         const int rows = g.c.n * g.c.dout * g.c.hout * g.c.wout, columns = g.N <= 32 ? 2 : 4;
         const dim3 grid((rows + 255) / 256, (g.N + columns * 16 - 1) / (columns * 16)), block(256);
         const NarrowSplit split{make_divider((unsigned)g.c.wout), make_divider((unsigned)g.c.hout), make_divider((unsigned)g.c.dout),
                                 small_reciprocal(g.c.ci), small_reciprocal(g.c.ks), small_reciprocal(g.c.ks * g.c.ks)};
-        if (columns == 2) hipLaunchKernelGGL(narrow_forward_kernel<2>, grid, block, 0, stream, g, rows, split);
-        else hipLaunchKernelGGL(narrow_forward_kernel<4>, grid, block, 0, stream, g, rows, split);
+        if (columns == 2) {
+            if (g.wide) hipLaunchKernelGGL((narrow_forward_kernel<2, true>), grid, block, 0, stream, g, rows, split);
+            else hipLaunchKernelGGL((narrow_forward_kernel<2, false>), grid, block, 0, stream, g, rows, split);
+        } else {
+            if (g.wide) hipLaunchKernelGGL((narrow_forward_kernel<4, true>), grid, block, 0, stream, g, rows, split);
+            else hipLaunchKernelGGL((narrow_forward_kernel<4, false>), grid, block, 0, stream, g, rows, split);
+        }
         return true;
     }
+    if (g.wide) return false;
     if (g.channels % 8 || !aligned16(g.source) || !aligned16(g.weight) || g.ldw % 8) return false;
     int classes = 1;
     if (g.dgrad && g.c.stride == 2) {
@@ -1228,8 +1242,9 @@ int tfdtd_conv_weights(const tfdtd_conv* convs, int32_t count, const float* cons
     return tfdtd_check_launch("conv weights");
 }
 
-int tfdtd_conv_forward_rows(const tfdtd_conv* d, const void* x, const void* weight, const int32_t* nonfinite, const float* bias,
-                            int32_t activation, float* pre, float* y, void* act, void* stream) {
+int tfdtd_conv_forward_rows(const tfdtd_conv* d, const void* x, int32_t x_dtype, const void* weight, const int32_t* nonfinite,
+                            const float* bias, int32_t activation, float* pre, float* y, void* act, void* stream) {
+    if (x_dtype != TFDTD_CONV_BF16 && x_dtype != TFDTD_F32) return tfdtd_fail(TFDTD_EINVAL, "conv forward: x is bf16 or float32");
     if (!d || !x || !weight || (!pre && !y && !act)) return tfdtd_fail(TFDTD_EINVAL, "conv forward: null pointer");
     int status = check_conv(*d);
     if (status) return status;
@@ -1237,6 +1252,7 @@ int tfdtd_conv_forward_rows(const tfdtd_conv* d, const void* x, const void* weig
     g.c = make_conv(*d);
     if ((long long)d->n * g.c.dout * g.c.hout * g.c.wout > 0x7fffffffLL) return tfdtd_fail(TFDTD_EINVAL, "conv: too many positions");
     g.N = d->co; g.channels = d->ci; g.ldw = d->kp;
+    g.wide = x_dtype == TFDTD_F32;
     g.source = static_cast<const bf16_bits*>(x);
     g.weight = static_cast<const bf16_bits*>(weight);
     g.nonfinite = nonfinite;

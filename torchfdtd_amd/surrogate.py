@@ -73,12 +73,18 @@ def _operands(shapes, weights, transposed):
 
 
 def _forward(shape, x16, w16, parts, bias, activation, pre=None, y=None, act=None):
-    """One layer: x16 -> any of pre (FP32), y (FP32 of the bf16 activation) and act (bf16), each [m, co] or None."""
+    """One layer: x16 -> any of pre (FP32), y (FP32 of the bf16 activation) and act (bf16), each [m, co] or None.
+    x16 may be FP32: a layer of at most 32 values of K rounds it as it reads it, others after a conversion."""
     lib, stream = N.library(), N.stream_handle()
-    status = lib.tfdtd_conv_forward_rows(ctypes.byref(shape), x16.data_ptr(), w16.data_ptr(), N.address(parts), bias.data_ptr(),
-                                         int(activation), N.address(pre), N.address(y), N.address(act), stream)
+    wide = x16.dtype == torch.float32
+    if wide and (shape.kp != 32 or x16.numel() >= 1 << 30):
+        x16, wide = x16.to(torch.bfloat16), False
+    status = lib.tfdtd_conv_forward_rows(ctypes.byref(shape), x16.data_ptr(), N.F32 if wide else N.CONV_BF16, w16.data_ptr(),
+                                         N.address(parts), bias.data_ptr(), int(activation), N.address(pre), N.address(y),
+                                         N.address(act), stream)
     if status != N.EUNSUPPORTED:
         return N.check(status, 'tfdtd_conv_forward_rows')
+    x16 = x16.to(torch.bfloat16)
     out = next(t for t in (pre, y, act) if t is not None)
     pre = torch.empty(out.shape, device=out.device, dtype=torch.float32) if pre is None else pre
     act16 = torch.empty(out.shape, device=out.device, dtype=torch.bfloat16) if act is None else act
@@ -188,7 +194,9 @@ class _Trunk(torch.autograd.Function):
             shapes.append(shape)
             dims = (dims[0], *out, w.shape[0])
         operands = _operands(shapes, weights, [keep and (k > 0 or ctx.needs_input_grad[3]) for k in range(len(shapes))])
-        inputs, pres = [x.detach().to(torch.bfloat16).contiguous()], []
+        # The first layer's bf16 input is kept for its weight gradient alone.
+        x = x.detach().contiguous()
+        inputs, pres = [x if not keep and x.dtype == torch.float32 else x.to(torch.bfloat16)], []
         for k, (shape, (w16, _, parts), bias) in enumerate(zip(shapes, operands, biases)):
             last = k+1 == len(shapes)
             m = conv_rows(shape)
