@@ -29,3 +29,32 @@ def test_wide_source_equals_the_rounded_one(gpu, n, d, h, w, ci, co, ks, stride,
         results.append(out)
     for a, b in zip(*results):
         assert torch.equal(torch.nan_to_num(a, nan=123.), torch.nan_to_num(b, nan=123.))
+
+
+@pytest.mark.parametrize('channels,batch', [((8,), 1), ((32, 40), 3), ((8,)*7, 2)])
+@pytest.mark.parametrize('trained', ['all', 'head', 'none'])
+def test_network_equals_its_layers(gpu, channels, batch, trained):
+    """The network, whose head shares the trunk's operand launch (not beyond eight layers) and keeps bf16 without a
+    backward, against conv3d and linear layer by layer: outputs and gradients equal."""
+    from torchfdtd_amd.surrogate import SurrogateNet, conv3d, linear
+    net = SurrogateNet(channels=channels, hidden=24, outputs=8, seed=2).to(gpu)
+    for p in net.parameters():
+        p.requires_grad_(trained == 'all')
+    for p in net.head:
+        p.requires_grad_(trained != 'none')
+    rho = torch.rand((batch, 17, 12, 8), device=gpu, generator=torch.Generator(device='cuda').manual_seed(1))
+
+    def layers():
+        x = rho.unsqueeze(-1)
+        for w, b in zip(net.weights, net.biases):
+            x = conv3d(x, w, b, 2, 1, True)
+        return linear(linear(x.mean(dim=(1, 2, 3)), net.head[0], net.head[1]), net.head[2], net.head[3], activation=False)
+
+    wanted = [p for p in net.parameters() if p.requires_grad]
+    results = []
+    for y in (net(rho), layers()):
+        results.append([y.detach(), *(torch.autograd.grad(y.square().sum(), wanted) if wanted else ())])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+    with torch.no_grad():
+        assert torch.equal(net(rho), results[0][0])

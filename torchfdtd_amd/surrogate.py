@@ -140,15 +140,20 @@ def _input_gradient(shape, dpre16, w16, wt, parts):
 
 
 class _Conv(torch.autograd.Function):
-    """y = act(conv(x) + b), x and y FP32 channels-last; bf16 operands on MFMA inside."""
+    """y = act(conv(x) + b), x and y FP32 channels-last; bf16 operands on MFMA inside.  `operands`: the layer's,
+    where the caller made them with others'.  `narrow` (no backward will follow): y stays bf16."""
 
     @staticmethod
-    def forward(ctx, x, weight, bias, stride, pad, activation):
+    def forward(ctx, x, weight, bias, stride, pad, activation, operands=None, narrow=False):
         co, ks, ci = weight.shape[0], weight.shape[1], weight.shape[-1]
         shape, (do, ho, wo) = conv_shape(tuple(x.shape), ci, co, ks, stride, pad)
         x16 = x.detach().to(torch.bfloat16).contiguous()
-        (w16, wt, parts), = _operands([shape], [weight.detach()], [ctx.needs_input_grad[0]])
+        w16, wt, parts = operands or _operands([shape], [weight.detach()], [ctx.needs_input_grad[0]])[0]
         m = x.shape[0]*do*ho*wo
+        if narrow:
+            act = torch.empty((m, co), device=x.device, dtype=torch.bfloat16)
+            _forward(shape, x16, w16, parts, bias.detach().float().contiguous(), activation, act=act)
+            return act.view(x.shape[0], do, ho, wo, co)
         pre = torch.empty((m, co), device=x.device, dtype=torch.float32)
         y = torch.empty((m, co), device=x.device, dtype=torch.float32)
         _forward(shape, x16, w16, parts, bias.detach().float().contiguous(), activation, pre=pre, y=y)
@@ -165,7 +170,7 @@ class _Conv(torch.autograd.Function):
         ks, ci = shape.ks, shape.ci
         grad_weight = dw[:, :ks**3*ci].reshape(shape.co, ks, ks, ks, ci)
         grad_x = _input_gradient(shape, dpre16, w16, wt, parts).view(x_shape) if ctx.needs_input_grad[0] else None
-        return grad_x, grad_weight, grad_bias, None, None, None
+        return grad_x, grad_weight, grad_bias, None, None, None, None, None
 
 
 def conv3d(x, weight, bias, stride=1, pad=0, activation=True):
@@ -175,25 +180,37 @@ def conv3d(x, weight, bias, stride=1, pad=0, activation=True):
 
 def linear(x, weight, bias, activation=True):
     """[n, ci] -> [n, co] through the same kernels (a 1x1x1 convolution)."""
+    return _linear(x, weight, bias, activation)
+
+
+def _linear(x, weight, bias, activation, operands=None, narrow=False):
     y = _Conv.apply(x.reshape(x.shape[0], 1, 1, 1, x.shape[1]), weight.reshape(weight.shape[0], 1, 1, 1, weight.shape[1]),
-                    bias, 1, 0, activation)
+                    bias, 1, 0, activation, operands, narrow)
     return y.reshape(x.shape[0], weight.shape[0])
 
 
 class _Trunk(torch.autograd.Function):
     """A chain of convolutions with GELU, x FP32 channels-last -> FP32 output of the last: what conv3d after conv3d
     computes, with the activations between the layers kept in the bf16 that the next layer reads.  Without
-    `keep` (no backward will follow) the pre-activations are not stored."""
+    `keep` (no backward will follow) the pre-activations are not stored.  `head`: weights of linear layers that
+    follow, whose operands are made in the same launch and put in the list `made`, their input gradients' with
+    `transposed`."""
 
     @staticmethod
-    def forward(ctx, keep, stride, pad, x, *parameters):
+    def forward(ctx, keep, stride, pad, head, transposed, made, x, *parameters):
         weights, biases = [w.detach() for w in parameters[::2]], parameters[1::2]
         shapes, dims = [], tuple(x.shape)
         for w in weights:
             shape, out = conv_shape(dims, w.shape[-1], w.shape[0], w.shape[1], stride, pad)
             shapes.append(shape)
             dims = (dims[0], *out, w.shape[0])
-        operands = _operands(shapes, weights, [keep and (k > 0 or ctx.needs_input_grad[3]) for k in range(len(shapes))])
+        if len(shapes)+len(head) > N.CONV_WEIGHT_JOBS or any(w.dtype != torch.float32 for w in head):
+            head = []
+        linears = [ConvShape(dims[0], 1, 1, 1, w.shape[1], w.shape[0], 1, 1, 0, padded_k(1, w.shape[1])) for w in head]
+        operands = _operands(shapes+linears, weights+[w.detach().reshape(w.shape[0], 1, 1, 1, w.shape[1]) for w in head],
+                             [keep and (k > 0 or ctx.needs_input_grad[6]) for k in range(len(shapes))]+[transposed]*len(head))
+        made.extend(operands[len(shapes):])
+        operands = operands[:len(shapes)]
         # The first layer's bf16 input is kept for its weight gradient alone.
         x = x.detach().contiguous()
         inputs, pres = [x if not keep and x.dtype == torch.float32 else x.to(torch.bfloat16)], []
@@ -223,9 +240,9 @@ class _Trunk(torch.autograd.Function):
             shape, (w16, wt, parts) = shapes[k], operands[3*k:3*k+3]
             dpre16, dw, grads[2*k+1] = _layer_gradients(shape, dy, pres[k], 1, inputs[k])
             grads[2*k] = dw[:, :shape.ks**3*shape.ci].reshape(shape.co, *(shape.ks,)*3, shape.ci)
-            if k > 0 or ctx.needs_input_grad[3]:
+            if k > 0 or ctx.needs_input_grad[6]:
                 dy = _input_gradient(shape, dpre16, w16, wt, parts)
-        return (None, None, None, dy.view(x_shape) if ctx.needs_input_grad[3] else None, *grads)
+        return (*(None,)*6, dy.view(x_shape) if ctx.needs_input_grad[6] else None, *grads)
 
 
 class SurrogateNet(nn.Module):
@@ -250,12 +267,16 @@ class SurrogateNet(nn.Module):
     def forward(self, rho):
         x = rho.unsqueeze(-1).float()
         parameters = [p for pair in zip(self.weights, self.biases) for p in pair]
+        grads = torch.is_grad_enabled()
+        train = grads and any(t.requires_grad for t in (x, *parameters, *self.head))
+        made = []
         if parameters:
-            keep = torch.is_grad_enabled() and any(t.requires_grad for t in (x, *parameters))
-            x = _Trunk.apply(keep, 2, 1, x, *parameters)
+            keep = grads and any(t.requires_grad for t in (x, *parameters))
+            x = _Trunk.apply(keep, 2, 1, [self.head[0], self.head[2]], train, made, x, *parameters)
+        first, second = made or (None, None)
         x = x.mean(dim=(1, 2, 3))
-        x = linear(x, self.head[0], self.head[1], activation=True)
-        return linear(x, self.head[2], self.head[3], activation=False)
+        x = _linear(x, self.head[0], self.head[1], True, first, not train)
+        return _linear(x, self.head[2], self.head[3], False, second)
 
     def parameter_count(self):
         return sum(p.numel() for p in self.parameters())
