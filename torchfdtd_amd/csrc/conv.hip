@@ -554,12 +554,13 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64) void gather_gemm_kernel(c
         }
     };
     // The barrier after a stage's loads have landed (all but those of later stages) also ends the reads of the
-    // buffer that the next loads overwrite.
+    // buffer that the next loads overwrite: both are waited for, as a raw barrier orders neither.
     constexpr int PerStage = XI + WI;
+    static_assert(PerStage <= 15, "vmcnt of one stage in the low bits of the wait");
     auto arrive = [&](bool later) {
         asm volatile("" ::: "memory");
-        if (Depth > 2 && later) __builtin_amdgcn_s_waitcnt(0x0f70 | PerStage);      // vmcnt(PerStage)
-        else __builtin_amdgcn_s_waitcnt(0x0f70);                                    // vmcnt(0)
+        if (Depth > 2 && later) __builtin_amdgcn_s_waitcnt(0x0070 | PerStage);      // vmcnt(PerStage) lgkmcnt(0)
+        else __builtin_amdgcn_s_waitcnt(0x0070);                                    // vmcnt(0) lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
@@ -933,7 +934,7 @@ __global__ __launch_bounds__(64 * Waves, Waves / 2) void weight_grad_kernel(cons
     };
     auto arrive = [&] {
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0x0f70);       // vmcnt(0): this wave's stage has landed
+        __builtin_amdgcn_s_waitcnt(0x0070);       // vmcnt(0) lgkmcnt(0): this wave's stage has landed, its reads are done
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
