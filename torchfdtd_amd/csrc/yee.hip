@@ -1084,6 +1084,43 @@ bool make_plane_step(const HalfStep<real>& h, bool forward, PlaneStep<real>* out
     return true;
 }
 
+// Lanes that a march leaves idle: those past the last cell of a plane's last column.
+template <typename real>
+long long idle_lanes(const PlaneStep<real>& a) {
+    return (64LL * a.columns - a.nyz) * a.chunks;
+}
+
+// Whether a plane fills less than `sixteenths` of the lanes of its columns.
+template <typename real>
+bool thin_plane(const PlaneStep<real>& a, int sixteenths) {
+    return 16LL * a.nyz < 64LL * a.columns * sixteenths;
+}
+
+// Whether the march is the faster step of a grid that it can take.  A plane of few cells leaves lanes idle, which
+// costs nothing until they are more than the chip holds at once (256 CUs of 2048 lanes).  us a step, march / general:
+//   FP32 8000x5x1 7.4 / 9.1, 80000x5x1 36 / 12.5, 1000000x5x1 381 / 69, 375000x16x1 148 / 81, 60000x5x5 34 / 33,
+//   187500x32x1 78 / 81; past the 256 MB cache 400000x65x1 386 / 364, 400000x7x5 234 / 229, 200000x9x8 231 / 235;
+//   FP64 80000x5x1 46 / 17, 93750x16x1 54 / 41, 62500x24x1 40 / 41, 60000x5x5 43 / 47.
+// FP64 fields past the cache are bound by HBM, where the march saves the neighbours' address arithmetic for nothing
+// unless there is memory along z: without it 1500x90x90 388 / 351, 400x180x170 394 / 365, 182^3 198 / 189, 171^3
+// (240 MB) 151 / 159; with it 464 / 517, 436 / 455, 222 / 235.
+constexpr long long kIdleLanes = 256 * 2048;
+
+template <typename real>
+bool march_pays(const PlaneStep<real>& a) {
+    constexpr bool wide = sizeof(real) == 8;
+    const bool past_cache = 6LL * (long long)sizeof(real) * a.nx * a.nyz > 256LL << 20;
+    if (wide && past_cache && a.axis[2].hi[0] == a.axis[2].lo[0] && a.axis[2].hi[1] == a.axis[2].lo[1]) return false;
+    return !thin_plane(a, wide ? 6 : past_cache ? 9 : 8) || idle_lanes(a) <= kIdleLanes;
+}
+
+// The same for a grid of a batch, whose workgroups look their grid up: a plane has to fill more of its lanes, and the
+// idle lanes are those of all such grids.  us a step, march / general: FP32 400 grids of 2000x5x1 746 / 77 (30: 54 / 17),
+// 272 of 300x7x7 95 / 87, 400 of 100x10x10 96 / 88, 178 of 400x56x1 79 / 83, 30 of 400x5x5 18 / 19; FP64 307 of
+// 100x13x10 140 / 128, 208 of 400x48x1 160 / 165.
+template <typename real>
+constexpr int kBatchThin = sizeof(real) == 8 ? 11 : 13;
+
 template <typename real>
 void launch_plane_step(const PlaneStep<real>& a, bool forward, int inverse_stride, hipStream_t stream) {
     const dim3 grid((unsigned)plane_blocks(a)), block(256);
@@ -1107,7 +1144,7 @@ int launch_half_step(const tfdtd_half_step* d, hipStream_t stream) {
     if (status) return status;
     const bool forward = d->family == TFDTD_FAMILY_H;
     PlaneStep<real> p;
-    if (make_plane_step(a, forward, &p)) {
+    if (make_plane_step(a, forward, &p) && march_pays(p)) {
         launch_plane_step(p, forward, d->inverse_stride, stream);
         return check_launch("yee_half_step");
     }
@@ -1297,7 +1334,7 @@ int pack_half_steps(const tfdtd_half_step* steps, int count, void* host_table, s
     if (count < 1 || !steps || !prefix) return fail(TFDTD_EINVAL, "batch: at least one descriptor and a prefix array");
     if (!host_table || bytes < sizeof(BatchStep<real>) * (size_t)count) return fail(TFDTD_EINVAL, "batch: table buffer too small");
     BatchStep<real>* table = static_cast<BatchStep<real>*>(host_table);
-    long long total = 0;
+    long long total = 0, idle = 0;
     for (int k = 0; k < count; ++k) {
         if (steps[k].family != steps[0].family || steps[k].dtype != steps[0].dtype)
             return fail(TFDTD_EINVAL, "batch: descriptor %d differs in family or dtype", k);
@@ -1306,6 +1343,11 @@ int pack_half_steps(const tfdtd_half_step* steps, int count, void* host_table, s
         if (status) return status;
         t.march = make_plane_step(t.general, steps[k].family == TFDTD_FAMILY_H, &t.plane) ? 1 : 0;
         t.inverse_stride = t.general.inverse_stride;
+        if (t.march && thin_plane(t.plane, kBatchThin<real>)) idle += idle_lanes(t.plane);
+    }
+    for (int k = 0; k < count; ++k) {
+        BatchStep<real>& t = table[k];
+        if (t.march && idle > kIdleLanes && thin_plane(t.plane, kBatchThin<real>)) t.march = 0;
         prefix[k] = (int32_t)total;
         total += t.march ? plane_blocks(t.plane)
                          : ((long long)steps[k].nx * steps[k].ny * steps[k].nz + 256 * kBatchSpan - 1) / (256 * kBatchSpan);
@@ -1422,7 +1464,7 @@ int observed_step(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, 
     if (!status) status = make_half_step(h_step, &h);
     if (status) return status;
     PlaneStep<real> pe, ph;
-    if (!make_plane_step(e, false, &pe) || !make_plane_step(h, true, &ph)) return TFDTD_OK;
+    if (!make_plane_step(e, false, &pe) || !make_plane_step(h, true, &ph) || !march_pays(pe) || !march_pays(ph)) return TFDTD_OK;
     CurlBox<real> box;
     if (record && !make_curl_box(*record, *e_step, *obs, pe, &box)) return TFDTD_OK;
     *done = true;
