@@ -256,7 +256,8 @@ int tfdtd_step_observed(const tfdtd_half_step* e_step, const tfdtd_half_step* h_
 /* `n_steps` (two or more) whole steps of one grid of one z plane, several to a launch, with its traces and counter: the
  * state ends in the grid's own buffers by way of `second`, a set of the same sizes whose contents do not matter.
  * Results are those of n_steps calls of tfdtd_step_observed.  TFDTD_EUNSUPPORTED where the grid has more planes, the
- * half steps do not take the plane march, or the traces are not given by `cells`; n_steps 0 only asks that. */
+ * half steps do not take the plane march, the grid is long and narrower than its patches (the half steps are then
+ * faster), or the traces are not given by `cells`; n_steps 0 only asks that. */
 typedef struct tfdtd_flat_buffers {
     void *e, *h, *psi_e, *psi_h;
 } tfdtd_flat_buffers;

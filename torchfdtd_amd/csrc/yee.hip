@@ -493,6 +493,15 @@ inline long long flat_tiles(int nx, int ny, int steps) {
 
 inline int flat_depth(int nx, int ny) { return flat_tiles(nx, ny, kFlatSteps) <= 512 ? kFlatSteps : flat_tiles(nx, ny, 6) <= 2048 ? 6 : 4; }
 
+// Whether the patches are the faster way.  A grid narrower than a patch leaves its lanes idle, which costs nothing while the
+// patches run in four rounds; beyond, a quarter of their lanes has to own a cell.  us per step, half steps / patches: FP32
+// 5x40000 7.9 / 5.9, 8x60000 8.5 / 8.7, 5x100000 10.6 / 13.5, 8x1000000 88 / 121, 12x1000000 149 / 122; FP64 8x60000
+// 12.3 / 15.8, 5x1000000 123 / 237, 12x100000 32 / 26.
+inline bool flat_pays(int nx, int ny) {
+    const int depth = flat_depth(nx, ny);
+    return depth > 4 || 4LL * nx * ny >= flat_tiles(nx, ny, depth) * (kFlatTile * kFlatTile);
+}
+
 template <typename real>
 struct FlatSet {            // one buffer set: fields and each family's CPML memory
     real *e, *h, *psi_e, *psi_h;
@@ -1500,6 +1509,7 @@ int flat_steps(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, con
     if (e.nz != 1 || e.nx != h.nx || e.ny != h.ny || e.nz != h.nz || e.src != h.dst || e.dst != h.src ||
         e.periodic_mask != h.periodic_mask || !make_plane_step(e, false, &a.e) || !make_plane_step(h, true, &a.h))
         return fail(TFDTD_EUNSUPPORTED, "flat_steps needs one grid of one z plane that the plane march takes");
+    if (!flat_pays(e.nx, e.ny)) return fail(TFDTD_EUNSUPPORTED, "flat_steps: the grid is too narrow for its patches");
     bool folded = false;
     status = fold_traces(obs, cells, &a.h, &folded);
     if (status) return status;
