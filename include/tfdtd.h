@@ -253,7 +253,8 @@ int tfdtd_step_observed(const tfdtd_half_step* e_step, const tfdtd_half_step* h_
                         int32_t plane_count, const tfdtd_observe* observe, const tfdtd_trace_cell* cells, int64_t* shadow,
                         void* stream);
 
-/* `n_steps` (two or more) whole steps of one grid of one z plane, several to a launch, with its traces and counter: the
+/* `n_steps` (two or more) whole steps of one grid of one z plane, several to a launch (two or three steps of a large grid
+ * as half steps, which are then faster), with its traces and counter: the
  * state ends in the grid's own buffers by way of `second`, a set of the same sizes whose contents do not matter.
  * Results are those of n_steps calls of tfdtd_step_observed.  TFDTD_EUNSUPPORTED where the grid has more planes, the
  * half steps do not take the plane march, the grid is long and narrower than its patches (the half steps are then

@@ -502,6 +502,19 @@ inline bool flat_pays(int nx, int ny) {
     return depth > 4 || 4LL * nx * ny >= flat_tiles(nx, ny, depth) * (kFlatTile * kFlatTile);
 }
 
+// Whether `n` steps are worth two launches of patches: two steps of patches load and store the state as often as two half
+// step pairs do, with a rim of each patch twice, and pay while the patches run at once (FP64: one to a CU).  us per step,
+// half steps / patches.  Two steps: FP32 300x300 9.4 / 8.4, 500x500 10.7 / 10.9, 800x800 13.9 / 16.9, 3000x3000 88 / 127;
+// FP64 300x300 9.9 / 10.0, 500x500 11.7 / 16.4, 1500x1500 51 / 60, 3000x3000 (past the cache) 259 / 247.  Three: FP32
+// 500x500 9.6 / 8.5, 3000x3000 88 / 89; FP64 500x500 10.8 / 12.7, 800x800 18.9 / 19.1, 1500x1500 50 / 44.  Four: FP32
+// 3000x3000 87 / 71, FP64 500x500 10.2 / 9.3.
+inline bool flat_block_pays(int nx, int ny, int n, bool wide) {
+    const long long tiles = flat_tiles(nx, ny, 2);
+    if (n >= 4 || tiles <= 256) return true;
+    if (n == 3) return !wide || tiles > 768;
+    return wide && 48LL * nx * ny > 256LL << 20;
+}
+
 template <typename real>
 struct FlatSet {            // one buffer set: fields and each family's CPML memory
     real *e, *h, *psi_e, *psi_h;
@@ -1515,6 +1528,11 @@ int flat_steps(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, con
     if (status) return status;
     if (obs->count > 0 && !folded) return fail(TFDTD_EUNSUPPORTED, "flat_steps records at most %d traces", kPlaneTraces);
     if (n == 0) return TFDTD_OK;
+    if (!flat_block_pays(e.nx, e.ny, n, sizeof(real) == 8)) {
+        for (int k = 0; k < n && !status; ++k)
+            status = tfdtd_step_observed(e_step, h_step, nullptr, 0, obs, cells, reinterpret_cast<int64_t*>(shadow), stream);
+        return status;
+    }
     long long* const counter = reinterpret_cast<long long*>(obs->counter);
     const FlatSet<real> own{a.e.dst, a.h.dst, a.e.psi, a.h.psi};
     const int depth = flat_depth(a.e.nx, a.e.ny), passes = (n + 2 * depth - 1) / (2 * depth) * 2;
