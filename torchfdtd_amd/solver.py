@@ -669,7 +669,8 @@ class Stepper:
 
     def flat(self):
         """Whether `block` takes this grid: one z plane, at most `FOLDED_TRACES` traces, no plane monitors, no ADE.
-        Allocates its second buffer set (on the caller's stream, outside any capture)."""
+        Allocates its second buffer set (on the caller's stream, outside any capture); a grid whose state fits only
+        once keeps single steps."""
         if self.kernel != 'hip' or self.dispersive or self.planes or self.grid.Nz != 1:
             return False
         status = self.lib.tfdtd_flat_steps(ctypes.byref(self.e_step), ctypes.byref(self.h_step), ctypes.byref(self.observe),
@@ -679,7 +680,10 @@ class Stepper:
         N.check(status, 'tfdtd_flat_steps')
         if self.flat_set is None:
             g = self.grid
-            self.flat_set = [torch.empty_like(t) for t in (g.E, g.H, g.psi_buffers[False], g.psi_buffers[True])]
+            try:
+                self.flat_set = [torch.empty_like(t) for t in (g.E, g.H, g.psi_buffers[False], g.psi_buffers[True])]
+            except torch.OutOfMemoryError:
+                return False
         return True
 
     def block(self, count):
@@ -743,22 +747,25 @@ class Simulation:
         control = r.run_control
         monitor = (RunMonitor([g], [p], check_count(p), energies=[run.oscillator_energy if run.dispersive else None])
                    if control.auto_shutoff or control.divergence_check else None)
+        interval = max(r.snapshot_interval, math.ceil(r.steps/100))
+        barriers = set(range(interval, r.steps+1, interval))
+        if monitor is not None:
+            barriers.update(range(control.check_interval, r.steps+1, control.check_interval))
+        # Blocks of steps need a second buffer set: only where a graph of several steps fits between two barriers.
+        ends = [0, *sorted(barriers | {r.steps})]
+        blocks = cuda_graph and 1 < min(cuda_graph_steps, r.steps) <= max(b-a for a, b in zip(ends, ends[1:]))
         graph = (StepGraphs(run.step, run.states(), r.steps, cuda_graph_steps, pair=run.step_pair if run.one_pass else None,
                             prepare=run.refresh_materials if run.one_pass else None,
-                            quad=run.quad if run.two_step else None, block=run.block if run.flat() else None)
+                            quad=run.quad if run.two_step else None, block=run.block if blocks and run.flat() else None)
                  if cuda_graph else None)
         view = DisplaySlice(p)
         plane_index = view.index
         eps_plane = view.epsilon(run.eps)
-        interval = max(r.snapshot_interval, math.ceil(r.steps/100))
         frames, frame_steps = [], []
         torch.cuda.synchronize()
         setup_seconds = time.perf_counter()-started
         compute_start = time.perf_counter()
         completed, termination, diagnostic_seconds, replays = 0, 'max_steps', 0., 0
-        barriers = set(range(interval, r.steps+1, interval))
-        if monitor is not None:
-            barriers.update(range(control.check_interval, r.steps+1, control.check_interval))
         width = graph.width if graph is not None else 1
         eager_steps = 0
         # Barriers enqueue the diagnostics and the frame copies on the GPU; the host waits only
