@@ -45,3 +45,13 @@ def test_a_state_that_fits_once_keeps_single_steps(gpu, monkeypatch):
     got = solver.Simulation(project(20)).run(cuda_graph_steps=20)
     assert answers == [False]
     assert np.array_equal(got.electric, ref.electric) and np.array_equal(got.magnetic, ref.magnetic)
+
+
+def test_the_report_counts_the_steps_of_blocks(gpu):
+    from torchfdtd_amd.solver import Simulation
+    steps = [Simulation(project(20)).run(cuda_graph_steps=width).summary['kernel_steps'] for width in (20, 7, 1)]
+    # Barriers at 20, 40, 50 and 60.
+    assert [s['flat'] for s in steps] == [40, 42, 0] and [s['split'] for s in steps] == [20, 18, 60]
+    from test_plane_march import project_for
+    cube = project_for((14, 13, 12), 'float32', 'cell', {})
+    assert Simulation(cube).run(cuda_graph_steps=10).summary['kernel_steps'] == dict(two_step=0, one_pass=0, split=20, flat=0)

@@ -573,7 +573,7 @@ def _run(cases, projects, launch, objective, root, keep_results, memory_fraction
         frames[i] = np.array([f.cpu().numpy() for f in frames[i]])
         if not np.isfinite(frames[i]).all():
             raise FloatingPointError(f'Case {case.id}: non-finite displayed field.')
-    kernel_steps = dict(graph.kernel_steps) if graph is not None else dict(two_step=0, one_pass=0, split=eager_steps)
+    kernel_steps = dict(graph.kernel_steps) if graph is not None else dict(two_step=0, one_pass=0, split=eager_steps, flat=0)
     if root:
         root.mkdir(parents=True, exist_ok=True)
     items = []

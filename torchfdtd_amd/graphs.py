@@ -39,10 +39,12 @@ class StepGraphs:
     before every replay (e.g. Stepper.refresh_materials, which follows permittivity changes).
     """
 
-    def __init__(self, step, states, steps, width=1, warmup=3, pair=None, prepare=None, quad=None, widths=(), block=None):
+    def __init__(self, step, states, steps, width=1, warmup=3, pair=None, prepare=None, quad=None, widths=(), block=None,
+                 block_path='split'):
         """`widths`: further step counts to capture a graph of each (<= 64), for callers that advance
         by counts other than 1 and `width` (a checkpoint segment and its remainder).  `block(n)`, when given,
-        takes n steps at once in place of n calls of `step`."""
+        takes n steps at once in place of n calls of `step`; `block_path` names the path of its two steps and more in
+        `kernel_steps` ('flat': several steps of a flat grid to a launch)."""
         self.prepare = prepare
         self.width = min(validate_graph_steps(width), steps)
         states = list(states)
@@ -62,14 +64,14 @@ class StepGraphs:
         torch.cuda.current_stream().wait_stream(stream)
         torch.cuda.synchronize()
         self.graphs = {}
-        self.kernel_steps = dict(two_step=0, one_pass=0, split=0)     # steps replayed through each path
+        self.kernel_steps = dict(two_step=0, one_pass=0, split=0, flat=0)     # steps replayed through each path
         self.composition = {}
         counts = {1, self.width} | {min(int(w), steps) for w in widths if 1 <= int(w) <= 64}
         if quad is not None and self.width > 4:
             counts.add(4)       # one four: replays that stop at any multiple of four stay on the quad path
         for count in sorted(counts):
             graph = torch.cuda.CUDAGraph()
-            made = dict(two_step=0, one_pass=0, split=0)
+            made = dict(two_step=0, one_pass=0, split=0, flat=0)
             with torch.cuda.stream(stream):
                 graph.capture_begin()
                 if pair is not None and count > 1:
@@ -91,7 +93,7 @@ class StepGraphs:
                     else:
                         for _ in range(count):
                             step()
-                    made['split'] = count
+                    made[block_path if block is not None and count > 1 else 'split'] = count
                 graph.capture_end()
             self.composition[count] = made
             self.graphs[count] = graph

@@ -756,7 +756,8 @@ class Simulation:
         blocks = cuda_graph and 1 < min(cuda_graph_steps, r.steps) <= max(b-a for a, b in zip(ends, ends[1:]))
         graph = (StepGraphs(run.step, run.states(), r.steps, cuda_graph_steps, pair=run.step_pair if run.one_pass else None,
                             prepare=run.refresh_materials if run.one_pass else None,
-                            quad=run.quad if run.two_step else None, block=run.block if blocks and run.flat() else None)
+                            quad=run.quad if run.two_step else None, block=run.block if blocks and run.flat() else None,
+                            block_path='flat')
                  if cuda_graph else None)
         view = DisplaySlice(p)
         plane_index = view.index
@@ -809,7 +810,7 @@ class Simulation:
         e, h = g.E.cpu().numpy().copy(), g.H.cpu().numpy().copy()
         if not np.isfinite(e).all() or not np.isfinite(h).all():
             raise FloatingPointError('Non-finite fields detected.')
-        kernel_steps = dict(graph.kernel_steps) if graph is not None else dict(two_step=0, one_pass=0, split=eager_steps)
+        kernel_steps = dict(graph.kernel_steps) if graph is not None else dict(two_step=0, one_pass=0, split=eager_steps, flat=0)
         summary = run_summary(p, run, e, completed, termination, seconds, setup_seconds, kernel_steps=kernel_steps,
                               launch=run.launch_shape() if run.one_pass else None, launch_tuning=run.launch_record,
                               cuda_graph=graph is not None, cuda_graph_steps=width, cuda_graph_replays=replays,
