@@ -53,6 +53,9 @@ from .solver import ENGINE_LOCK, DisplaySlice, Result, Stepper, pack_table as _p
 # 37.5 / 31.7, 40 grids 74.7 / 65.6; 28 grids in groups of 160 MB 44.5, of 213 MB 49.2.
 WHOLE_BYTES = 232 << 20
 GROUP_BYTES = 208 << 20
+# Steps that repay a group's first pass, which finds nothing in the cache: two steps, whole against grouped, 146 / 152 us a
+# step on 12 grids and 551 / 561 on 40; three 146 / 141 and 550 / 532.
+GROUP_STEPS = 3
 
 
 @dataclass
@@ -368,7 +371,7 @@ class Cohort:
     def step_block(self, count):
         """`count` steps of every grid with the split kernels.  A cohort larger than the memory-side cache advances
         its resident groups one after the other, each by all the steps, the counter set back in between."""
-        if not self.groups or count < 2:
+        if not self.groups or count < GROUP_STEPS:
             for _ in range(count):
                 self.step()
             return
