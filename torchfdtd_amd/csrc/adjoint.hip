@@ -719,7 +719,7 @@ bool make_record_march(const Record<real>& d, RecordMarch<real>* out) {
     a.box.by_nz = make_divider((unsigned)bz);
     a.box.by_columns = make_divider((unsigned)a.box.columns);
     const long long items = (long long)a.box.columns * ((a.box.nx + a.box.span - 1) / a.box.span);
-    if (items > 0x7ffffff0LL) return false;
+    if (items > kLaunchItems) return false;
     a.box.xcd = (int)xcd_run((items + 3) / 4);
     a.nx = d.n[0];
     for (int k = 0; k < 3; ++k) a.lo[k] = d.box_lo[k];
@@ -756,7 +756,7 @@ bool make_march(const Adjoint<real>& d, const Family<real>& f, AdjointMarch<real
     a.by_nz = make_divider((unsigned)a.nz);
     a.by_columns = make_divider((unsigned)a.columns);
     const long long items = (long long)a.columns * ((a.nx + a.span - 1) / a.span);
-    if (items > 0x7ffffff0LL) return false;
+    if (items > kLaunchItems) return false;
     a.xcd = (int)xcd_run((items + 3) / 4);
     a.e_bar = d.e_bar; a.h_bar = d.h_bar; a.inv_eps = d.inv_eps; a.inv_mu = d.inv_mu;
     a.psi_in = f.psi_in; a.psi_out = f.psi_out; a.coef = f.coef;

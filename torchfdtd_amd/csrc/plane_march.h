@@ -91,6 +91,9 @@ __device__ __forceinline__ long long slot_of(long long t, long long modulus) {
 
 constexpr unsigned kXcdRun = 128;
 
+// A launch holds fewer than 2^32 threads: wavefronts of a march, patches of 1024 threads.
+constexpr long long kLaunchItems = 0x3ffffffLL & ~3LL, kLaunchPatches = 0x3fffffLL;
+
 // Planes per march: two share the lane's set-up and the plane between them (18.9 against 20.7 us a step on
 // 160x120x40 cells, 12,000 column-planes; 22.2 against 24.7 us on 97x83x61 in FP64, 7,760; four planes:
 // 18.8 and 22.3).  A grid of few wavefronts keeps one, as it needs them all to fill the chip: 7.3 us

@@ -1090,7 +1090,7 @@ bool make_plane_step(const HalfStep<real>& h, bool forward, PlaneStep<real>* out
     a.by_columns = make_divider((unsigned)a.columns);
     a.chunks = (h.nx + a.span - 1) / a.span;
     const long long items = (long long)a.columns * a.chunks;
-    if (items > 0x7ffffff0LL) return false;
+    if (items > kLaunchItems) return false;
     a.xcd = (int)xcd_run(plane_blocks(a));
     a.src = h.src; a.dst = h.dst; a.inverse = h.inverse;
     a.courant = h.courant;
@@ -1522,6 +1522,8 @@ int flat_steps(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, con
     if (e.nz != 1 || e.nx != h.nx || e.ny != h.ny || e.nz != h.nz || e.src != h.dst || e.dst != h.src ||
         e.periodic_mask != h.periodic_mask || !make_plane_step(e, false, &a.e) || !make_plane_step(h, true, &a.h))
         return fail(TFDTD_EUNSUPPORTED, "flat_steps needs one grid of one z plane that the plane march takes");
+    if (flat_tiles(e.nx, e.ny, flat_depth(e.nx, e.ny)) > kLaunchPatches)
+        return fail(TFDTD_EUNSUPPORTED, "flat_steps: the grid is too large for one launch of patches");
     if (!flat_pays(e.nx, e.ny)) return fail(TFDTD_EUNSUPPORTED, "flat_steps: the grid is too narrow for its patches");
     bool folded = false;
     status = fold_traces(obs, cells, &a.h, &folded);
@@ -1545,9 +1547,7 @@ int flat_steps(const tfdtd_half_step* e_step, const tfdtd_half_step* h_step, con
         a.steps = n / passes + (k < n % passes);
         const int width = kFlatTile - 2 * a.steps;
         a.tiles_y = (a.e.ny + width - 1) / width;
-        const long long tiles = flat_tiles(a.e.nx, a.e.ny, a.steps);
-        if (tiles > 0x7fffffffLL) return fail(TFDTD_EINVAL, "grid too large for one launch");
-        const dim3 grid((unsigned)tiles), block(kFlatTile * kFlatTile);
+        const dim3 grid((unsigned)flat_tiles(a.e.nx, a.e.ny, a.steps)), block(kFlatTile * kFlatTile);
         if (e_step->inverse_stride == 1) hipLaunchKernelGGL((flat_steps_kernel<real, 1>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((flat_steps_kernel<real, 3>), grid, block, 0, stream, a);
         status = check_launch("flat_steps");
