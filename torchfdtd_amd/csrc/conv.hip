@@ -217,15 +217,21 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Gemm g) {
 __global__ __launch_bounds__(256) void split_sum_kernel(const float* partial, int splits, long long count, float* out) {
     __shared__ float sums[3][64];
     const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
-    const long long i = (long long)blockIdx.x * 64 + lane;
-    float s = 0.f;
-    if (i < count)
+    for (long long first = (long long)blockIdx.x * 64; first < count; first += 64LL * gridDim.x) {
+        const long long i = first + lane;
+        float s = 0.f;
+        if (i < count)
 #pragma unroll 4
-        for (int z = part; z < splits; z += 4) s += partial[z * count + i];
-    if (part) sums[part - 1][lane] = s;
-    __syncthreads();
-    if (part == 0 && i < count) out[i] = s + sums[0][lane] + sums[1][lane] + sums[2][lane];
+            for (int z = part; z < splits; z += 4) s += partial[z * count + i];
+        if (part) sums[part - 1][lane] = s;
+        __syncthreads();
+        if (part == 0 && i < count) out[i] = s + sums[0][lane] + sums[1][lane] + sums[2][lane];
+        __syncthreads();
+    }
 }
+
+// A launch holds fewer than 2^32 threads: more values than 2^29 are summed in several turns.
+unsigned split_sum_blocks(long long count) { return (unsigned)std::min<long long>((count + 63) / 64, 1 << 23); }
 
 // dPre = dY * GELU'(pre) (or dY), written in FP32 and BF16.
 __global__ __launch_bounds__(256) void gelu_backward_kernel(const float* dy, const float* pre, long long count, int activation,
@@ -1218,7 +1224,7 @@ int tfdtd_conv_wgrad(const tfdtd_conv* d, const void* dy_t, const void* x, int32
     status = tfdtd_check_launch("conv wgrad");
     if (status) return status;
     const long long count = (long long)g.M * g.N;
-    hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((count + 63) / 64)), dim3(256), 0, s, partial, used, count, dw);
+    hipLaunchKernelGGL(split_sum_kernel, dim3(split_sum_blocks(count)), dim3(256), 0, s, partial, used, count, dw);
     return tfdtd_check_launch("conv wgrad sum");
 }
 
@@ -1330,7 +1336,7 @@ int tfdtd_conv_wgrad_rows(const tfdtd_conv* d, const void* dy, const void* x, fl
     status = tfdtd_check_launch("conv wgrad");
     if (status) return status;
     const long long count = (long long)d->co * d->kp;
-    hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((count + 63) / 64)), dim3(256), 0, s, partial, used, count, dw);
+    hipLaunchKernelGGL(split_sum_kernel, dim3(split_sum_blocks(count)), dim3(256), 0, s, partial, used, count, dw);
     return tfdtd_check_launch("conv wgrad sum");
 }
 
