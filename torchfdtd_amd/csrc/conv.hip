@@ -762,7 +762,9 @@ __global__ __launch_bounds__(256) void narrow_forward_kernel(const GatherGemm g,
 // Runs the gathered GEMM when source and weights allow 16-byte chunks; false leaves it to gemm_kernel.
 bool gather_gemm(GatherGemm g, hipStream_t stream) {
     const long long inside = (long long)g.c.di * g.c.hi * g.c.wi, outside = (long long)g.c.dout * g.c.hout * g.c.wout;
-    if (g.c.n * inside > 0x7fffffffLL || inside * g.channels > 0x7fffffffLL || outside * g.channels > 0x7fffffffLL) return false;
+    // Rows are counted in 32 bits, the last workgroup's past the end among them.
+    if (g.c.n * inside > 0x7fffffffLL - 256 || g.c.n * outside > 0x7fffffffLL - 256) return false;
+    if (inside * g.channels > 0x7fffffffLL || outside * g.channels > 0x7fffffffLL) return false;
     if (g.N % 4 == 0 && (!aligned16(g.pre) || !aligned16(g.y) || (reinterpret_cast<uintptr_t>(g.act) & 7u))) return false;
     if (!g.dgrad && g.ldw == 32 && aligned16(g.weight) && g.c.n * inside * g.c.ci <= (g.wide ? 0x3fffffffLL : 0x7fffffffLL)) {     // 32-bit byte offsets
         const int rows = g.c.n * g.c.dout * g.c.hout * g.c.wout, columns = g.N <= 32 ? 2 : 4;
