@@ -291,7 +291,12 @@ def address(tensor):
 def stream_handle(device=None):
     """The current stream's handle, without the 4 us of a torch Stream object."""
     import torch
-    index = None if device is None else torch.device(device).index
+    index = None
+    if device is not None:
+        device = torch.device(device)
+        if device.type != 'cuda':
+            raise ValueError(f'Expected a cuda device, but got: {device}')
+        index = device.index
     if index is None:
         index = torch.cuda.current_device()
     torch.cuda.init()
