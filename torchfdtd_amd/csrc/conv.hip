@@ -441,18 +441,13 @@ __global__ __launch_bounds__(BM / WM * (BN / WN) * 64) void gather_gemm_kernel(c
     }
     unsigned todo = taps == 32 ? ~0u : (1u << taps) - 1u;
     if (Whole && g.nonfinite) {
+        int bad = 0;
+        for (int i = tid; i < g.parts; i += 64 * Waves) bad |= g.nonfinite[i];
         atomicOr(&s_mask, any);
+        if (bad) s_bad = 1u;
         __syncthreads();
-        // Only a workgroup that has a tap to skip looks the weights' parts up: 262,144 of them on 16384 x 16384, where the
-        // look-up was 360 of a linear layer's 496 us (8 rows).
-        const unsigned met = (unsigned)__builtin_amdgcn_readfirstlane((int)s_mask);
-        if (met != todo) {
-            int bad = 0;
-            for (int i = tid; i < g.parts; i += 64 * Waves) bad |= g.nonfinite[i];
-            if (bad) s_bad = 1u;
-            __syncthreads();
-            if (!__builtin_amdgcn_readfirstlane((int)s_bad)) todo = met;
-        }
+        if (!s_bad) todo = s_mask;
+        todo = (unsigned)__builtin_amdgcn_readfirstlane((int)todo);
     }
     // Elements from a row's position under tap offset 0 to its position under a tap (one sample is below 2^31).
     auto tap_offset = [&](int tap) -> int {
@@ -627,6 +622,9 @@ constexpr unsigned kRowRun = 64;
 template <int BM, int BN, int WM, int WN, int Depth>
 void launch_gather(GatherGemm g, int classes, hipStream_t stream) {
     g.run = kRowRun;
+    // A single tap is never padding, so its flags are not read: 262,144 of them on 16384 x 16384, where every workgroup's
+    // look-up was 360 of a linear layer's 496 us (8 rows).
+    if (g.c.ks == 1) g.nonfinite = nullptr;
     const dim3 grid((g.rows_max + BM - 1) / BM, (g.N + BN - 1) / BN, classes), block(BM / WM * (BN / WN) * 64);
     if (g.channels % 32 == 0) hipLaunchKernelGGL((gather_gemm_kernel<BM, BN, WM, WN, Depth, true>), grid, block, 0, stream, g);
     else hipLaunchKernelGGL((gather_gemm_kernel<BM, BN, WM, WN, Depth, false>), grid, block, 0, stream, g);
