@@ -250,7 +250,7 @@ class Cohort:
 
     def _resident_groups(self):
         """Runs of consecutive grids whose state stays in the memory-side cache, each with tables of its own
-        ([] where the whole cohort fits, or has traces, whose rows hold every grid of the cohort)."""
+        ([] where the whole cohort fits, or has traces: their launch records a row of every grid of the cohort at once)."""
         if self.observe.count:
             return []
         sizes = [sum(t.numel()*t.element_size() for t in (g.E, g.H, g.inverse_permittivity, *g.psi_buffers.values()))

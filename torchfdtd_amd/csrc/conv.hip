@@ -815,7 +815,9 @@ bool gather_gemm(GatherGemm g, hipStream_t stream) {
 // the 16 rows of a transposed read over the banks.  The positions are split over blockIdx.z; each split
 // writes its partial sums, which split_sum_kernel adds.  64x32x32x16 positions, 64 -> 128 channels: 0.75 ms
 // (620 TFLOP/s), against 3.1 ms and 1.2 ms for the transposed copy of dY; 0.99 ms while each chunk's position
-// was found by division in every stage, 0.78 ms with four wavefronts a tile.
+// was found by division in every stage, 0.78 ms with four wavefronts a tile.  The next stage's loads are issued before
+// a stage is multiplied, but do not run beside it: the compiler cannot tell the transposed reads from the buffer being
+// loaded and waits for the loads before the first of them, so a stage takes its loads' latency and its products in turn.
 
 struct WeightGrad {
     Conv c;
@@ -1054,7 +1056,8 @@ WeightGradShape weight_grad_shape(const tfdtd_conv& d, const Conv& c) {
     } else {
         return s;
     }
-    // Enough workgroups to fill the chip, and no FP32 sum longer than 12,288 positions (4,096 up to 64 splits).
+    // Enough workgroups to fill the chip, and up to 6.3 M positions (512 splits, which bound the partial sums' memory) no
+    // FP32 sum longer than 12,288 positions (4,096 up to 64 splits); beyond, sums of a 512th of the positions.
     const long long fill = std::min<long long>(768 / tiles, (m + least - 1) / least);
     const long long precise = std::max<long long>((m + 12287) / 12288, std::min<long long>(64, m / 4096));
     s.splits = (int)std::max<long long>(1, std::min<long long>(std::max(fill, precise), 512));

@@ -94,16 +94,16 @@ constexpr unsigned kXcdRun = 128;
 // A launch holds fewer than 2^32 threads: wavefronts of a march, patches of 1024 threads.
 constexpr long long kLaunchItems = 0x3ffffffLL & ~3LL, kLaunchPatches = 0x3fffffLL;
 
-// Planes per march: two share the lane's set-up and the plane between them (18.9 against 20.7 us a step on
-// 160x120x40 cells, 12,000 column-planes; 22.2 against 24.7 us on 97x83x61 in FP64, 7,760; four planes:
-// 18.8 and 22.3).  A grid of few wavefronts keeps one, as it needs them all to fill the chip: 7.3 us
-// against 8.5 on 160x120x1, 320 column-planes.
+// Planes per march: two share the lane's set-up and the plane between them.  us a step with 1 / 2 / 4 planes: 160x120x40
+// cells (12,000 column-planes) 17.6 / 16.8 / 17.6, 200x160x60 33.3 / 31.9 / 33.3, 192^3 102 / 95.6 / 95.3, 256^3 286 / 283 /
+// 292, FP64 97x83x61 (7,760) 19.2 / 19.1 / 20.3.  A grid of few wavefronts keeps one, as it needs them all to fill the
+// chip: 6.0 us against 7.2 on 160x120x1, 320 column-planes.
 constexpr long long kSpanItems = 4096;
 
 // Workgroups that one XCD takes in a row: neighbouring rows and planes are then read through one L2.
-// Runs of 1 / 32 / 128 take 40.0 / 36.5 / 35.7 us on 200x160x60 cells, 117.7 / 106.8 / 105.9 us on 192^3 and
-// 292 / 304 / 286 us on 256^3 (384: 299); grids of few workgroups take shorter runs (97x83x61, 970
-// workgroups: 20.9 us with 32, 22.2 with 128) so that every XCD has its share.
+// Runs of 1 / 32 / 128 / 384 take 37.5 / 34.0 / 31.9 / 32.0 us on 200x160x60 cells, 108 / 96.7 / 95.6 / 92.6 us on 192^3
+// and 290 / 303 / 283 / 298 us on 256^3; grids of few workgroups take shorter runs (FP64 97x83x61, 970 workgroups:
+// 19.1 us, 20.4 with 128) so that every XCD has its share.
 inline unsigned xcd_run(long long blocks) { return (unsigned)std::min<long long>(std::max<long long>(blocks / 32, 1), kXcdRun); }
 
 }  // namespace

@@ -196,11 +196,11 @@ __global__ __launch_bounds__(256) void yee_half_step_kernel(const HalfStep<real>
 // addresses are scalar), and every field access is a uniform base plus a 32-bit lane offset, so a cell
 // costs little more than its own arithmetic.  One thread per cell of the whole grid (half_step_cell) was
 // bound by its 64-bit divisions, per-term slab tests and dependent descriptor loads: a step of both
-// families plus its trace took 26.5 us on 160x120x40 cells, 49.1 us on 200x160x60, 124 us on 192^3, 325 us
-// on 256^3 (FP32), 30.5 us on 97x83x61 (FP64); the march takes 16.7, 33.6, 108, 285 and 18.9 us.  A cell of a
+// families plus its trace took 26.5 us on 160x120x40 cells, 49.1 us on 200x160x60, 121 us on 192^3, 317 us
+// on 256^3 (FP32), 30.4 us on 97x83x61 (FP64); the march takes 16.7, 32.0, 95.6, 283 and 19.1 us.  A cell of a
 // wavefront without slab rows executes about 45 vector instructions (with the lanes' 64-bit address sums and
-// the slabs' arithmetic left to every wavefront: 110, and 18.1, 35.7, 106, 286 and 20.9 us).  What bounds it
-// now is the traffic: past the 256 MB cache 5.3 TB/s of a copy's 5.5, inside it 6.4 of 8.2.
+// the slabs' arithmetic left to every wavefront: 110).  What bounds it now is the traffic: past the 256 MB cache
+// 5.3 TB/s where a float4 copy reaches 6.15, inside it 6.4 of 8.4.
 constexpr int kPlaneTraces = TFDTD_FOLDED_TRACES;
 
 struct PlaneTrace {         // a point trace: its cell and value, and its column among the run's traces
@@ -470,22 +470,23 @@ __global__ __launch_bounds__(256, sizeof(real) == 8 ? 4 : 8) void recorded_half_
 
 // ---------------------------------------------------------------- several steps of a flat grid in one launch
 //
-// A grid of one z plane with few cells is bound by its launches: two of 3 us a step, whatever its cells.  A workgroup here loads a 32 x 32 patch of cells, a lane each, with their CPML memory and
-// coefficients, takes `steps` steps with the fields exchanged through LDS, and stores the cells that are right:
+// A grid of one z plane with few cells is bound by its launches: two of 3 us a step, whatever its cells.  A workgroup here
+// loads a 32 x 32 patch of cells, a lane each, with their CPML memory and coefficients, takes `steps` steps with the fields exchanged through LDS, and stores the cells that are right:
 // a step spoils one more row on each side, so the patch owns its inner (32 - 2 steps)^2 cells and its
 // neighbours compute the rest again.  Fields and memory go from one buffer set to the other (neighbours still read
 // the old state).  Every cell's arithmetic is the half steps' in their order, so results are equal bit for bit.
 //
 // us per step in a graph, half steps and patches: 160x120 6.2 -> 1.34 (FP64 6.3 -> 1.82), 256x256 5.6 -> 1.4, 400x400
-// 6.8 -> 2.4, 800x800 11.4 -> 5.5 (FP64 17.5 -> 10.2), 1500x1500 27.6 -> 14, 3000x3000 85 -> 48 (FP64 274 -> 109).  A small
+// 6.8 -> 2.4, 800x800 11.4 -> 5.5 (FP64 17.5 -> 10.2), 1500x1500 27.6 -> 14, 3000x3000 85 -> 48 (FP64 257 -> 109).  A small
 // grid is bound by one patch's chain (two barriers and two rounds through LDS a step, its load and store), a large
 // one by the cells computed twice.
 constexpr int kFlatTile = 32, kFlatSteps = 8;
 
-// Steps per launch.  More steps share the load, the store and the launch, but own fewer cells of the patch (64% at
+// Steps per launch.  More steps share the load, the store and the launch, but own fewer cells of the patch (66% at
 // 3, 56% at 4, 39% at 6, 25% at 8).  8 while all patches run at once, two to a CU (256x256: 1.41 us a step, 1.63 with
 // 6); 6 up to four such rounds (400x400: 2.43, 2.69 with 8 and 2.74 with 4; 800x800: 5.5, 6.4 and 5.9); 4 beyond (1500x1500:
-// 14.0, 14.8 with 6 and 19.0 with 2; 3000x3000: 48, 55 and 69).
+// 14.0, 14.8 with 6 and 19.0 with 2; 3000x3000: 48, 55 and 69).  The times are FP32's; FP64, whose patches run one to a CU
+// (its registers), takes the same line: 257 to 512 of its patches run in two rounds of 8 steps.
 inline long long flat_tiles(int nx, int ny, int steps) {
     const int own = kFlatTile - 2 * steps;
     return (long long)((nx + own - 1) / own) * ((ny + own - 1) / own);

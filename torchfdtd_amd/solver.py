@@ -34,11 +34,13 @@ from .run_control import RunMonitor, check_count
 
 C0 = 299792458.0
 ENGINE_LOCK = threading.Lock()
-# Default step path by grid size (measured on MI355X, per step, tiles at their best shapes): the split
-# step beats the one-pass tiles by 11-48% on 0.8-7.1 M-cell grids, by 9% at 256^3 and ties them at
-# 320^3 (32.8 M cells); the two-step pass ties the split step at 256^3 and beats it by 21% at 320^3.
-# So float32 grids without plane monitors or traces take the two-step pass from TWO_STEP_MIN_CELLS,
-# other grids the one-pass step from ONE_PASS_MIN_CELLS, and smaller grids the split step.
+# Default step path by grid size (us per step on MI355X, tiles at the best of their shapes; split, one-pass
+# and two-step): 192^3 94 / 195 / 226, 256^3 284 / 353 / 314, 288^3 (23.9 M cells) 394 / 444 / 398, 320^3
+# 522 / 603 / 461, 384^3 (56.6 M) 884 / 980 / 694, 512^3 2177 / 2235 / 1343; float64, split and one-pass,
+# 320^3 1132 / 1242, 384^3 1909 / 2012, 512^3 4735 / 4392.  So float32 grids take the two-step pass from
+# TWO_STEP_MIN_CELLS, where it meets the split step, and smaller grids the split step.  Other grids take the
+# one-pass step from ONE_PASS_MIN_CELLS, a line that stems from a slower split step: the one-pass step is now
+# 3-10% slower in float32 above it, in float64 5% slower at 384^3 and 7% faster at 512^3.
 # tuning.tune_launch measures every path on the grid itself.
 TWO_STEP_MIN_CELLS = 20_000_000
 ONE_PASS_MIN_CELLS = 48_000_000
