@@ -11,7 +11,7 @@ def test_blocks_of_two_steps_stay_whole(gpu, monkeypatch):
     for _ in range(5):
         whole.step()
     monkeypatch.setattr(batch, 'WHOLE_BYTES', 0)
-    monkeypatch.setattr(batch, 'GROUP_BYTES', 1)
+    monkeypatch.setattr(batch, 'GROUP_BYTES', 1 << 20)
     grouped = cohort('float32')
     assert len(grouped.groups) > 1
     step, calls = grouped.step, []
